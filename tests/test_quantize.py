@@ -1,0 +1,59 @@
+"""The quantizers and the 1-bit packing at the edges of their lane groups: row lengths around
+each group's width, rows past the last workgroup's, tables off the 16-byte alignment, and values
+at the ends of the float range, bit for bit against the oracle."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import quantize as oq
+
+from conftest import rng
+
+
+def _table(g, n, d):
+    """Rows of spread scales, with zeros, halves of a code, tiny and huge magnitudes."""
+    x = (g.standard_normal((n, d)) * np.exp(3 * g.standard_normal((n, 1)))).astype(np.float32)
+    x[0] = 0.0
+    if n > 1:
+        x[1] = np.float32(1e-42) * g.integers(-3, 4, d)
+    if n > 2:
+        x[2] = np.float32(3e38) * g.uniform(-1, 1, d)
+    if n > 3:
+        x[3] = g.integers(-254, 255, d) * np.float32(0.5)
+        x[3, 0] = 127.0
+    return np.ascontiguousarray(x)
+
+
+def test_quotient_rounds_once():
+    """fp32(fp64(x) / fp64(a)) * 127 rounded to a whole code is what the fp32 quotient gives: the
+    kernels divide in fp32."""
+    g = rng(40)
+    x = np.concatenate([g.standard_normal(2_000_000), g.uniform(-1, 1, 1_000_000) * 1e-30,
+                        g.uniform(-1, 1, 1_000_000) * 3e38]).astype(np.float32)
+    a = np.maximum(np.abs(x) * np.float32(1) + np.exp(10 * g.standard_normal(x.size)),
+                   1e-8).astype(np.float32)
+    a = np.minimum(a, np.float32(3.4e38))
+    twice = (x.astype(np.float64) / a.astype(np.float64)).astype(np.float32)
+    once = x / a
+    same = (twice == once) | (np.abs(once) < np.finfo(np.float32).tiny)
+    assert same.all()
+    assert np.array_equal(np.rint(twice * np.float32(127)), np.rint(once * np.float32(127)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("n,d", [(1, 4), (17, 60), (33, 64), (9, 68), (5, 128), (7, 132), (3, 256),
+                                 (6, 260), (4, 1024), (4, 1028), (5, 2048), (4, 2052), (40, 7),
+                                 (140_001, 32)])
+def test_rows(n, d, offset):
+    import retrieve_amd.hip  # noqa: F401
+
+    print(f"quantize_int8 n={n} d={d} offset={offset}", flush=True)
+    x = _table(rng(n + d), n, d)
+    flat = torch.zeros(n * d + offset, device="cuda:0")
+    flat[offset:] = torch.from_numpy(x).reshape(-1).to("cuda:0")
+    codes, scales = torch.ops.retrieve_amd.quantize_int8(flat[offset:].view(n, d))
+    want_c, want_s = oq.quantize_int8(x, divide=True)
+    assert np.array_equal(codes.cpu().numpy(), want_c)
+    assert np.array_equal(scales.cpu().numpy(), want_s)
