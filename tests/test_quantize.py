@@ -57,3 +57,24 @@ def test_rows(n, d, offset):
     want_c, want_s = oq.quantize_int8(x, divide=True)
     assert np.array_equal(codes.cpu().numpy(), want_c)
     assert np.array_equal(scales.cpu().numpy(), want_s)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("n,d", [(1, 4), (33, 64), (9, 68), (5, 128), (7, 132), (6, 260),
+                                 (4, 1028), (4, 2052), (40, 7), (140_001, 32)])
+def test_global(n, d, offset):
+    import retrieve_amd.hip  # noqa: F401
+
+    print(f"quantize_int8_global n={n} d={d} offset={offset}", flush=True)
+    g = rng(n * 3 + d)
+    x = g.standard_normal((n, d)).astype(np.float32)
+    flat = torch.zeros(n * d + offset, device="cuda:0")
+    flat[offset:] = torch.from_numpy(x).reshape(-1).to("cuda:0")
+    perm = g.permutation(n)
+    for rows in (None, perm):
+        codes, abs_max = torch.ops.retrieve_amd.quantize_int8_global(
+            flat[offset:].view(n, d), None if rows is None else torch.from_numpy(rows).to("cuda:0"))
+        want_c, want_m = oq.quantize_int8_global(x, rows)
+        assert np.array_equal(codes.cpu().numpy(), want_c)
+        assert abs_max.cpu().numpy()[0] == want_m
