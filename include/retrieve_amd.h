@@ -453,6 +453,15 @@ int rt_quantize_int8_global(const float* x, int64_t rows, int64_t dim, const int
 int rt_pack_signs(const float* x, int64_t rows, int64_t dim, uint64_t* words,
                   rt_stream_t stream);
 
+/* Sign-OPORP codes of float32 rows [rows, dim] with one dimension a bin (dim a multiple of 64 up
+ * to 2048; signs int8 [dim], perm a permutation int64 [dim]): bit b of word w of row r is
+ * (x[r, p] * signs[p]) / max(norm, 1e-8) > 0 for p = perm[64 w + b], norm the fp32 2-norm of the
+ * row's products.
+ * Replaces: quantize_oporp_1bit's sketch and packing (retrieve/src/retrieve/indexing/quantize.py:
+ *   97-140) for k_bits = dim. */
+int rt_pack_oporp(const float* x, int64_t rows, int64_t dim, const int8_t* signs,
+                  const int64_t* perm, uint64_t* words, rt_stream_t stream);
+
 /* The exact clause filter over st::search's clause-major int32 slot layout (slots [R, N]; clause
  * c in rows clause_slots[c] .. clause_slots[c+1], -1 pads; query_values [B, C] int32, -1 =
  * inactive) -> packed bits [B, ceil(N/64)] as rt_clause_filter's mode 0, AND-ed with and_mask.

@@ -911,11 +911,21 @@ def _(valid):
     return valid.new_empty((valid.shape[0], (valid.shape[1] + 63) // 64), dtype=torch.int64)
 
 
+# The widest row whose OPORP sketch and packing are one kernel (a wave holds the row).
+OPORP_MAX_DIM = 2048
+
+
 @torch.library.custom_op("retrieve_amd::pack_signs", mutates_args=(), device_types="cuda")
-def pack_signs(values: Tensor) -> Tensor:
+def pack_signs(values: Tensor, signs: Tensor | None = None,
+               perm: Tensor | None = None) -> Tensor:
     """``[R, D]`` floats → ``[R, D // 64]`` int64, bit ``b`` of word ``w`` set iff ``values[:,
     64 w + b] > 0`` (``_pack_signs_to_int64``, ``retrieve/src/retrieve/indexing/quantize.py:
-    63-72``). fp16 / bf16 inputs are widened to fp32 first (exact, so the signs are kept)."""
+    63-72``). fp16 / bf16 inputs are widened to fp32 first (exact, so the signs are kept).
+
+    With ``signs`` (int8 ``[D]``) and ``perm`` (a permutation, int64 ``[D]``) the bits are those of
+    the Sign-OPORP sketch with one dimension a bin, ``(values * signs)[:, perm]`` over its row
+    norm (``quantize.py:97-140``), from float32 values in one kernel (``D`` up to
+    ``OPORP_MAX_DIM``)."""
     if values.dim() != 2:
         raise ValueError(f"values must be [R, D], got {tuple(values.shape)}")
     if not values.is_floating_point():
@@ -923,18 +933,32 @@ def pack_signs(values: Tensor) -> Tensor:
     r, d = values.shape
     if d % 64:
         raise ValueError(f"D must be a multiple of 64, got {d}")
+    if (signs is None) != (perm is None):
+        raise ValueError("signs and perm go together")
+    if signs is not None:
+        if values.dtype != torch.float32 or signs.dtype != torch.int8 or perm.dtype != torch.int64:
+            raise TypeError("the sketch takes float32 values, int8 signs and an int64 perm")
+        if signs.shape != (d,) or perm.shape != (d,) or d > OPORP_MAX_DIM:
+            raise ValueError(f"signs and perm must be [D] = [{d}], D at most {OPORP_MAX_DIM}")
     v = values.to(torch.float32).contiguous()
     dev = nat.require_device(v)
     out = torch.empty((r, d // 64), dtype=torch.int64, device=dev)
-    if out.numel():
-        with torch.cuda.device(dev):
+    if not out.numel():
+        return out
+    with torch.cuda.device(dev):
+        if signs is None:
             st = nat.lib().rt_pack_signs(nat.ptr(v), r, d, nat.ptr(out), nat.stream(dev))
-        nat.check(st)
+        else:
+            nat.require_device(v, signs, perm)
+            sg, pm = signs.contiguous(), perm.contiguous()
+            st = nat.lib().rt_pack_oporp(nat.ptr(v), r, d, nat.ptr(sg), nat.ptr(pm),
+                                         nat.ptr(out), nat.stream(dev))
+    nat.check(st)
     return out
 
 
 @pack_signs.register_fake
-def _(values):
+def _(values, signs=None, perm=None):
     return values.new_empty((values.shape[0], values.shape[1] // 64), dtype=torch.int64)
 
 

@@ -332,6 +332,20 @@ def _oporp_sketch(x: Tensor, signs: Tensor, perm: Tensor, k_bits: int) -> Tensor
     return binned / binned.norm(dim=-1, keepdim=True).clamp_min(1e-8)
 
 
+def _oporp_pack(x: Tensor, signs: Tensor, perm: Tensor, k_bits: int) -> Tensor:
+    """The packed signs of ``_oporp_sketch``. With one dimension a bin (``k_bits == D``) and
+    float32 rows in memory order, one kernel reads the rows once; wider bins sum several values
+    and 16-bit rows round each step, so they keep the sketch in torch, chunk by chunk."""
+    r, d = x.shape
+    if (k_bits == d <= _hip.OPORP_MAX_DIM and x.dtype == torch.float32 and x.is_contiguous()
+            and signs.shape == perm.shape == (d,) and signs.dtype == torch.int8
+            and perm.dtype == torch.int64):
+        return xops.pack_signs(x, signs, perm)
+    if r <= _CODE_CHUNK_ROWS:
+        return xops.pack_signs(_oporp_sketch(x, signs, perm, k_bits))
+    return _pack_rows(x, k_bits // 64, lambda c: _oporp_sketch(c, signs, perm, k_bits))
+
+
 class _PackedBitsKNN(RetrievalModule):
     """Hamming KNN over packed sign bits, score ``64 W - 2 popcount(q ^ item)``
     (``modules/bit_knn.py:21-81``): the full scan is ``oporp_1bit_match_topk_full``, the
@@ -403,9 +417,7 @@ class OneBitKNN(_PackedBitsKNN):
         signs = torch.randint(0, 2, (d,), generator=g, device=item_embs.device,
                               dtype=torch.int8) * 2 - 1
         perm = torch.randperm(d, generator=g, device=item_embs.device)
-        bits = _pack_rows(item_embs, self.k_bits // 64,
-                          lambda x: _oporp_sketch(x, signs, perm, self.k_bits))
-        self.register_buffer("item_bits", bits)
+        self.register_buffer("item_bits", _oporp_pack(item_embs, signs, perm, self.k_bits))
         self.register_buffer("oporp_signs", signs)
         self.register_buffer("oporp_perm", perm)
 
@@ -413,7 +425,7 @@ class OneBitKNN(_PackedBitsKNN):
         if query.dim() != 2:
             raise ValueError(f"expected 2-D [B, D] query, got shape {tuple(query.shape)}")
         k_bits = _oporp_k_bits(query.shape[1], self.k_bits)
-        return xops.pack_signs(_oporp_sketch(query, self.oporp_signs, self.oporp_perm, k_bits))
+        return _oporp_pack(query, self.oporp_signs, self.oporp_perm, k_bits)
 
 
 def _rederive_k_bits(module: OneBitKNN, incompatible_keys) -> None:

@@ -78,3 +78,31 @@ def test_global(n, d, offset):
         want_c, want_m = oq.quantize_int8_global(x, rows)
         assert np.array_equal(codes.cpu().numpy(), want_c)
         assert abs_max.cpu().numpy()[0] == want_m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("n,d", [(1, 64), (67, 64), (5, 128), (9, 192), (3, 256), (6, 320),
+                                 (4, 512), (5, 1024), (3, 2048), (140_003, 64)])
+def test_oporp(n, d, offset):
+    """The fused sketch and packing against the sketch's own steps in torch, with rows of zeros,
+    denormals, huge values (an infinite norm), NaN and infinities."""
+    from retrieve_amd.modules import _oporp_sketch
+
+    print(f"oporp n={n} d={d} offset={offset}", flush=True)
+    g = rng(n * 5 + d)
+    x = _table(g, n, d)
+    if n > 5:
+        x[4, d // 2] = np.nan
+        x[5, 1] = np.inf
+        x[5, 2] = -np.inf
+    flat = torch.zeros(n * d + offset, device="cuda:0")
+    flat[offset:] = torch.from_numpy(x).reshape(-1).to("cuda:0")
+    xt = flat[offset:].view(n, d)
+    signs = torch.from_numpy(g.choice([-1, 1], d).astype(np.int8)).to("cuda:0")
+    perm = torch.from_numpy(g.permutation(d)).to("cuda:0")
+    got = torch.ops.retrieve_amd.pack_signs(xt, signs, perm)
+    want = torch.ops.retrieve_amd.pack_signs(_oporp_sketch(xt, signs, perm, d))
+    assert torch.equal(got, want)
+    assert np.array_equal(got.cpu().numpy(),
+                          oq.pack_signs(_oporp_sketch(xt, signs, perm, d).cpu().numpy()))
