@@ -503,7 +503,7 @@ static int launch_merge_grid(const MergeArgs& m, int64_t blocks, hipStream_t str
 }
 
 // A small batch's merge is split when the caller gave room: each query's lists go to up to
-// kMergeParts workgroups (a part at least kMergeMinPartSlots lists), each keeping its part's
+// kMergeParts workgroups (a part at least part_slots lists), each keeping its part's
 // best k in part_buf, then one workgroup per query merges those (flat, kMergeParts * k
 // entries) with the call's own outputs. Same results: the best k of the union is among the
 // parts' best k.
@@ -514,9 +514,9 @@ int launch_merge(const MergeArgs& m, hipStream_t stream) {
                static_cast<long long>(kMaxK), m.k);
   RT_CHECK_ARG(m.S >= 1 && m.S <= kMaxMergeSlots, "too many scan lists per query");
   if (m.B == 0) return kOk;
-  int64_t parts = m.S / kMergeMinPartSlots;
+  int64_t parts = m.S / (m.part_slots > 0 ? m.part_slots : kMergeMinPartSlots);
   parts = parts < kMergeParts ? parts : kMergeParts;
-  if (m.part_buf == nullptr || m.B > kMergeSplitMaxB || parts < 2) {
+  if (m.part_buf == nullptr || parts < 2) {
     MergeArgs one = m;
     one.parts = 1;
     one.part_out = nullptr;

@@ -91,6 +91,7 @@ struct MergeArgs {
   // splits a small batch's lists into parts, each a workgroup keeping its part's best k there,
   // and merges those (flat) in a second launch.
   uint64_t* part_buf;
+  int part_slots;  // lists a part holds at least (0: kMergeMinPartSlots)
   // (set by launch_merge) parts per query, and the parts' output in the first launch
   int parts;
   uint64_t* part_out;

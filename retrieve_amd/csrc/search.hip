@@ -14,9 +14,9 @@
 // Keys: the int32 dot (divisor -1), or the fp16 score fp16(float(dot) / divisor) of the serving
 // path (index_mm_helpers.cuh:48-65), ordered as fp16 values (ties merge distinct dots).
 //
-// The range scan is the candidate kernel's layout: a group of L lanes loads one item row with
-// 16-byte loads and reduces its v_dot4 partial sums by xor-shuffles; every wave keeps a
-// candidate list under a rising threshold; the shared merge picks the k best composites.
+// The range scan filters 64 slots of a wave at a time and queues the ones that pass; queued rows
+// are scored by groups of lanes, several rows in flight a group; every wave keeps a candidate
+// list under a rising threshold; the shared merge picks the k best composites.
 #include "scan_common.h"
 #include "wave_lists.h"
 
@@ -29,7 +29,7 @@ constexpr int64_t kQuantMaxGrid = 4096;  // sixteen workgroups a CU: two rounds 
 constexpr int kIvfThreads = 256;
 constexpr int kIvfWaves = kIvfThreads / kWave;
 constexpr int kIvfMaxProbe = 1024;
-constexpr int kIvfMaxWgsPerRow = 64;
+constexpr int kIvfMaxWgsPerRow = 256;
 
 // ---- query quantization (A1 / A2) ------------------------------------------------------------
 
@@ -425,15 +425,22 @@ struct IvfArgs {
   int* list_counts;
 };
 
+constexpr int kIvfMaxClauses = 32;
+constexpr int kIvfUnroll = 4;  // 64-slot steps a wave filters together
+constexpr int kIvfQueue = kIvfUnroll * kWave + kWave;  // a step's slots and an unscored rest
+
 // The row's 2 n_probe slot ranges in slot order: range j < n_probe is probe j's full warps
 // (its first len_j / 32 * 32 items), range n_probe + j probe j's remaining len_j % 32 items.
 // start[r] is range r's first sorted position and prefix[r] the slots before it (prefix[2n] =
 // total, clamped at width). Invalid clusters, or clusters reaching outside the table, are empty.
-__device__ inline int64_t load_ranges(const IvfArgs& a, int64_t b, int64_t* start,
-                                      int64_t* prefix) {
+// The lengths are summed by a block scan (a serial sum over 2 n_probe LDS entries took longer
+// than a workgroup's scoring). `part` holds kIvfThreads / kWave int64.
+__device__ inline uint32_t load_ranges(const IvfArgs& a, int64_t b, int64_t* start,
+                                       uint32_t* prefix, int64_t* part) {
   const int tid = threadIdx.x;
-  const int64_t np = a.n_probe;
-  for (int64_t j = tid; j < np; j += blockDim.x) {
+  const int np = static_cast<int>(a.n_probe);
+  const int nr = 2 * np;
+  for (int j = tid; j < np; j += kIvfThreads) {
     const int64_t c = a.probe_ids[b * np + j];
     int64_t s = 0;
     int64_t len = 0;
@@ -442,35 +449,57 @@ __device__ inline int64_t load_ranges(const IvfArgs& a, int64_t b, int64_t* star
       len = a.cluster_sizes[c];
       if (s < 0 || len < 0 || s > a.N || len > a.N - s) len = 0;
     }
+    // (a range longer than the width ends the row either way)
     const int64_t full = len / 32 * 32;
     start[j] = s;
-    prefix[j + 1] = full;
+    prefix[j + 1] = static_cast<uint32_t>(full < a.width ? full : a.width);
     start[np + j] = s + full;
-    prefix[np + j + 1] = len - full;
+    prefix[np + j + 1] = static_cast<uint32_t>(len - full);
   }
   __syncthreads();
-  if (tid == 0) {
-    prefix[0] = 0;
-    for (int64_t r = 0; r < 2 * np; ++r) {
-      const int64_t t = prefix[r] + prefix[r + 1];
-      prefix[r + 1] = t < a.width ? t : a.width;
+  // each thread takes a run of lengths, then the runs' sums are scanned across the block
+  const int per = (nr + kIvfThreads - 1) / kIvfThreads;
+  int64_t run = 0;
+  for (int i = 0; i < per; ++i) {
+    const int r = tid * per + i;
+    if (r < nr) run += prefix[r + 1];
+  }
+  int64_t incl = run;
+  const int lane = lane_id();
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int64_t t = __shfl_up(incl, off);
+    incl += lane >= off ? t : 0;
+  }
+  if (lane == kWave - 1) part[tid / kWave] = incl;
+  __syncthreads();
+  int64_t sum = incl - run;
+  for (int w = 0; w < tid / kWave; ++w) sum += part[w];
+  for (int i = 0; i < per; ++i) {
+    const int r = tid * per + i;
+    if (r < nr) {
+      sum += prefix[r + 1];
+      prefix[r + 1] = static_cast<uint32_t>(sum < a.width ? sum : a.width);
     }
   }
+  if (tid == 0) prefix[0] = 0;
   __syncthreads();
-  return prefix[2 * np];
+  return prefix[nr];
 }
 
-// LDS bytes of a row's ranges (start[2 n], prefix[2 n + 1]).
-inline size_t ranges_lds(int64_t n_probe) {
-  return static_cast<size_t>(4 * n_probe + 1) * sizeof(int64_t);
+// LDS bytes of a row's ranges (start[2 n], the scan's partial sums, prefix[2 n + 1]), rounded to
+// whole 16-byte chunks.
+__host__ __device__ inline size_t ranges_lds(int64_t n_probe) {
+  return (static_cast<size_t>(2 * n_probe + kIvfWaves) * sizeof(int64_t) +
+          static_cast<size_t>(2 * n_probe + 1) * sizeof(uint32_t) + 15) / 16 * 16;
 }
 
 // the range holding slot s: the last j with prefix[j] <= s
-__device__ inline int64_t range_of(const int64_t* prefix, int64_t n, int64_t s) {
-  int64_t lo = 0;
-  int64_t hi = n - 1;
+__device__ inline int range_of(const uint32_t* prefix, int n, uint32_t s) {
+  int lo = 0;
+  int hi = n - 1;
   while (lo < hi) {
-    const int64_t mid = (lo + hi + 1) >> 1;
+    const int mid = (lo + hi + 1) >> 1;
     if (prefix[mid] <= s) {
       lo = mid;
     } else {
@@ -486,58 +515,102 @@ __device__ inline uint32_t search_key(int32_t dot, int divisor) {
   return key_of_f32(static_cast<float>(h));
 }
 
-// Bit `off` of probe j's payload in row b's Bloom words (out of range: no match), as
-// fused_kmean_ann_with_partial_masks reads it (fused_kmean_ann_cuda.cu:2264-2501).
-__device__ inline bool payload_bit(const IvfArgs& a, int64_t b, int64_t j, int64_t off) {
-  const int64_t e = b * a.n_probe + j;
-  if (e >= a.p_entries) return false;
-  const int64_t w0 = e == 0 ? 0 : static_cast<int64_t>(a.pcum[e - 1]);
-  const int64_t bit = static_cast<int64_t>(a.pfirst[e]) + off;
-  const int64_t w = w0 + (bit >> 6);
-  return bit >= 0 && w < a.p_words && ((a.pwords[w] >> (63 - (bit & 63))) & 1ull);
-}
+// The row's active exact clauses (LDS): value, slot rows [r0, r1) inside the table, reverse. A
+// doc passes a clause when one of its values equals the query's, negated for a reverse clause
+// (fork_filters.cuh:15-41).
+struct IvfClauses {
+  int n;
+  int32_t value[kIvfMaxClauses];
+  int32_t reverse[kIvfMaxClauses];
+  int64_t r0[kIvfMaxClauses];
+  int64_t r1[kIvfMaxClauses];
+};
 
-// The exact recheck of one probed doc (fork_filters.cuh:15-41): every active clause matches
-// (one of the doc's values equals the query's), negated for a reverse clause.
-__device__ inline bool exact_pass(const IvfArgs& a, int64_t b, int64_t pos, uint32_t rev_mask) {
-  const int32_t* q = a.qv + b * a.C;
-  uint32_t active = 0;
-  uint32_t match = 0;
-  for (int c = 0; c < a.C; ++c) {
-    const int32_t v = q[c];
-    if (v == -1) continue;
-    active |= 1u << c;
-    bool eq = false;
-    const int64_t r0 = a.cslots[c] > 0 ? a.cslots[c] : 0;
-    const int64_t r1 = a.cslots[c + 1] < a.R ? a.cslots[c + 1] : a.R;  // rows inside the table
-    for (int64_t r = r0; r < r1; ++r) eq |= a.slots[r * a.N + pos] == v;
-    match |= eq ? 1u << c : 0u;
+// Fills the row's clauses in clause order; called by the block, followed by a barrier.
+__device__ inline void load_clauses(const IvfArgs& a, int64_t b, IvfClauses* cl) {
+  const int tid = threadIdx.x;
+  if (tid >= kWave) return;
+  const bool have = a.qv != nullptr && tid < a.C;
+  const int32_t v = have ? a.qv[b * a.C + tid] : -1;
+  const uint64_t active = __ballot(v != -1);
+  if (v != -1) {
+    const int i = __popcll(active & ((1ull << tid) - 1ull));
+    // (values below -1 stand for "no doc holds it")
+    cl->value[i] = v < -1 ? INT32_MIN : v;
+    cl->reverse[i] = a.reverse[tid] != 0;
+    const int64_t r0 = a.cslots[tid];
+    const int64_t r1 = a.cslots[tid + 1];
+    cl->r0[i] = r0 > 0 ? r0 : 0;
+    cl->r1[i] = r1 < a.R ? r1 : a.R;
   }
-  return ((match ^ rev_mask) & active) == active;
+  if (tid == 0) cl->n = __popcll(active);
 }
 
-template <int L, int NC>
+// The LDS of a scan workgroup beside the ranges.
+struct IvfLds {
+  int64_t qpos[kIvfWaves][kIvfQueue];  // per wave: sorted positions of the slots that passed
+  uint32_t qslot[kIvfWaves][kIvfQueue];
+  IvfClauses clauses;
+  int cnt[kIvfWaves];
+};
+
+__host__ __device__ constexpr size_t ivf_lds_bytes() { return (sizeof(IvfLds) + 15) / 16 * 16; }
+
+// One workgroup's share of a row's slots. Each wave takes one contiguous run of them: the range
+// of a slot is found once by bisection and then only walked forward. kIvfUnroll x 64 slots a
+// step are filtered lane by lane (neighbouring slots are neighbouring docs, so their mask words
+// and attribute rows coalesce, kIvfUnroll loads in flight a lane), and those that pass are
+// queued in LDS; then the queue is scored R * V rows at a time: a group of L lanes holds the
+// query's chunks and loads V rows of NC 16-byte chunks a lane before it uses the first, and V
+// partial dots are folded across the lanes by halves (each exchange hands half of the values to
+// the other lane), so a lane ends with one row's dot. Bound: the latency of the dependent loads
+// (filter, then row), hidden by the rows in flight and eight workgroups a CU. Docs that the
+// filter drops cost no row load and no reduction, and plain (not streaming) loads keep rows that
+// other queries of the batch probe in the caches. Filtering and scoring one slot a group step by
+// step, the same scans took (before, now): 3M x 128, 64 queries of 64 probes in 1024 lists under
+// the exact filter 992, 80 us; 10M x 256, 16 queries of 128 probes in 4096 lists under Bloom
+// words and the recheck 917, 56 us; unfiltered 2M x 512, 16 queries, the whole search 587, 301.
+template <int L, int NC, int V>
 __global__ void __launch_bounds__(kIvfThreads) ivf_scan_kernel(IvfArgs a) {
   constexpr int R = kWave / L;
-  extern __shared__ uint64_t smem[];
-  const int64_t nr = 2 * a.n_probe;  // slot ranges
+  constexpr int E = R * V;  // rows scored at a time
+  static_assert(V <= L && E <= kWave, "a lane owns at most one of the rows scored together");
+  extern __shared__ __attribute__((aligned(16))) uint64_t smem[];
+  const int nr = static_cast<int>(2 * a.n_probe);  // slot ranges
   int64_t* start = reinterpret_cast<int64_t*>(smem);
-  int64_t* prefix = start + nr;
-  uint64_t* scratch = reinterpret_cast<uint64_t*>(prefix + nr + 1);
+  int64_t* part = start + nr;
+  uint32_t* prefix = reinterpret_cast<uint32_t*>(part + kIvfWaves);
+  char* after = reinterpret_cast<char*>(smem) + ranges_lds(a.n_probe);
+  IvfLds* lds = reinterpret_cast<IvfLds*>(after);
+  uint64_t* scratch = reinterpret_cast<uint64_t*>(after + ivf_lds_bytes());
+  // per probe: the payload's first Bloom word and its first doc's bit there (-1: no entry)
+  uint32_t* pw = reinterpret_cast<uint32_t*>(scratch + kIvfWaves * a.capw);
+  int32_t* pb = reinterpret_cast<int32_t*>(pw + a.n_probe);
   const int tid = threadIdx.x;
   const int lane = lane_id();
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = lane / L;
   const int gl = lane % L;
-  int* cnt_lds = reinterpret_cast<int*>(scratch + kIvfWaves * a.capw);
   const int64_t b = blockIdx.y;
-  const int64_t gx = gridDim.x;
-  const int64_t S = gx * kIvfWaves;
-  const int64_t slot_list = static_cast<int64_t>(blockIdx.x) * kIvfWaves + wave;
-  uint64_t* list = a.lists + (b * S + slot_list) * a.capw;
+  const int64_t S = static_cast<int64_t>(gridDim.x) * kIvfWaves;
+  const int64_t list_at = static_cast<int64_t>(blockIdx.x) * kIvfWaves + wave;
+  uint64_t* list = a.lists + (b * S + list_at) * a.capw;
   scratch += wave * a.capw;
+  int64_t* qpos = lds->qpos[wave];
+  uint32_t* qslot = lds->qslot[wave];
 
-  const int64_t total = load_ranges(a, b, start, prefix);
+  load_clauses(a, b, &lds->clauses);
+  if (a.pwords != nullptr) {
+    for (int j = tid; j < a.n_probe; j += kIvfThreads) {
+      const int64_t e = b * a.n_probe + j;
+      const bool have = e < a.p_entries;
+      pw[j] = have && e > 0 ? static_cast<uint32_t>(a.pcum[e - 1]) : 0u;
+      pb[j] = have ? static_cast<int32_t>(a.pfirst[e]) : INT32_MIN;
+    }
+  }
+  const uint32_t total = load_ranges(a, b, start, prefix, part);  // (its barriers cover both)
+  const int ncl = lds->clauses.n;
+
   const int nchunks = a.RB / 16;
   v4i qv[NC];
 #pragma unroll
@@ -547,60 +620,174 @@ __global__ void __launch_bounds__(kIvfThreads) ivf_scan_kernel(IvfArgs a) {
                         : v4i{0, 0, 0, 0};
   }
   const uint64_t* mrow = a.mask != nullptr ? a.mask + b * a.mask_words : nullptr;
-  uint32_t rev_mask = 0;
-  if (a.qv != nullptr) {
-    for (int c = 0; c < a.C; ++c) rev_mask |= a.reverse[c] != 0 ? 1u << c : 0u;
-  }
 
   uint64_t tau = 0;
-  int cnt = 0;
-  const int64_t step = gx * kIvfWaves * R;
-  for (int64_t base = slot_list * R; base < total; base += step) {
-    const int64_t s = base + grp;
-    bool ok = s < total;
-    int64_t pos = 0;
-    if (ok) {
-      const int64_t j = range_of(prefix, nr, s);
-      pos = start[j] + (s - prefix[j]);
-      if (mrow != nullptr) {
-        ok = (mrow[pos >> 6] >> (63 - (pos & 63))) & 1ull;
-      } else if (a.pwords != nullptr) {
-        const int64_t p = j < a.n_probe ? j : j - a.n_probe;  // the probe of range j
-        ok = payload_bit(a, b, p, pos - start[p]);
-      }
-      if (ok && a.qv != nullptr) ok = exact_pass(a, b, pos, rev_mask);
-    }
-    int32_t dot = 0;
-    if (ok) {
-      const int8_t* row = a.items + pos * a.RB;
+  int cnt = 0;     // entries of this wave's list
+  int queued = 0;  // slots waiting to be scored
+  // the row of the scored batch that this lane owns: the folds below leave lane gl (its low bits
+  // reversed) with row v of its group
+  int own = 0;
+#pragma unroll
+  for (int i = 1, v = V / 2; v > 0; i <<= 1, v >>= 1) own |= (gl & i) ? v : 0;
+
+  // scores queue entries [0, n), n <= E
+  auto score = [&](int at, int n) {
+    v4i x[V][NC];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const int e = v * R + grp;
+      const int8_t* row = a.items + qpos[at + (e < n ? e : 0)] * a.RB;
 #pragma unroll
       for (int j = 0; j < NC; ++j) {
         const int c = gl + j * L;
-        if (c < nchunks) {
-          const v4i x = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(row + c * 16));
+        x[v][j] = c < nchunks && e < n ? *reinterpret_cast<const v4i*>(row + c * 16)
+                                       : v4i{0, 0, 0, 0};
+      }
+    }
+    int32_t d[V];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dot = __builtin_amdgcn_sdot4(x[e], qv[j][e], dot, false);
+    for (int v = 0; v < V; ++v) {
+      d[v] = 0;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          d[v] = __builtin_amdgcn_sdot4(x[v][j][i], qv[j][i], d[v], false);
         }
       }
     }
 #pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off);
-    const uint64_t c = composite(search_key(dot, a.divisor), static_cast<uint32_t>(s));
-    const bool keep = ok && gl == 0 && c >= tau;
-    const uint64_t bal = __ballot(keep);
-    if (bal != 0ull) {
-      const int before = __popcll(bal & ((1ull << lane) - 1ull));
-      if (keep) list[cnt + before] = c;
-      cnt += __popcll(bal);
-      if (cnt > a.capw - R) {
-        if (lane == 0) cnt_lds[wave] = cnt;
-        const uint64_t nt = wave_compact(list, &cnt_lds[wave], scratch, a.capw, a.k);
-        cnt = cnt_lds[wave];
-        tau = nt > tau ? nt : tau;
+    for (int off = 1, half = V / 2; half > 0; off <<= 1, half >>= 1) {
+      const bool up = (gl & off) != 0;
+#pragma unroll
+      for (int v = 0; v < half; ++v) {
+        const int32_t send = up ? d[v] : d[v + half];
+        const int32_t keep = up ? d[v + half] : d[v];
+        d[v] = keep + __shfl_xor(send, off);
       }
     }
+#pragma unroll
+    for (int off = V; off < L; off <<= 1) d[0] += __shfl_xor(d[0], off);
+    const int e = own * R + grp;
+    const bool mine = gl < V && e < n;
+    const uint32_t s = qslot[at + (mine ? e : 0)];
+    const uint64_t c = composite(search_key(d[0], a.divisor), s);
+    const bool keep = mine && c >= tau;
+    const uint64_t bal = __ballot(keep);
+    if (bal == 0ull) return;
+    if (keep) list[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = c;
+    cnt += __popcll(bal);
+    if (cnt > a.capw - E) {
+      if (lane == 0) lds->cnt[wave] = cnt;
+      const uint64_t nt = wave_compact(list, &lds->cnt[wave], scratch, a.capw, a.k);
+      cnt = lds->cnt[wave];
+      tau = nt > tau ? nt : tau;
+    }
+  };
+
+  // this wave's slots: a run of whole 64s
+  const uint32_t span = static_cast<uint32_t>(
+      (static_cast<uint64_t>(total) + static_cast<uint64_t>(S) * kWave - 1) /
+      (static_cast<uint64_t>(S) * kWave) * kWave);
+  const uint64_t first = static_cast<uint64_t>(list_at) * span;
+  const uint32_t s0 = first < total ? static_cast<uint32_t>(first) : total;
+  const uint32_t s1 = total - s0 < span ? total : s0 + span;
+  int jr = s0 < s1 ? range_of(prefix, nr, s0) : 0;  // the range of the step's first slot
+  for (uint32_t base = s0; base < s1; base += kIvfUnroll * kWave) {
+    bool ok[kIvfUnroll];
+    int64_t pos[kIvfUnroll];
+    const uint64_t* word[kIvfUnroll];
+    int bit[kIvfUnroll];
+    int j = jr;
+#pragma unroll
+    for (int u = 0; u < kIvfUnroll; ++u) {
+      const uint32_t s = base + u * kWave + lane;  // (below total + 256 < 2^32)
+      ok[u] = s < s1 && s >= base;
+      while (true) {
+        const bool next = ok[u] && s >= prefix[j + 1];
+        if (!__any(next)) break;
+        j += next ? 1 : 0;
+      }
+      pos[u] = ok[u] ? start[j] + (s - prefix[j]) : 0;
+      word[u] = nullptr;
+      bit[u] = 0;
+      if (mrow != nullptr) {
+        word[u] = mrow + (pos[u] >> 6);
+        bit[u] = 63 - static_cast<int>(pos[u] & 63);
+      } else if (a.pwords != nullptr) {
+        // as fused_kmean_ann_with_partial_masks reads it (fused_kmean_ann_cuda.cu:2264-2501);
+        // outside the words: no match
+        const int p = j < a.n_probe ? j : j - static_cast<int>(a.n_probe);
+        const int64_t at = static_cast<int64_t>(pb[p]) + (pos[u] - start[p]);
+        const int64_t w = static_cast<int64_t>(pw[p]) + (at >> 6);
+        ok[u] = ok[u] && at >= 0 && pb[p] != INT32_MIN && w < a.p_words;
+        word[u] = a.pwords + w;
+        bit[u] = 63 - static_cast<int>(at & 63);
+      }
+      // (lanes are in slot order, so the last one holds the furthest range; lanes past the run
+      // keep theirs)
+      j = __builtin_amdgcn_readlane(j, kWave - 1);
+    }
+    jr = j;
+    if (mrow != nullptr || a.pwords != nullptr) {
+      uint64_t m[kIvfUnroll];
+#pragma unroll
+      for (int u = 0; u < kIvfUnroll; ++u) m[u] = ok[u] ? *word[u] : 0ull;
+#pragma unroll
+      for (int u = 0; u < kIvfUnroll; ++u) ok[u] = ok[u] && ((m[u] >> bit[u]) & 1ull);
+    }
+    for (int c = 0; c < ncl; ++c) {
+      const int32_t v = lds->clauses.value[c];
+      bool eq[kIvfUnroll] = {};
+      for (int64_t r = lds->clauses.r0[c]; r < lds->clauses.r1[c]; ++r) {
+        const int32_t* slot_row = a.slots + r * a.N;
+        int32_t x[kIvfUnroll];
+#pragma unroll
+        for (int u = 0; u < kIvfUnroll; ++u) x[u] = ok[u] ? slot_row[pos[u]] : -1;
+#pragma unroll
+        for (int u = 0; u < kIvfUnroll; ++u) eq[u] |= x[u] == v;
+      }
+      const bool rev = lds->clauses.reverse[c] != 0;
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < kIvfUnroll; ++u) {
+        ok[u] = ok[u] && eq[u] != rev;
+        any |= ok[u];
+      }
+      if (!__any(any)) break;
+    }
+#pragma unroll
+    for (int u = 0; u < kIvfUnroll; ++u) {
+      const uint64_t bal = __ballot(ok[u]);
+      if (ok[u]) {
+        const int at = queued + __popcll(bal & ((1ull << lane) - 1ull));
+        qpos[at] = pos[u];
+        qslot[at] = base + u * kWave + lane;
+      }
+      queued += __popcll(bal);
+    }
+    wave_sync_memory();
+    const bool last = s1 - base <= kIvfUnroll * kWave;
+    int at = 0;
+    for (; queued - at >= E; at += E) score(at, E);
+    if (last) {
+      if (at < queued) score(at, queued - at);
+      break;
+    }
+    // the remainder (fewer than E <= 64) moves to the front
+    queued -= at;
+    if (at > 0 && queued > 0) {
+      const int64_t mp = lane < queued ? qpos[at + lane] : 0;
+      const uint32_t ms = lane < queued ? qslot[at + lane] : 0;
+      wave_sync_memory();
+      if (lane < queued) {
+        qpos[lane] = mp;
+        qslot[lane] = ms;
+      }
+    }
+    wave_sync_memory();
   }
-  if (lane == 0) a.list_counts[b * S + slot_list] = cnt;
+  if (lane == 0) a.list_counts[b * S + list_at] = cnt;
 }
 
 // ---- epilogue -------------------------------------------------------------------------------
@@ -626,10 +813,10 @@ struct EpiArgs {
 __global__ void __launch_bounds__(kIvfThreads) search_epilogue_kernel(EpiArgs e) {
   extern __shared__ uint64_t smem[];
   const int64_t b = blockIdx.x;
-  const int64_t nr = e.ranges ? 2 * e.a.n_probe : 0;  // slot ranges
+  const int nr = e.ranges ? static_cast<int>(2 * e.a.n_probe) : 0;  // slot ranges
   int64_t* start = reinterpret_cast<int64_t*>(smem);
-  int64_t* prefix = start + nr;
-  if (e.ranges) load_ranges(e.a, b, start, prefix);
+  uint32_t* prefix = reinterpret_cast<uint32_t*>(start + nr + kIvfWaves);
+  if (e.ranges) load_ranges(e.a, b, start, prefix, start + nr);
   const float qs = e.q_scales[b];
   const float gs = e.global_scale[0];
   for (int64_t i = threadIdx.x; i < e.k; i += blockDim.x) {
@@ -639,7 +826,7 @@ __global__ void __launch_bounds__(kIvfThreads) search_epilogue_kernel(EpiArgs e)
     if (x >= 0) {
       int64_t pos = x;
       if (e.ranges) {
-        const int64_t j = range_of(prefix, nr, x);
+        const int j = range_of(prefix, nr, static_cast<uint32_t>(x));
         pos = start[j] + (x - prefix[j]);
       }
       if (pos >= 0 && pos < e.n_perm) {
@@ -658,16 +845,39 @@ __global__ void __launch_bounds__(kIvfThreads) search_epilogue_kernel(EpiArgs e)
   }
 }
 
-template <int L, int NC>
-static void launch_ivf(const IvfArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
+template <int L, int NC, int V>
+static int launch_ivf(const IvfArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
   if (lds > 64 * 1024) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&ivf_scan_kernel<L, NC>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    RT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&ivf_scan_kernel<L, NC, V>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     static_cast<int>(lds)));
   }
-  ivf_scan_kernel<L, NC><<<grid, kIvfThreads, lds, stream>>>(a);
+  ivf_scan_kernel<L, NC, V><<<grid, kIvfThreads, lds, stream>>>(a);
+  RT_CHECK_HIP(hipGetLastError());
+  return kOk;
+}
+
+// L lanes of NC chunks a row: narrow groups fold few partial dots (8 lanes take a 128-byte line
+// together); V rows in flight a group, 64 or fewer registers of them.
+static int dispatch_ivf(int64_t D, const IvfArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
+  if (D <= 64) return launch_ivf<4, 1, 4>(a, grid, lds, stream);
+  if (D <= 128) return launch_ivf<8, 1, 8>(a, grid, lds, stream);
+  if (D <= 192) return launch_ivf<4, 3, 4>(a, grid, lds, stream);
+  if (D <= 256) return launch_ivf<8, 2, 8>(a, grid, lds, stream);
+  if (D <= 512) return launch_ivf<16, 2, 8>(a, grid, lds, stream);
+  if (D <= 1024) return launch_ivf<32, 2, 8>(a, grid, lds, stream);
+  if (D <= 2048) return launch_ivf<64, 2, 8>(a, grid, lds, stream);
+  if (D <= 4096) return launch_ivf<64, 4, 4>(a, grid, lds, stream);
+  return launch_ivf<64, 8, 2>(a, grid, lds, stream);
 }
 
 static int ivf_capw(int64_t k) { return static_cast<int>(next_pow2(k + kWave)); }
+
+// A row's lists hold up to k entries each (a wave starts without a bound), so its merge is split
+// from far fewer lists than a seeded scan's, up to a batch whose merges fill the CUs: 64 rows of
+// 128 lists and 19K entries 63 us in one launch, 32 + 14 us split.
+constexpr int kIvfPartSlots = 16;
+constexpr int64_t kIvfSplitMaxB = 128;
 
 static int64_t ivf_gx(int64_t B, int64_t width) {
   int64_t gx = cdiv(2048, B > 0 ? B : 1);
@@ -793,7 +1003,8 @@ extern "C" size_t rt_ivf_search_workspace(int64_t B, int64_t width, int64_t k) {
   const int64_t S = ivf_gx(B, width) * kIvfWaves;
   return align_up(static_cast<size_t>(B * S) * ivf_capw(k) * sizeof(uint64_t), 256) +
          align_up(static_cast<size_t>(B * S) * sizeof(int), 256) +
-         align_up(static_cast<size_t>(B * k) * sizeof(float), 256);
+         align_up(static_cast<size_t>(B * k) * sizeof(float), 256) +
+         (B <= kIvfSplitMaxB ? static_cast<size_t>(B) * kMergeParts * k * sizeof(uint64_t) : 0);
 }
 
 // Top-k over each row's probed ranges of int8 codes (slots, ties to the lower slot), then the
@@ -862,30 +1073,16 @@ static int ivf_search(const int8_t* q_codes, const float* q_scales, int64_t B,
   a.list_counts = reinterpret_cast<int*>(ws);
   ws += align_up(static_cast<size_t>(B * S) * sizeof(int), 256);
   void* raw = ws;
+  ws += align_up(static_cast<size_t>(B * k) * sizeof(float), 256);
+  uint64_t* parts = B <= kIvfSplitMaxB ? reinterpret_cast<uint64_t*>(ws) : nullptr;
   const int score_kind = divisor == -1 ? kScoreI32 : kScoreF32;
   if (n_probe > 0) {
-    const size_t lds = ranges_lds(n_probe) +
+    const size_t lds = ranges_lds(n_probe) + ivf_lds_bytes() +
                        static_cast<size_t>(kIvfWaves) * capw * sizeof(uint64_t) +
-                       kIvfWaves * sizeof(int);
+                       static_cast<size_t>(n_probe) * 2 * sizeof(uint32_t);
     const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(B));
-    if (D <= 1024) {
-      switch (D) {
-        case 16: launch_ivf<1, 1>(a, grid, lds, stream); break;
-        case 32: launch_ivf<2, 1>(a, grid, lds, stream); break;
-        case 64: launch_ivf<4, 1>(a, grid, lds, stream); break;
-        case 128: launch_ivf<8, 1>(a, grid, lds, stream); break;
-        case 256: launch_ivf<16, 1>(a, grid, lds, stream); break;
-        case 512: launch_ivf<32, 1>(a, grid, lds, stream); break;
-        default: launch_ivf<64, 1>(a, grid, lds, stream); break;
-      }
-    } else if (D <= 2048) {
-      launch_ivf<64, 2>(a, grid, lds, stream);
-    } else if (D <= 4096) {
-      launch_ivf<64, 4>(a, grid, lds, stream);
-    } else {
-      launch_ivf<64, 8>(a, grid, lds, stream);
-    }
-    RT_CHECK_HIP(hipGetLastError());
+    int st = dispatch_ivf(D, a, grid, lds, stream);
+    if (st != kOk) return st;
     MergeArgs m{};
     m.lists = a.lists;
     m.counts = a.list_counts;
@@ -897,7 +1094,9 @@ static int ivf_search(const int8_t* q_codes, const float* q_scales, int64_t B,
     m.out_ids = out_ids;
     m.out_scores = raw;
     m.score_kind = score_kind;
-    const int st = launch_merge(m, stream);
+    m.part_buf = parts;
+    m.part_slots = kIvfPartSlots;
+    st = launch_merge(m, stream);
     if (st != kOk) return st;
   } else {
     const int st = launch_pad(out_ids, raw, B, k, score_kind, stream);

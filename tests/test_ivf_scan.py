@@ -1,0 +1,73 @@
+"""The IVF scan at the edges of its work split: row widths on every lane layout, lists shorter than
+a warp and empty ones, a width that cuts the row, one wave's run ending inside a step, queues that
+fill exactly, and every filter form, against the oracle bit for bit."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import filters as of
+from oracle import silvertorch as ost
+from tests.conftest import rng
+from tests.test_int8_scan import _pack
+from tests.test_search import _ivf, _run, _t
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [16, 64, 80, 128, 192, 208, 256, 512, 528, 1024, 1040, 2064, 4112])
+def test_widths(dev, d):
+    g = rng(300 + d)
+    n, b, k, lists = 3000, 3, 40, 30
+    items, offsets, sizes, perm = _ivf(g, n, d, lists)
+    q = g.standard_normal((b, d)).astype(np.float32)
+    probes = np.stack([g.permutation(lists)[:12] for _ in range(b)]).astype(np.int64)
+    ids, sc = _run(dev, q, probes, offsets, sizes, items, perm, 1.5, k, n, 128)
+    want = ost.search(q, probes, offsets, sizes, items, perm, [1.5], k, n, 128)
+    assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+
+
+@pytest.mark.parametrize("b,n,n_lists,n_probe,k,width", [
+    (1, 60_000, 200, 190, 1000, 60_000),   # one row over many workgroups, lists filling up
+    (2, 4096, 2, 2, 10, 4096),             # whole runs of 64
+    (3, 700, 400, 300, 7, 700),            # lists of one or two docs: remainders only
+    (130, 5000, 20, 5, 20, 1000),          # more rows than split merges, the width cuts rows
+    (2, 5000, 1024, 1024, 33, 4000),       # the most probes
+    (1, 40, 3, 1, 50, 64),                 # fewer slots than k
+])
+def test_layouts(dev, b, n, n_lists, n_probe, k, width):
+    """Unfiltered, under a full-N mask and under exact clauses with several values a doc, a
+    reverse clause and a value no doc may hold."""
+    g = rng(310 + n + b)
+    d, c, vals = 128, 3, 2
+    items, offsets, sizes, perm = _ivf(g, n, d, n_lists)
+    empty = g.random(n_lists) < 0.1  # lists cut to nothing
+    sizes = np.where(empty, 0, sizes)
+    q = g.standard_normal((b, d)).astype(np.float32)
+    probes = np.stack([g.permutation(n_lists)[:n_probe] for _ in range(b)]).astype(np.int64)
+    probes[0, -1] = n_lists + 3  # no such list
+    args = (dev, q, probes, offsets, sizes, items, perm, 0.7, k, width)
+    want_args = (q, probes, offsets, sizes, items, perm, [0.7], k, width)
+    ids, sc = _run(*args)
+    want = ost.search(*want_args)
+    assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+    valid = g.random((b, n)) < 0.15
+    valid[-1] = False
+    ids, sc = _run(*args, filtering_bit_mask=_t(dev, _pack(valid)))
+    want = ost.search(*want_args, valid=valid)
+    assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+    attrs = g.integers(0, 4, (n, c, vals)).astype(np.int64)
+    attrs[g.random((n, c, vals)) < 0.3] = -1
+    qa = g.integers(0, 4, (b, c)).astype(np.int64)
+    qa[g.random((b, c)) < 0.4] = -1
+    qa[0, 0] = -7
+    rev = np.array([False, True, False])
+    exact = of.clause_match(attrs, rev, qa)
+    slots = attrs.transpose(1, 2, 0).reshape(c * vals, n).astype(np.int32)
+    kw = dict(item_clause_attrs=_t(dev, slots),
+              clause_slots=_t(dev, vals * np.arange(c + 1, dtype=np.int64)),
+              clause_is_reverse=_t(dev, rev))
+    want = ost.search(*want_args, valid=exact)
+    for dtype in (np.int64, np.int32):
+        ids, sc = _run(*args, **kw, query_clause_attrs=_t(dev, qa.astype(dtype)))
+        assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
