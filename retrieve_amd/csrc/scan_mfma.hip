@@ -94,9 +94,13 @@ __global__ void __launch_bounds__(kScanThreads) seed_mfma_kernel(ScanArgs a) {
   const int64_t qrow = static_cast<int64_t>(blockIdx.y) * 16 + col;
   v4i qf[KSTEPS];
   load_query_fragments<KSTEPS>(a, qrow, grp, qf);
-  const uint64_t* qmask =
-      a.mask != nullptr && qrow < a.B ? a.mask + qrow * a.mask_words : nullptr;
-  const bool clauses = a.clause.active != nullptr && qrow < a.B;
+  // The filters are switched for the whole wave: a matrix product reads the rows of every lane, so
+  // no lane may leave the tile loop for another instance of it. Padding columns filter as the
+  // last query and write nothing.
+  const int64_t frow = qrow < a.B ? qrow : a.B - 1;
+  const bool real = qrow < a.B;
+  const uint64_t* qmask = a.mask != nullptr ? a.mask + frow * a.mask_words : nullptr;
+  const bool clauses = a.clause.active != nullptr;
   const uint64_t* bm = nullptr;
   if (a.clause.active != nullptr && a.clause_lds) {
     // the group's set bitmaps in LDS (the host sized the launch for them)
@@ -110,7 +114,7 @@ __global__ void __launch_bounds__(kScanThreads) seed_mfma_kernel(ScanArgs a) {
     __syncthreads();
     bm = seed_bm + col * per_row;
   }
-  const ClauseRow crow = clauses ? clause_row(a.clause, qrow, bm) : ClauseRow{};
+  const ClauseRow crow = clauses ? clause_row(a.clause, frow, bm) : ClauseRow{};
   const bool held = clauses && a.clause.held;
 
   const int64_t r0 = static_cast<int64_t>(blockIdx.x) * a.strip;
@@ -169,7 +173,7 @@ __global__ void __launch_bounds__(kScanThreads) seed_mfma_kernel(ScanArgs a) {
       const int64_t row = rb + 4 * grp + r;
       cs[r] = composite(KeyOps<Score>::key(acc[r]),
                         static_cast<uint32_t>(sample_item(row, a.row_stride)));
-      cand |= row < r1 && cs[r] > best ? 1u << r : 0u;
+      cand |= real && row < r1 && cs[r] > best ? 1u << r : 0u;
     }
     if (MASKED && cand != 0u) {
       const int64_t item0 = sample_item(rb + 4 * grp, a.row_stride);
