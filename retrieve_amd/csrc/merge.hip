@@ -28,6 +28,10 @@ static constexpr int64_t kTargetWorkgroups = 2048;
 // At least this many sampled rows per wanted item (keeps the main pass's candidates near
 // k * N / seed_rows for large k).
 static constexpr int64_t kSeedRowsPerK = 1024;
+// The smallest sample worth its two launches and the fallback's.
+static constexpr int64_t kSeedMinRows = 4096;
+// Rows of a main pass's workgroup at least (half without a bound).
+static constexpr int64_t kMainMinRows = 256;
 // Upper bound on the candidate lists' workspace (a pass may exceed it only at one workgroup
 // per query group).
 static constexpr int64_t kMaxListBytes = int64_t{2} << 30;
@@ -74,18 +78,37 @@ int64_t main_workgroups() {
   return t < kMaxResidentWorkgroups ? t : kMaxResidentWorkgroups;
 }
 
+// Sampled rows of a table too small for the full sample: one row in 16, 8 or 4, the sparsest whose
+// one-entry lists are enough for the bound's rank; 0 where none is (the scan then runs unseeded).
+// Without a bound a scan's lists take every row, and each full list is sorted by its wave. fp16
+// D = 128 top-100 calls unseeded (with today's spread) and seeded: 10K rows at B = 1 / 50 / 300
+// 35 / 43 / 77 us against 53 / 45 / 82 (so no sample below kSeedMinRows rows); 20K rows
+// 55 / 62 / 115 against 43 / 45 / 62; 1M rows at B = 16 / 50 / 300 334 / 1216 / 4811 against
+// 77 / 89 / 169; exact fp32 100K rows at B = 1024 2230 against 302.
+static int64_t small_seed_rows(int64_t N, int64_t k, int64_t rows_per_wg, int64_t lpq) {
+  for (const int64_t stride : {16, 8, 4}) {
+    const int64_t rows = N / stride / kSeedBlock * kSeedBlock;
+    if (rows < kSeedMinRows) continue;
+    if (rows / rows_per_wg * lpq * 4 >= 5 * sample_rank(k, N / rows)) return rows;
+  }
+  return 0;
+}
+
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
                    int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t seed_rows_min) {
+                   int64_t seed_rows_min, bool ranked) {
   ScanPlan s;
   s.qpg = qpg;
   s.n_qgroups = cdiv(B, qpg);
   // a query's lists per workgroup: every wave scores all of the row's queries (lists_per_wg ==
   // waves * qpg), or one wave owns each query (lists_per_wg == qpg)
   const int64_t lpq = lists_per_wg / qpg;
-  const int64_t seed_rows =
-      seed_rows_min > kSeedRowsPerK * k ? seed_rows_min : kSeedRowsPerK * k;
+  int64_t seed_rows = seed_rows_min > kSeedRowsPerK * k ? seed_rows_min : kSeedRowsPerK * k;
   s.seeded = N >= 8 * seed_rows;
+  if (!s.seeded && ranked) {
+    seed_rows = small_seed_rows(N, k, seed_rows_per_wg, lpq);
+    s.seeded = seed_rows > 0;
+  }
   if (s.seeded) {
     // one-entry lists (each seed wave's best); at least 2k of them per query (their k-th is the
     // safe bound, their rank-th the speculative one; 4k cost configuration 5's step 1.5 % in
@@ -93,7 +116,12 @@ ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_p
     s.seed = plan_pass(seed_rows, N / seed_rows, s.n_qgroups, seed_rows_per_wg, 1, lists_per_wg,
                        lpq, kTargetWorkgroups, cdiv(2 * k, lpq));
   }
-  s.main = plan_pass(N, 1, s.n_qgroups, 1024, main_capw, lists_per_wg, lpq, target_wgs);
+  // A small table is spread over as many workgroups as its rows allow: behind a bound its lists
+  // stay short, and without one they hold every row they meet, so few rows a list end in the
+  // merge instead of in repeated sorts of full lists by one wave (3K rows of fp16 D = 128,
+  // top-100, at 1024 and at 128 rows a workgroup: B = 16 195, 31 us; B = 300 1989, 51 us).
+  s.main = plan_pass(N, 1, s.n_qgroups, s.seeded ? kMainMinRows : kMainMinRows / 2, main_capw,
+                     lists_per_wg, lpq, target_wgs);
   const size_t lists = s.main.lists_bytes > s.seed.lists_bytes ? s.main.lists_bytes
                                                               : s.seed.lists_bytes;
   const size_t counts = s.main.counts_bytes > s.seed.counts_bytes ? s.main.counts_bytes

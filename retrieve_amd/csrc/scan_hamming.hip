@@ -274,7 +274,7 @@ extern "C" size_t rt_hamming_scan_topk_workspace(int64_t B, int64_t N, int64_t W
   }
   const int qpw = ham_qpw(B > 0 ? B : 1);
   return plan_scan(B, N, k, qpw, kScanWaves * qpw, kMaxResidentWorkgroups, ham_capw(k),
-                   kScanWaves * kHamTile)
+                   kScanWaves * kHamTile, kSeedRows, false)
       .total;
 }
 
@@ -311,7 +311,7 @@ extern "C" int rt_hamming_scan_topk(const uint64_t* query_bits, int64_t B,
   }
   const int qpw = ham_qpw(B);
   const ScanPlan plan = plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), ham_capw(k),
-                                  kScanWaves * kHamTile);
+                                  kScanWaves * kHamTile, kSeedRows, false);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;
