@@ -81,10 +81,10 @@ int64_t main_workgroups() {
 // Sampled rows of a table too small for the full sample: one row in 16, 8 or 4, the sparsest whose
 // one-entry lists are enough for the bound's rank; 0 where none is (the scan then runs unseeded).
 // Without a bound a scan's lists take every row, and each full list is sorted by its wave. fp16
-// D = 128 top-100 calls unseeded (with today's spread) and seeded: 10K rows at B = 1 / 50 / 300
-// 35 / 43 / 77 us against 53 / 45 / 82 (so no sample below kSeedMinRows rows); 20K rows
-// 55 / 62 / 115 against 43 / 45 / 62; 1M rows at B = 16 / 50 / 300 334 / 1216 / 4811 against
-// 77 / 89 / 169; exact fp32 100K rows at B = 1024 2230 against 302.
+// D = 128 top-100 calls at B = 1 / 50 / 300: 15K rows unseeded 44 / 51 / 97 us, 20K rows seeded
+// 43 / 45 / 62 us (6K rows at B = 50: 35 us unseeded, 51 seeded, so no sample below
+// kSeedMinRows rows); 1M rows unseeded 152 / 1216 / 4811 us, seeded 73 / 89 / 169; exact fp32
+// 100K rows at B = 1024 2230 us unseeded, 302 seeded.
 static int64_t small_seed_rows(int64_t N, int64_t k, int64_t rows_per_wg, int64_t lpq) {
   for (const int64_t stride : {16, 8, 4}) {
     const int64_t rows = N / stride / kSeedBlock * kSeedBlock;

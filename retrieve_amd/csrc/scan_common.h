@@ -2,7 +2,7 @@
 // workspace layout and the merge kernel's interface.
 //
 // One top-k call is up to four launches on the caller's stream, with no host sync:
-//   1. seed scan over a strided sample of the items (only when N is large),
+//   1. seed scan over a strided sample of the items (not for the smallest tables),
 //   2. seed merge: the exact k-th best composite of the sample per query (a lower bound on the
 //      k-th best over all items),
 //   3. main scan over all items, appending only composites >= that bound,
