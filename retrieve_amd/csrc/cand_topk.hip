@@ -5,10 +5,10 @@
 // The LiNR V2 / V3 operators fused_masked_knn_topk and oporp_1bit_match_topk_indirect
 // (retrieve/src/retrieve/ops/reference/fused_masked_knn_topk.py:9-29,
 // ops/reference/oporp_1bit_match_topk.py:29-41) and SilverTorch's int8 re-rank of given ids
-// (modules/silvertorch.py:363-379). Each query has its own rows, so the work is a gather:
-// a group of L lanes loads one row, 16 bytes per lane per step, dots it with the query chunks
-// it holds in registers and reduces across the group with xor-shuffles; a wave scores 64 / L
-// rows per step. A workgroup scans one query's positions round-robin with the other
+// (modules/silvertorch.py:363-379). Each query has its own rows, so the work is a gather: a wave
+// takes 64 candidates at a time, one id a lane, and groups of L lanes load their rows, V rows in
+// flight a group, dot them with the query chunks they hold in registers and fold the partial
+// dots across the lanes. A workgroup scans one query's positions round-robin with the other
 // workgroups of that query; every wave keeps a candidate list under a running threshold (no
 // seed: the list fills, is compacted to the best k and the threshold rises), and the shared
 // merge picks the final k. The item id rides in the composites, so ties go to the lower item
@@ -22,7 +22,7 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr int kCandThreads = 256;
 constexpr int kCandWaves = kCandThreads / kWave;
-constexpr int kCandMaxWgsPerQuery = 64;
+constexpr int kCandMaxWgsPerQuery = 256;
 constexpr int kCandMaxChunks = 8;  // 16-byte chunks per lane: rows up to 64 * 16 * 8 bytes
 
 enum CandKind : int {
@@ -140,19 +140,25 @@ struct CandArgs {
   int* list_counts;  // [B, S]
 };
 
-template <int KIND, int L, int NC>
+// Bound: the gather of P rows a query, at best the row bytes from HBM; what limits it is how
+// many rows are in flight. One row a group and step, its id load waited for first, 16 queries
+// over 80K of 800K fp16 rows of 128 each took 263 us; 64 ids a load and V rows in flight take 65.
+template <int KIND, int L, int NC, int V>
 __global__ void __launch_bounds__(kCandThreads) cand_scan_kernel(CandArgs a) {
   using Op = CandOp<KIND>;
+  using Acc = typename Op::Acc;
   constexpr bool kFloat = KIND == kCandF16 || KIND == kCandBF16 || KIND == kCandF32;
-  constexpr int R = kWave / L;  // rows per wave step
+  constexpr int R = kWave / L;  // groups a wave
+  constexpr int E = R * V;      // rows scored at a time
+  static_assert(V <= L && kWave % E == 0, "a lane owns at most one of the rows scored together");
   // elements of a 16-byte item chunk, and the query floats they meet
   constexpr int QF = KIND == kCandF32 ? 4 : 8;
   extern __shared__ uint64_t smem[];
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int wave = tid >> 6;
-  const int grp = lane / L;  // row within the step
-  const int gl = lane % L;   // lane within the row's group
+  const int grp = lane / L;  // row group of the wave
+  const int gl = lane % L;   // lane within it
   uint64_t* scratch = smem + wave * a.capw;
   int* cnt_lds = reinterpret_cast<int*>(smem + kCandWaves * a.capw);
   const int64_t b = blockIdx.y;
@@ -187,57 +193,91 @@ __global__ void __launch_bounds__(kCandThreads) cand_scan_kernel(CandArgs a) {
     qs = a.qscale[b];
     gs = a.gscale[0];
   }
+  // the row of the batch that this lane owns: the folds leave lane gl (its low bits reversed)
+  // with row v of its group
+  int own = 0;
+#pragma unroll
+  for (int i = 1, v = V / 2; v > 0; i <<= 1, v >>= 1) own |= (gl & i) ? v : 0;
   uint64_t tau = 0;  // composites below it cannot reach this wave's best k
   int cnt = 0;
-  const int64_t step = gx * kCandWaves * R;
-  const int64_t first = slot * R;
+  const int64_t step = S * kWave;
   const int8_t* I = static_cast<const int8_t*>(a.items);
-  for (int64_t base = first; base < count; base += step) {
-    const int64_t p = base + grp;
-    bool ok = p < count;
-    int64_t item = ok ? a.ids[b * a.P + p] : 0;
-    ok = ok && item >= 0 && item < a.N;  // ids outside the table are skipped, not read
-    int64_t r = item;
+  const int64_t* ids = a.ids + b * a.P;
+  int64_t next = slot * kWave + lane < count ? ids[slot * kWave + lane] : -1;
+  for (int64_t base = slot * kWave; base < count; base += step) {
+    int64_t item = next;
+    next = base + step + lane < count ? ids[base + step + lane] : -1;
+    bool ok = item >= 0 && item < a.N;  // ids outside the table are skipped, not read
+    int64_t r = ok ? item : 0;
     if (a.rows != nullptr && ok) {
       r = a.rows[item];
       ok = r >= 0 && r < a.N;
     }
-    typename Op::Acc s = 0;
-    if (ok) {
-      const int8_t* row = I + r * a.RB;
+    const uint64_t have = __ballot(ok);
+    // (the row's byte offset, the same 64 bits the group's lanes add their chunk to)
+    const int64_t at = ok ? r * a.RB : 0;
+#pragma unroll 1
+    for (int e0 = 0; e0 < kWave; e0 += E) {
+      if (E < kWave && ((have >> e0) & ((1ull << (E % kWave)) - 1ull)) == 0ull) continue;
+      v4i x[V][NC];
 #pragma unroll
-      for (int j = 0; j < NC; ++j) {
-        const int c = gl + j * L;
-        if (c < nchunks) {
-          const v4i x = load_chunk<true>(row, c, a.RB);
+      for (int v = 0; v < V; ++v) {
+        const int e = e0 + v * R + grp;
+        const int8_t* row = I + __shfl(at, e);
+        const bool live = (have >> e) & 1ull;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+          const int c = gl + j * L;
+          x[v][j] = live && c < nchunks ? load_chunk<false>(row, c, a.RB) : v4i{0, 0, 0, 0};
+        }
+      }
+      Acc s[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        s[v] = 0;
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
           if constexpr (kFloat) {
-            s += Op::chunk(x, qf[j]);
+            s[v] += Op::chunk(x[v][j], qf[j]);
           } else {
-            s += Op::chunk(x, qb[j]);
+            s[v] += Op::chunk(x[v][j], qb[j]);
           }
         }
       }
-    }
+      // each exchange hands half of the rows' sums to the other lane of a pair
 #pragma unroll
-    for (int off = L / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if constexpr (KIND == kCandBits) s += 8 * a.RB;
-    uint64_t c = 0;
-    if constexpr (kFloat) {
-      c = composite(key_of_f32(static_cast<float>(s)), static_cast<uint32_t>(item));
-    } else if constexpr (KIND == kCandI8Scaled) {
-      // two roundings in this order, as (dots * q_scales) * global_scale in fp32
-      const float v = (static_cast<float>(s) * qs) * gs;
-      c = composite(key_of_f32(v), static_cast<uint32_t>(item));
-    } else {  // int8 dots and bit-code scores are exact int32
-      c = composite(key_of_i32(static_cast<int32_t>(s)), static_cast<uint32_t>(item));
-    }
-    const bool keep = ok && gl == 0 && c >= tau;
-    const uint64_t bal = __ballot(keep);
-    if (bal != 0ull) {
-      const int before = __popcll(bal & ((1ull << lane) - 1ull));
-      if (keep) list[cnt + before] = c;
+      for (int off = 1, half = V / 2; half > 0; off <<= 1, half >>= 1) {
+        const bool up = (gl & off) != 0;
+#pragma unroll
+        for (int v = 0; v < half; ++v) {
+          const Acc send = up ? s[v] : s[v + half];
+          const Acc keep = up ? s[v + half] : s[v];
+          s[v] = keep + __shfl_xor(send, off);
+        }
+      }
+#pragma unroll
+      for (int off = V; off < L; off <<= 1) s[0] += __shfl_xor(s[0], off);
+      const int e = e0 + own * R + grp;
+      const uint32_t id = static_cast<uint32_t>(__shfl(static_cast<int>(item), e));
+      const bool mine = gl < V && ((have >> e) & 1ull);
+      Acc t = s[0];
+      if constexpr (KIND == kCandBits) t += 8 * a.RB;
+      uint64_t c = 0;
+      if constexpr (kFloat) {
+        c = composite(key_of_f32(static_cast<float>(t)), id);
+      } else if constexpr (KIND == kCandI8Scaled) {
+        // two roundings in this order, as (dots * q_scales) * global_scale in fp32
+        const float v = (static_cast<float>(t) * qs) * gs;
+        c = composite(key_of_f32(v), id);
+      } else {  // int8 dots and bit-code scores are exact int32
+        c = composite(key_of_i32(static_cast<int32_t>(t)), id);
+      }
+      const bool keep = mine && c >= tau;
+      const uint64_t bal = __ballot(keep);
+      if (bal == 0ull) continue;
+      if (keep) list[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = c;
       cnt += __popcll(bal);
-      if (cnt > a.capw - R) {
+      if (cnt > a.capw - E) {
         if (lane == 0) cnt_lds[wave] = cnt;
         const uint64_t nt = wave_compact(list, &cnt_lds[wave], scratch, a.capw, a.k);
         cnt = cnt_lds[wave];
@@ -248,52 +288,46 @@ __global__ void __launch_bounds__(kCandThreads) cand_scan_kernel(CandArgs a) {
   if (lane == 0) a.list_counts[b * S + slot] = cnt;
 }
 
-// A winner with a non-finite float score becomes id -1 (functional.py:81-82).
-__global__ void cand_ids_kernel(int64_t* ids, const float* scores, int64_t n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n && !__builtin_isfinite(scores[i])) ids[i] = -1;
-}
-
-template <int KIND, int L, int NC>
-static void launch_cand(const CandArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
+template <int KIND, int L, int NC, int V>
+static int launch_cand(const CandArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
   if (lds > 64 * 1024) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&cand_scan_kernel<KIND, L, NC>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    RT_CHECK_HIP(hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&cand_scan_kernel<KIND, L, NC, V>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   }
-  cand_scan_kernel<KIND, L, NC><<<grid, kCandThreads, lds, stream>>>(a);
+  cand_scan_kernel<KIND, L, NC, V><<<grid, kCandThreads, lds, stream>>>(a);
+  RT_CHECK_HIP(hipGetLastError());
+  return kOk;
 }
 
+// L lanes of NC 16-byte chunks a row, V rows in flight a group (at most 64 registers of them):
+// narrow groups fold few partial dots and still read whole 128-byte lines.
 template <int KIND>
 static int dispatch_cand(const CandArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
-  // L lanes per row (16 bytes each, up to 64), NC 16-byte chunks per lane
-  switch ((a.RB + 15) / 16 * 16) {
-    case 16: launch_cand<KIND, 1, 1>(a, grid, lds, stream); break;
-    case 32: launch_cand<KIND, 2, 1>(a, grid, lds, stream); break;
-    case 64: launch_cand<KIND, 4, 1>(a, grid, lds, stream); break;
-    case 128: launch_cand<KIND, 8, 1>(a, grid, lds, stream); break;
-    case 256: launch_cand<KIND, 16, 1>(a, grid, lds, stream); break;
-    case 512: launch_cand<KIND, 32, 1>(a, grid, lds, stream); break;
-    default:
-      if (a.RB <= 1024) {
-        launch_cand<KIND, 64, 1>(a, grid, lds, stream);
-      } else if (a.RB <= 2048) {
-        launch_cand<KIND, 64, 2>(a, grid, lds, stream);
-      } else if (a.RB <= 4096) {
-        launch_cand<KIND, 64, 4>(a, grid, lds, stream);
-      } else {
-        launch_cand<KIND, 64, 8>(a, grid, lds, stream);
-      }
-  }
-  return kOk;
+  if (a.RB <= 16) return launch_cand<KIND, 1, 1, 1>(a, grid, lds, stream);
+  if (a.RB <= 32) return launch_cand<KIND, 2, 1, 2>(a, grid, lds, stream);
+  if (a.RB <= 64) return launch_cand<KIND, 4, 1, 4>(a, grid, lds, stream);
+  if (a.RB <= 128) return launch_cand<KIND, 8, 1, 8>(a, grid, lds, stream);
+  if (a.RB <= 192) return launch_cand<KIND, 4, 3, 4>(a, grid, lds, stream);
+  if (a.RB <= 256) return launch_cand<KIND, 8, 2, 8>(a, grid, lds, stream);
+  if (a.RB <= 512) return launch_cand<KIND, 16, 2, 8>(a, grid, lds, stream);
+  if (a.RB <= 1024) return launch_cand<KIND, 32, 2, 8>(a, grid, lds, stream);
+  if (a.RB <= 2048) return launch_cand<KIND, 64, 2, 8>(a, grid, lds, stream);
+  if (a.RB <= 4096) return launch_cand<KIND, 64, 4, 4>(a, grid, lds, stream);
+  return launch_cand<KIND, 64, 8, 2>(a, grid, lds, stream);
 }
 
 static int cand_capw(int64_t k) { return static_cast<int>(next_pow2(k + kWave)); }
 
-// Workgroups per query: ~2048 in all, at most one per 128 candidates (a wave's rows are an id
-// load then the row's loads, one step after another: the grid, not the loop, hides that latency).
+// A query's lists hold up to k entries each (a wave starts without a bound), so its merge is split
+// from few lists, up to a batch whose merges fill the CUs.
+constexpr int kCandPartSlots = 16;
+constexpr int64_t kCandSplitMaxB = 128;
+
+// Workgroups per query: ~2048 in all, at most one per 256 candidates (64 a wave).
 static int64_t cand_gx(int64_t B, int64_t P) {
   int64_t gx = cdiv(2048, B > 0 ? B : 1);
-  const int64_t by_rows = cdiv(P, 128);
+  const int64_t by_rows = cdiv(P, kCandThreads);
   gx = gx < by_rows ? gx : by_rows;
   gx = gx < 1 ? 1 : gx;
   return gx < kCandMaxWgsPerQuery ? gx : kCandMaxWgsPerQuery;
@@ -307,7 +341,8 @@ extern "C" size_t rt_cand_topk_workspace(int64_t B, int64_t P, int64_t k) {
   if (B <= 0 || P <= 0 || k <= 0) return 256;
   const int64_t S = cand_gx(B, P) * kCandWaves;
   return align_up(static_cast<size_t>(B * S) * cand_capw(k) * sizeof(uint64_t), 256) +
-         align_up(static_cast<size_t>(B * S) * sizeof(int), 256);
+         align_up(static_cast<size_t>(B * S) * sizeof(int), 256) +
+         (B <= kCandSplitMaxB ? static_cast<size_t>(B) * kMergeParts * k * sizeof(uint64_t) : 0);
 }
 
 namespace rt {
@@ -334,8 +369,9 @@ static int cand_topk(const void* queries, int64_t B, const void* items, int64_t 
                "queries and items must be %lld-byte aligned", static_cast<long long>(unit));
   RT_CHECK_ARG(N < 0xffffffffll, "N must be < 2**32 - 1");
   // bit codes score as exact int32 keys, written as float
+  // (a winner with a non-finite float score becomes id -1, functional.py:81-82)
   const int score_kind =
-      kind == kCandI8 ? kScoreI32 : (kind == kCandBits ? kScoreF32FromI32 : kScoreF32);
+      kind == kCandI8 ? kScoreI32 : (kind == kCandBits ? kScoreF32FromI32 : kScoreF32Finite);
   RT_CHECK_ARG(kind != kCandI8Scaled || (qscale != nullptr && gscale != nullptr),
                "the scaled int8 kind needs query and global scales");
   if (B == 0) return kOk;
@@ -370,15 +406,16 @@ static int cand_topk(const void* queries, int64_t B, const void* items, int64_t 
   const size_t lds = static_cast<size_t>(kCandWaves) * capw * sizeof(uint64_t) +
                      kCandWaves * sizeof(int);
   const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(B));
+  int st = kOk;
   switch (kind) {
-    case kCandF16: dispatch_cand<kCandF16>(a, grid, lds, stream); break;
-    case kCandBF16: dispatch_cand<kCandBF16>(a, grid, lds, stream); break;
-    case kCandF32: dispatch_cand<kCandF32>(a, grid, lds, stream); break;
-    case kCandI8: dispatch_cand<kCandI8>(a, grid, lds, stream); break;
-    case kCandI8Scaled: dispatch_cand<kCandI8Scaled>(a, grid, lds, stream); break;
-    default: dispatch_cand<kCandBits>(a, grid, lds, stream); break;
+    case kCandF16: st = dispatch_cand<kCandF16>(a, grid, lds, stream); break;
+    case kCandBF16: st = dispatch_cand<kCandBF16>(a, grid, lds, stream); break;
+    case kCandF32: st = dispatch_cand<kCandF32>(a, grid, lds, stream); break;
+    case kCandI8: st = dispatch_cand<kCandI8>(a, grid, lds, stream); break;
+    case kCandI8Scaled: st = dispatch_cand<kCandI8Scaled>(a, grid, lds, stream); break;
+    default: st = dispatch_cand<kCandBits>(a, grid, lds, stream); break;
   }
-  RT_CHECK_HIP(hipGetLastError());
+  if (st != kOk) return st;
   MergeArgs m{};
   m.lists = a.lists;
   m.counts = a.list_counts;
@@ -391,14 +428,13 @@ static int cand_topk(const void* queries, int64_t B, const void* items, int64_t 
   m.out_ids = out_ids;
   m.out_scores = out_scores;
   m.score_kind = score_kind;
-  int st = launch_merge(m, stream);
-  if (st != kOk) return st;
-  if (score_kind == kScoreF32) {
-    cand_ids_kernel<<<static_cast<unsigned>(cdiv(B * k, 256)), 256, 0, stream>>>(
-        out_ids, static_cast<const float*>(out_scores), B * k);
-    RT_CHECK_HIP(hipGetLastError());
+  if (B <= kCandSplitMaxB) {
+    m.part_buf = reinterpret_cast<uint64_t*>(
+        reinterpret_cast<char*>(a.list_counts) +
+        align_up(static_cast<size_t>(B * S) * sizeof(int), 256));
+    m.part_slots = kCandPartSlots;
   }
-  return kOk;
+  return launch_merge(m, stream);
 }
 
 }  // namespace rt

@@ -473,8 +473,10 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(MergeArgs m) {
   for (int j = tid; j < k; j += kMergeThreads) {
     const uint64_t c = buf[j];
     const bool ok = c != 0ull;
-    m.out_ids[q * k + j] = ok ? static_cast<int64_t>(composite_item(c)) : -1;
     const uint32_t key = composite_key(c);
+    const bool named =
+        ok && (m.score_kind != kScoreF32Finite || __builtin_isfinite(f32_of_key(key)));
+    m.out_ids[q * k + j] = named ? static_cast<int64_t>(composite_item(c)) : -1;
     if (m.score_kind == kScoreI32) {
       static_cast<int32_t*>(m.out_scores)[q * k + j] = ok ? i32_of_key(key) : INT32_MIN;
     } else if (m.score_kind == kScoreF32FromI32) {

@@ -59,6 +59,7 @@ enum ScoreKind : int {
   kScoreI32 = 0,       // the key is an int32 score; write int32
   kScoreF32FromI32 = 1,  // the key is an int32 score; write it as float
   kScoreF32 = 2,       // the key is a float score; write float
+  kScoreF32Finite = 3,  // as kScoreF32, the id -1 where the score is not finite
 };
 
 struct MergeArgs {
