@@ -170,7 +170,7 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
               void* out_scores, int score_kind, void* workspace, size_t workspace_bytes,
               hipStream_t stream);
 // The 1-bit full scan for kMaxK < k <= kMaxKHamming (scan_hamming_large.hip).
-size_t hamming_large_k_workspace(int64_t B, int64_t N, int64_t W);
+size_t hamming_large_k_workspace(int64_t B, int64_t N, int64_t W, int64_t k);
 int hamming_large_k(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, int64_t N,
                     int64_t W, int64_t k, const uint64_t* mask, int64_t mask_words,
                     int64_t* out_ids, void* out_scores, int score_kind, void* workspace,

@@ -267,7 +267,7 @@ using namespace rt;
 
 extern "C" size_t rt_hamming_scan_topk_workspace(int64_t B, int64_t N, int64_t W, int64_t k,
                                                  int masked) {
-  if (k > kMaxK) return hamming_large_k_workspace(B > 0 ? B : 1, N, W);
+  if (k > kMaxK) return hamming_large_k_workspace(B > 0 ? B : 1, N, W, k);
   if (ham_bits_mfma(B, W, k)) return bits_mfma_workspace(B, N, k);
   if (ham_mfma(B, W, k, masked != 0)) {
     return blocked_hamming_workspace(B, N, W, k, masked != 0);

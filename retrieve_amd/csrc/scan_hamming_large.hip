@@ -4,18 +4,25 @@
 // 261-273, then torch.topk). Same result as the scan: top-k by (score desc, id asc) of
 // score = 64 W - 2 popcount(q ^ item) over the items that pass the mask.
 //
-// A Hamming score takes only 64 W + 1 values, so the k-th score is found by counting:
-//   1. histogram pass: per query, the number of passing items at each popcount h;
-//   2. cut: the popcount h* of the k-th best, lt = #(h < h*), need = k - lt;
-//   3. emit pass: items with h < h* appended (at most k - 1 of them); the items with h == h*
-//      counted per bin of 8192 ids;
-//   4. cut: the id bin b* where the ties reach `need`, need2 = what bin b* must give;
-//   5. emit pass: the ties in bins below b* appended (fewer than need), those of bin b* apart
-//      (at most 8192);
-//   6. per query: bin b*'s ties sorted (their composites order by id), the first need2 kept,
-//      everything sorted by composite and written.
-// Each pass is the popcount scan of the small-batch path (lane <-> item, query codes in SGPRs);
-// the appends go through global atomics and are rare (at most k + 8192 per query).
+// A Hamming score takes only 64 W + 1 values, so the selection is a counting sort by (popcount h,
+// range of ids):
+//   1. count pass: each workgroup scores one contiguous range of items for its queries and
+//      writes how many passing items it met at each popcount (its own row of counts: no
+//      clearing, no global atomics);
+//   2. prefix: per query and popcount the running sums of those counts over the ranges, in
+//      place, and the totals;
+//   3. cut: per query the popcount h* of the k-th best, where each popcount's entries start in
+//      the result, and how many there are (kk = min(k, passing items));
+//   4. emit pass: the same ranges scored again; an item with h <= h* goes to its popcount's
+//      start plus its range's running sum plus an LDS counter. Ties at h* are emitted by the
+//      ranges up to the one where they reach kk, whose ties may run past it;
+//   5. rank: entries of one popcount and range lie together in no order; each finds its place
+//      among them by id and is written there if that is below kk.
+// Two passes over the codes, whose bound is the popcounts (2 W XOR and 2 W bit counts an item
+// and query) and the mask bits. Counting into one histogram a query and appending through one
+// counter a query (same-address atomics, a third pass for the ties and two block sorts) took
+// 516 us for 3M 128-bit codes, 16 queries at k = 5000 under a 10 % mask; these five launches take
+// 108 (count 40, prefix 12, cut 4, emit 46, rank 6).
 #include "scan_common.h"
 
 namespace rt {
@@ -23,31 +30,36 @@ namespace {
 
 constexpr int kLkThreads = 256;
 constexpr int kLkWaves = kLkThreads / kWave;
-constexpr int kLkQpw = 8;        // queries a workgroup scores per pass
-constexpr int kLkIdShift = 13;   // bins of 8192 ids for the ties at the cut
-constexpr int kLkCap = 8192;     // entries per query of each buffer (>= k and >= a bin)
-constexpr int kLkFinalThreads = 1024;
-constexpr int kLkMaxGx = 512;    // workgroups per query group (each flushes one histogram)
+constexpr int kLkQpw = 8;           // queries a workgroup scores
+constexpr int kLkTiles = 2;         // 64-item tiles a wave scores together
+constexpr int64_t kLkMaxRows = 8192;  // items of a range at most (its ties may overrun k)
+constexpr int64_t kLkMinRows = 1024;  // and at least, where the table allows
+constexpr int64_t kLkTargetWgs = 2048;
+constexpr int kLkPrefixThreads = 1024;
+constexpr int kLkPrefixSegs = kLkPrefixThreads / kWave;
+// Counts and entries of the queries taken at a time (the others follow on the same workspace).
+constexpr size_t kLkMaxBytes = size_t{256} << 20;
 
 typedef __attribute__((address_space(4))) const uint32_t ku32;
+typedef __attribute__((address_space(4))) const uint64_t ku64;
 
 struct LkArgs {
   const uint64_t* q;
-  int64_t B;
+  int64_t B;         // queries of this batch
   const uint64_t* items;
   int64_t N;
+  int64_t rows;      // items of a range, a multiple of 64
+  int gx;            // ranges
   int k;
   const uint64_t* mask;
   int64_t mask_words;
-  int nb;            // 64 W + 1 popcount bins
-  int64_t nbin;      // id bins
-  uint32_t* hist;    // [B][nb] (N < 2^32 items: a count fits)
-  int32_t* cnt;      // [B][4]: appends to A, B, C
-  uint32_t* idhist;  // [B][nbin]
-  int32_t* cut;      // [B][8]: h*, lt, need, b*, need2
-  uint64_t* buf_a;   // [B][kLkCap]: h < h*
-  uint64_t* buf_b;   // [B][kLkCap]: h == h*, id bin < b*
-  uint64_t* buf_c;   // [B][kLkCap]: h == h*, id bin == b*
+  int nb;            // 64 W + 1 popcounts
+  int nbp;           // a row of counts: nb rounded up to 64
+  uint16_t* counts;  // [B][gx][nbp]: items of the range at a popcount, then the sums before it
+  uint32_t* totals;  // [B][nbp]: items at a popcount, then its entries' start
+  int32_t* cut;      // [B][4]: h* (-1: nothing passes), kk, entries emitted
+  int64_t cap;       // entries of a query's buffer: k + rows
+  uint64_t* buf;     // [B][cap]
 };
 
 template <int W>
@@ -73,269 +85,267 @@ __device__ inline void lk_load(const uint32_t* __restrict__ I, int64_t item, uin
   }
 }
 
-// MODE 0: histogram; 1: append h < h*, count the ties per id bin; 2: append the ties of the
-// bins up to b*.
-template <int W, int MODE>
+// One range of items for kLkQpw queries. EMIT: the entries up to the cut, else the counts.
+template <int W, bool EMIT>
 __global__ void __launch_bounds__(kLkThreads) lk_pass_kernel(LkArgs a) {
-  extern __shared__ uint32_t lh[];  // MODE 0: [kLkQpw][nb]
+  extern __shared__ uint32_t lh[];  // [kLkQpw][nb]: counts, or the next entry of each popcount
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t q0 = static_cast<int64_t>(blockIdx.y) * kLkQpw;
   const int nq = static_cast<int>(a.B - q0 < kLkQpw ? a.B - q0 : kLkQpw);
-  if constexpr (MODE == 0) {
-    for (int i = threadIdx.x; i < kLkQpw * a.nb; i += kLkThreads) lh[i] = 0;
-    __syncthreads();
-  }
-  ku32* qc = (ku32*)(a.q) + q0 * 2 * W;
-  const uint32_t* I = reinterpret_cast<const uint32_t*>(a.items);
-  const int64_t ntiles = (a.N + kWave - 1) / kWave;
-  for (int64_t t = static_cast<int64_t>(blockIdx.x) * kLkWaves + wave; t < ntiles;
-       t += static_cast<int64_t>(gridDim.x) * kLkWaves) {
-    const int64_t row = t * kWave + lane;
-    const bool valid = row < a.N;
-    uint32_t iw[2 * W];
-    lk_load<W>(I, valid ? row : a.N - 1, iw);
+  const int64_t wg = blockIdx.x;
+  // EMIT: the highest popcount the range emits (-1: none), and where its ties start
+  __shared__ int hs[kLkQpw];
+  __shared__ int first_tie[kLkQpw];
+  if constexpr (EMIT) {
     for (int qi = 0; qi < nq; ++qi) {
       const int64_t q = q0 + qi;
-      int h = 0;
-#pragma unroll
-      for (int d = 0; d < 2 * W; ++d) h = __builtin_popcount(iw[d] ^ qc[qi * 2 * W + d]) + h;
-      bool ok = valid;
-      if (ok && a.mask != nullptr) {
-        ok = (a.mask[q * a.mask_words + (row >> 6)] >> (63 - (row & 63))) & 1ull;
+      const int h = a.cut[q * 4];
+      const int kk = a.cut[q * 4 + 1];
+      const uint16_t* before = a.counts + (q * a.gx + wg) * a.nbp;
+      // ties start in this range at the sums before it (saturated far above any k)
+      const int tie = h < 0 ? 0 : static_cast<int>(a.totals[q * a.nbp + h] + before[h]);
+      const int top = h >= 0 && tie >= kk ? h - 1 : h;
+      for (int i = threadIdx.x; i <= top; i += kLkThreads) {
+        lh[qi * a.nb + i] = a.totals[q * a.nbp + i] + before[i];
       }
-      if constexpr (MODE == 0) {
-        if (ok) atomicAdd(&lh[qi * a.nb + h], 1u);
-      } else {
-        const int hs = a.cut[q * 8];
-        if (!__any(ok && h <= hs)) continue;
-        const uint64_t c = composite(key_of_i32(64 * W - 2 * h), static_cast<uint32_t>(row));
-        if constexpr (MODE == 1) {
-          if (ok && h < hs) {
-            const int pos = atomicAdd(&a.cnt[q * 4], 1);
-            if (pos < kLkCap) a.buf_a[q * kLkCap + pos] = c;
-          } else if (ok && h == hs) {
-            atomicAdd(&a.idhist[q * a.nbin + (row >> kLkIdShift)], 1u);
-          }
+      if (threadIdx.x == 0) {
+        hs[qi] = top;
+        first_tie[qi] = tie;
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < kLkQpw * a.nb; i += kLkThreads) lh[i] = 0;
+  }
+  __syncthreads();
+  ku32* qc = (ku32*)(a.q) + q0 * 2 * W;
+  const uint32_t* I = reinterpret_cast<const uint32_t*>(a.items);
+  const int64_t r0 = wg * a.rows;
+  const int64_t r1 = r0 + a.rows < a.N ? r0 + a.rows : a.N;
+  // waves take kLkTiles consecutive tiles in turn
+  constexpr int64_t kStep = static_cast<int64_t>(kLkWaves) * kLkTiles * kWave;
+  for (int64_t t0 = r0 + wave * (kLkTiles * kWave); t0 < r1; t0 += kStep) {
+    uint32_t iw[kLkTiles][2 * W];
+#pragma unroll
+    for (int t = 0; t < kLkTiles; ++t) {
+      const int64_t row = t0 + t * kWave + lane;
+      lk_load<W>(I, row < r1 ? row : r1 - 1, iw[t]);
+    }
+    for (int qi = 0; qi < nq; ++qi) {
+      uint64_t m[kLkTiles];
+#pragma unroll
+      for (int t = 0; t < kLkTiles; ++t) {
+        // bit 63 - lane of the tile's word: the row passes (ranges are whole words)
+        const int64_t left = r1 - (t0 + t * kWave);
+        m[t] = left >= kWave ? ~0ull : (left > 0 ? ~(~0ull >> left) : 0ull);
+      }
+      if (a.mask != nullptr) {
+        ku64* mrow = (ku64*)(a.mask) + (q0 + qi) * a.mask_words;
+#pragma unroll
+        for (int t = 0; t < kLkTiles; ++t) {
+          if (m[t] != 0ull) m[t] &= mrow[(t0 >> 6) + t];
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < kLkTiles; ++t) {
+        if (m[t] == 0ull) continue;  // (wave-uniform)
+        int h = 0;
+#pragma unroll
+        for (int d = 0; d < 2 * W; ++d) h = __builtin_popcount(iw[t][d] ^ qc[qi * 2 * W + d]) + h;
+        const bool ok = (m[t] >> (63 - lane)) & 1ull;
+        if constexpr (!EMIT) {
+          if (ok) atomicAdd(&lh[qi * a.nb + h], 1u);
         } else {
-          const int64_t bs = a.cut[q * 8 + 3];
-          const int64_t bin = row >> kLkIdShift;
-          if (ok && h == hs && bin <= bs) {
-            const int which = bin < bs ? 1 : 2;
-            const int pos = atomicAdd(&a.cnt[q * 4 + which], 1);
-            uint64_t* dst = which == 1 ? a.buf_b : a.buf_c;
-            if (pos < kLkCap) dst[q * kLkCap + pos] = c;
+          if (ok && h <= hs[qi]) {
+            const uint32_t row = static_cast<uint32_t>(t0 + t * kWave + lane);
+            const uint32_t pos = atomicAdd(&lh[qi * a.nb + h], 1u);
+            if (pos < a.cap) {
+              a.buf[(q0 + qi) * a.cap + pos] = composite(key_of_i32(64 * W - 2 * h), row);
+            }
           }
         }
       }
     }
   }
-  if constexpr (MODE == 0) {
-    __syncthreads();
-    for (int i = threadIdx.x; i < nq * a.nb; i += kLkThreads) {
-      const uint32_t v = lh[i];
-      if (v != 0u) atomicAdd(&a.hist[(q0 + i / a.nb) * a.nb + i % a.nb], v);
+  __syncthreads();
+  if constexpr (EMIT) {
+    // the range in which the ties reach kk knows how many entries there are
+    if (threadIdx.x < nq) {
+      const int qi = threadIdx.x;
+      int32_t* cut = a.cut + (q0 + qi) * 4;
+      const int h = cut[0];
+      const int kk = cut[1];
+      if (h >= 0 && hs[qi] == h) {
+        const int end = static_cast<int>(lh[qi * a.nb + h]);
+        if (first_tie[qi] < kk && end >= kk) cut[2] = end;
+      }
+    }
+  } else {
+    for (int qi = 0; qi < nq; ++qi) {
+      uint16_t* out = a.counts + ((q0 + qi) * a.gx + wg) * a.nbp;
+      for (int i = threadIdx.x; i < a.nbp; i += kLkThreads) {
+        out[i] = i < a.nb ? static_cast<uint16_t>(lh[qi * a.nb + i]) : uint16_t{0};
+      }
     }
   }
 }
 
-// Inclusive prefix sum over the wave (64-bit: the counts of up to 2^32 items).
-__device__ inline uint64_t lk_wave_scan(uint64_t x) {
+// Per query (grid y) and 64 popcounts (grid x): each range's counts become the sums before it,
+// saturated at 65535 (sums that matter stay below k <= 8192), and the totals are written. A wave
+// takes a segment of the ranges, a lane a popcount.
+__global__ void __launch_bounds__(kLkPrefixThreads) lk_prefix_kernel(LkArgs a) {
+  __shared__ uint32_t seg_sum[kLkPrefixSegs][kWave];
   const int lane = lane_id();
+  const int seg = threadIdx.x >> 6;
+  const int64_t q = blockIdx.y;
+  const int h = blockIdx.x * kWave + lane;  // < nbp
+  uint16_t* c = a.counts + q * a.gx * a.nbp + h;
+  const int per = (a.gx + kLkPrefixSegs - 1) / kLkPrefixSegs;
+  const int g0 = seg * per;
+  const int g1 = g0 + per < a.gx ? g0 + per : a.gx;
+  uint32_t sum = 0;
+#pragma unroll 8
+  for (int g = g0; g < g1; ++g) sum += c[static_cast<int64_t>(g) * a.nbp];
+  seg_sum[seg][lane] = sum;
+  __syncthreads();
+  uint32_t run = 0;
+  for (int s = 0; s < seg; ++s) run += seg_sum[s][lane];
+  constexpr int kAhead = 8;
+  for (int g = g0; g < g1; g += kAhead) {
+    uint32_t v[kAhead];
 #pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint64_t y = __shfl_up(x, off);
-    x += lane >= off ? y : 0ull;
-  }
-  return x;
-}
-
-// The first index of counts[0, n) at which the running sum reaches `want` (>= 1), and the sum
-// before it (< want); n when the counts never reach it. One wave.
-__device__ inline void lk_find(const uint32_t* counts, int64_t n, int want, int64_t* at,
-                               int* before) {
-  const int lane = lane_id();
-  uint64_t run = 0;
-  for (int64_t c0 = 0; c0 < n; c0 += kWave) {
-    const uint64_t v = c0 + lane < n ? counts[c0 + lane] : 0u;
-    const uint64_t incl = lk_wave_scan(v);
-    const uint64_t hit = __ballot(run + incl >= static_cast<uint64_t>(want));
-    if (hit != 0ull) {
-      const int f = __builtin_ctzll(hit);
-      *at = c0 + f;
-      *before = static_cast<int>(run + __shfl(incl - v, f));
-      return;
+    for (int i = 0; i < kAhead; ++i) {
+      v[i] = g + i < g1 ? c[static_cast<int64_t>(g + i) * a.nbp] : 0u;
     }
-    run += __shfl(incl, kWave - 1);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (g + i < g1) {
+        c[static_cast<int64_t>(g + i) * a.nbp] =
+            static_cast<uint16_t>(run < 0xffffu ? run : 0xffffu);
+      }
+      run += v[i];
+    }
   }
-  *at = n;
-  *before = static_cast<int>(run < static_cast<uint64_t>(want) ? run : want);
+  if (seg == kLkPrefixSegs - 1) a.totals[q * a.nbp + h] = run;
 }
 
-// Step 2: h*, lt, need per query (one wave each).
+// Per query (one wave): the totals become each popcount's start (saturated: only starts up to
+// h* matter), h* and kk.
 __global__ void __launch_bounds__(kWave) lk_cut_kernel(LkArgs a) {
   const int64_t q = blockIdx.x;
-  const uint32_t* h = a.hist + q * a.nb;
-  uint64_t total = 0;
-  for (int i = lane_id(); i < a.nb; i += kWave) total += h[i];
+  const int lane = lane_id();
+  uint32_t* t = a.totals + q * a.nbp;
+  uint64_t run = 0;
+  int hs = -1;
+  for (int c0 = 0; c0 < a.nbp; c0 += kWave) {
+    const uint64_t v = t[c0 + lane];
+    uint64_t incl = v;
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
-  const int kk = total < static_cast<uint64_t>(a.k) ? static_cast<int>(total) : a.k;
-  int64_t hs = -1;  // no passing item: nothing is emitted
-  int lt = 0;
-  if (kk > 0) lk_find(h, a.nb, kk, &hs, &lt);
-  if (lane_id() == 0) {
-    a.cut[q * 8] = static_cast<int32_t>(hs);
-    a.cut[q * 8 + 1] = lt;
-    a.cut[q * 8 + 2] = kk - lt;
-    a.cut[q * 8 + 3] = -1;
-    a.cut[q * 8 + 4] = 0;
-  }
-}
-
-// Step 4: b*, need2 per query (one wave each).
-__global__ void __launch_bounds__(kWave) lk_cut2_kernel(LkArgs a) {
-  const int64_t q = blockIdx.x;
-  const int need = a.cut[q * 8 + 2];
-  if (need <= 0) return;
-  int64_t bs = 0;
-  int before = 0;
-  lk_find(a.idhist + q * a.nbin, a.nbin, need, &bs, &before);
-  if (lane_id() == 0) {
-    a.cut[q * 8 + 3] = static_cast<int32_t>(bs);
-    a.cut[q * 8 + 4] = need - before;
-  }
-}
-
-// Descending bitonic sort of s[0, n) (n a power of two) by the whole workgroup.
-__device__ inline void lk_block_sort(uint64_t* s, int n) {
-  for (int size = 2; size <= n; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int t = threadIdx.x; t < (n >> 1); t += kLkFinalThreads) {
-        const int i = 2 * t - (t & (stride - 1));
-        const int j = i + stride;
-        const bool desc = (i & size) == 0;
-        const uint64_t x = s[i];
-        const uint64_t y = s[j];
-        if ((x < y) == desc) {
-          s[i] = y;
-          s[j] = x;
-        }
-      }
-      __syncthreads();
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint64_t y = __shfl_up(incl, off);
+      incl += lane >= off ? y : 0ull;
     }
+    const uint64_t before = run + incl - v;
+    t[c0 + lane] = static_cast<uint32_t>(before < 0x7fffffffull ? before : 0x7fffffffull);
+    // the popcount of the k-th best, or the last one that holds an item
+    const uint64_t here = __ballot(v != 0ull && before < static_cast<uint64_t>(a.k));
+    if (here != 0ull) hs = c0 + 63 - __builtin_clzll(here);
+    run += __shfl(incl, kWave - 1);
+  }
+  if (lane == 0) {
+    const int kk = run < static_cast<uint64_t>(a.k) ? static_cast<int>(run) : a.k;
+    a.cut[q * 4] = hs;
+    a.cut[q * 4 + 1] = kk;
+    a.cut[q * 4 + 2] = 0;  // (the emit pass writes it where kk > 0)
   }
 }
 
-__device__ inline int lk_pow2(int n) {
-  int p = 1;
-  while (p < n) p <<= 1;
+// An entry's place: its cell (entries of one popcount and range) starts where the entries to its
+// left stop being of the cell, and it follows those of the cell that have lower ids.
+__global__ void __launch_bounds__(kLkThreads) lk_rank_kernel(LkArgs a, int64_t* out_ids,
+                                                             void* out_scores, int score_kind) {
+  const int64_t q = blockIdx.y;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kLkThreads + threadIdx.x;
+  const int kk = a.cut[q * 4 + 1];
+  const int n = a.cut[q * 4 + 2];
+  auto put = [&](int64_t at, int64_t id, int32_t score, bool pad) {
+    out_ids[q * a.k + at] = id;
+    if (score_kind == kScoreI32) {
+      static_cast<int32_t*>(out_scores)[q * a.k + at] = pad ? INT32_MIN : score;
+    } else {
+      static_cast<float*>(out_scores)[q * a.k + at] =
+          pad ? -INFINITY : static_cast<float>(score);
+    }
+  };
+  if (i >= kk && i < a.k) put(i, -1, 0, true);
+  if (i >= n) return;
+  const uint64_t* e = a.buf + q * a.cap;
+  const uint64_t c = e[i];
+  const uint32_t rows = static_cast<uint32_t>(a.rows);
+  const uint32_t cell = composite_item(c) / rows;
+  auto same = [&](uint64_t x) {
+    return composite_key(x) == composite_key(c) && composite_item(x) / rows == cell;
+  };
+  int64_t at = i;
+  for (int64_t j = i - 1; j >= 0; --j) {
+    const uint64_t x = e[j];
+    if (!same(x)) break;
+    at -= x < c ? 1 : 0;  // (smaller composite: higher id)
+  }
+  for (int64_t j = i + 1; j < n; ++j) {
+    const uint64_t x = e[j];
+    if (!same(x)) break;
+    at += x > c ? 1 : 0;
+  }
+  if (at < kk) put(at, composite_item(c), i32_of_key(composite_key(c)), false);
+}
+
+struct LkPlan {
+  int64_t rows, gx, nbp, cap, batch;
+  size_t totals, cut, counts, buf, total;
+};
+
+LkPlan lk_plan(int64_t B, int64_t N, int64_t W, int64_t k) {
+  LkPlan p{};
+  const int64_t gy = cdiv(B, kLkQpw);
+  // ranges of at most kLkMaxRows items, and enough of them to fill the GPU where they stay
+  // above kLkMinRows
+  int64_t gx = cdiv(kLkTargetWgs, gy);
+  const int64_t most = cdiv(N, kLkMinRows);
+  gx = gx < most ? gx : most;
+  const int64_t least = cdiv(N, kLkMaxRows);
+  gx = gx > least ? gx : least;
+  p.rows = cdiv(cdiv(N, gx), kWave) * kWave;
+  p.gx = cdiv(N, p.rows);
+  p.nbp = cdiv(64 * W + 1, kWave) * kWave;
+  p.cap = k + p.rows;
+  const size_t per = static_cast<size_t>(p.gx * p.nbp) * sizeof(uint16_t) +
+                     static_cast<size_t>(p.cap) * sizeof(uint64_t);
+  p.batch = static_cast<int64_t>(kLkMaxBytes / per) / kLkQpw * kLkQpw;
+  p.batch = p.batch < kLkQpw ? kLkQpw : p.batch;
+  p.batch = p.batch < B ? p.batch : B;
+  p.totals = 0;
+  p.cut = align_up(static_cast<size_t>(p.batch * p.nbp) * sizeof(uint32_t), 256);
+  p.counts = p.cut + align_up(static_cast<size_t>(p.batch) * 16, 256);
+  p.buf = p.counts + align_up(static_cast<size_t>(p.batch * p.gx * p.nbp) * sizeof(uint16_t), 256);
+  p.total = p.buf + static_cast<size_t>(p.batch * p.cap) * sizeof(uint64_t);
   return p;
 }
 
-// Step 6: one workgroup per query.
-__global__ void __launch_bounds__(kLkFinalThreads) lk_final_kernel(LkArgs a, int64_t* out_ids,
-                                                                   void* out_scores,
-                                                                   int score_kind) {
-  extern __shared__ uint64_t sm[];
-  uint64_t* tie = sm;             // [kLkCap]
-  uint64_t* all = sm + kLkCap;    // [kLkCap]
-  const int64_t q = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int need2 = a.cut[q * 8 + 4];
-  const int na = a.cnt[q * 4] < kLkCap ? a.cnt[q * 4] : kLkCap;  // == lt
-  const int nb_ = a.cnt[q * 4 + 1] < kLkCap ? a.cnt[q * 4 + 1] : kLkCap;
-  const int nc = a.cnt[q * 4 + 2] < kLkCap ? a.cnt[q * 4 + 2] : kLkCap;
-  const int take = need2 < nc ? need2 : nc;
-  if (take > 0) {
-    const int p = lk_pow2(nc);
-    for (int i = tid; i < p; i += kLkFinalThreads) tie[i] = i < nc ? a.buf_c[q * kLkCap + i] : 0ull;
-    __syncthreads();
-    lk_block_sort(tie, p);  // one score: descending composites = ascending ids
-  }
-  int n = na + nb_ + take;
-  n = n < kLkCap ? n : kLkCap;
-  const int p = lk_pow2(n > 0 ? n : 1);
-  for (int i = tid; i < p; i += kLkFinalThreads) {
-    uint64_t v = 0ull;
-    if (i < na) {
-      v = a.buf_a[q * kLkCap + i];
-    } else if (i < na + nb_) {
-      v = a.buf_b[q * kLkCap + (i - na)];
-    } else if (i < n) {
-      v = tie[i - na - nb_];
-    }
-    all[i] = v;
-  }
-  __syncthreads();
-  lk_block_sort(all, p);
-  for (int i = tid; i < a.k; i += kLkFinalThreads) {
-    const int64_t o = q * a.k + i;
-    if (i < n && all[i] != 0ull) {
-      out_ids[o] = composite_item(all[i]);
-      const int32_t s = i32_of_key(composite_key(all[i]));
-      if (score_kind == kScoreI32) {
-        static_cast<int32_t*>(out_scores)[o] = s;
-      } else {
-        static_cast<float*>(out_scores)[o] = static_cast<float>(s);
-      }
+template <int W>
+int lk_dispatch(int64_t w, const LkArgs& a, dim3 grid, hipStream_t stream, bool emit) {
+  if (w == W) {
+    const size_t lds = static_cast<size_t>(kLkQpw) * a.nb * sizeof(uint32_t);
+    if (emit) {
+      lk_pass_kernel<W, true><<<grid, kLkThreads, lds, stream>>>(a);
     } else {
-      out_ids[o] = -1;
-      if (score_kind == kScoreI32) {
-        static_cast<int32_t*>(out_scores)[o] = INT32_MIN;
-      } else {
-        static_cast<float*>(out_scores)[o] = -INFINITY;
-      }
+      lk_pass_kernel<W, false><<<grid, kLkThreads, lds, stream>>>(a);
     }
+    RT_CHECK_HIP(hipGetLastError());
+    return kOk;
   }
-}
-
-__global__ void __launch_bounds__(256) lk_zero_kernel(int32_t* p, int64_t n) {
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * 256) {
-    p[i] = 0;
-  }
-}
-
-struct LkLayout {
-  size_t hist, cnt, idhist, zero_end, cut, a, b, c, total;
-};
-
-LkLayout lk_layout(int64_t B, int64_t N, int64_t W) {
-  LkLayout l{};
-  const int64_t nb = 64 * W + 1;
-  const int64_t nbin = (N + (int64_t{1} << kLkIdShift) - 1) >> kLkIdShift;
-  l.hist = 0;
-  l.cnt = l.hist + static_cast<size_t>(B * nb) * 4;
-  l.idhist = l.cnt + static_cast<size_t>(B) * 16;
-  l.zero_end = l.idhist + static_cast<size_t>(B * (nbin > 0 ? nbin : 1)) * 4;
-  l.cut = align_up(l.zero_end, 256);
-  l.a = align_up(l.cut + static_cast<size_t>(B) * 32, 256);
-  l.b = l.a + static_cast<size_t>(B) * kLkCap * 8;
-  l.c = l.b + static_cast<size_t>(B) * kLkCap * 8;
-  l.total = l.c + static_cast<size_t>(B) * kLkCap * 8;
-  return l;
-}
-
-template <int W>
-int lk_passes(const LkArgs& a, dim3 grid, hipStream_t stream, int mode) {
-  if (mode == 0) {
-    const size_t lds = static_cast<size_t>(kLkQpw) * a.nb * sizeof(int32_t);
-    lk_pass_kernel<W, 0><<<grid, kLkThreads, lds, stream>>>(a);
-  } else if (mode == 1) {
-    lk_pass_kernel<W, 1><<<grid, kLkThreads, 0, stream>>>(a);
-  } else {
-    lk_pass_kernel<W, 2><<<grid, kLkThreads, 0, stream>>>(a);
-  }
-  RT_CHECK_HIP(hipGetLastError());
-  return kOk;
-}
-
-template <int W>
-int lk_dispatch(int64_t w, const LkArgs& a, dim3 grid, hipStream_t stream, int mode) {
-  if (w == W) return lk_passes<W>(a, grid, stream, mode);
   if constexpr (W < 16) {
-    return lk_dispatch<W + 1>(w, a, grid, stream, mode);
+    return lk_dispatch<W + 1>(w, a, grid, stream, emit);
   } else {
     set_error("Hamming scan supports W in [1, 16], got %lld", static_cast<long long>(w));
     return kInvalidArgument;
@@ -344,8 +354,9 @@ int lk_dispatch(int64_t w, const LkArgs& a, dim3 grid, hipStream_t stream, int m
 
 }  // namespace
 
-size_t hamming_large_k_workspace(int64_t B, int64_t N, int64_t W) {
-  return lk_layout(B, N, W).total;
+size_t hamming_large_k_workspace(int64_t B, int64_t N, int64_t W, int64_t k) {
+  if (B <= 0 || N <= 0 || W <= 0) return 256;
+  return lk_plan(B, N, W, k).total;
 }
 
 int hamming_large_k(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, int64_t N,
@@ -354,59 +365,51 @@ int hamming_large_k(const uint64_t* query_bits, int64_t B, const uint64_t* item_
                     size_t workspace_bytes, hipStream_t stream) {
   RT_CHECK_ARG(k > kMaxK && k <= kMaxKHamming, "k must be in (%lld, %lld] here",
                static_cast<long long>(kMaxK), static_cast<long long>(kMaxKHamming));
-  const LkLayout l = lk_layout(B, N, W);
-  if (workspace_bytes < l.total) {
-    set_error("workspace too small: %zu < %zu", workspace_bytes, l.total);
+  const LkPlan p = lk_plan(B, N, W, k);
+  if (workspace_bytes < p.total) {
+    set_error("workspace too small: %zu < %zu", workspace_bytes, p.total);
     return kWorkspaceTooSmall;
   }
+  RT_CHECK_ARG(p.gx < (int64_t{1} << 31), "N too large");
   char* ws = static_cast<char*>(workspace);
-  LkArgs a{};
-  a.q = query_bits;
-  a.B = B;
-  a.items = item_bits;
-  a.N = N;
-  a.k = static_cast<int>(k);
-  a.mask = mask;
-  a.mask_words = mask_words;
-  a.nb = static_cast<int>(64 * W + 1);
-  a.nbin = (N + (int64_t{1} << kLkIdShift) - 1) >> kLkIdShift;
-  a.hist = reinterpret_cast<uint32_t*>(ws + l.hist);
-  a.cnt = reinterpret_cast<int32_t*>(ws + l.cnt);
-  a.idhist = reinterpret_cast<uint32_t*>(ws + l.idhist);
-  a.cut = reinterpret_cast<int32_t*>(ws + l.cut);
-  a.buf_a = reinterpret_cast<uint64_t*>(ws + l.a);
-  a.buf_b = reinterpret_cast<uint64_t*>(ws + l.b);
-  a.buf_c = reinterpret_cast<uint64_t*>(ws + l.c);
-
-  const int64_t nzero = static_cast<int64_t>(l.zero_end / 4);
-  const int64_t zg = cdiv(nzero, 256) < 4096 ? cdiv(nzero, 256) : 4096;
-  lk_zero_kernel<<<static_cast<unsigned>(zg), 256, 0, stream>>>(
-      reinterpret_cast<int32_t*>(ws + l.hist), nzero);
-  RT_CHECK_HIP(hipGetLastError());
-
-  const int64_t tiles = cdiv(N, kWave);
-  int64_t gx = cdiv(tiles, kLkWaves);
-  gx = gx < kLkMaxGx ? gx : kLkMaxGx;
-  const int64_t gy = cdiv(B, kLkQpw);
-  RT_CHECK_ARG(gy <= 65535, "too many queries");
-  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy));
-  int st = lk_dispatch<1>(W, a, grid, stream, 0);
-  if (st != kOk) return st;
-  lk_cut_kernel<<<static_cast<unsigned>(B), kWave, 0, stream>>>(a);
-  RT_CHECK_HIP(hipGetLastError());
-  st = lk_dispatch<1>(W, a, grid, stream, 1);
-  if (st != kOk) return st;
-  lk_cut2_kernel<<<static_cast<unsigned>(B), kWave, 0, stream>>>(a);
-  RT_CHECK_HIP(hipGetLastError());
-  st = lk_dispatch<1>(W, a, grid, stream, 2);
-  if (st != kOk) return st;
-  const size_t lds = 2 * kLkCap * sizeof(uint64_t);
-  RT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&lk_final_kernel),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   static_cast<int>(lds)));
-  lk_final_kernel<<<static_cast<unsigned>(B), kLkFinalThreads, lds, stream>>>(
-      a, out_ids, out_scores, score_kind);
-  RT_CHECK_HIP(hipGetLastError());
+  const int64_t elem = score_kind == kScoreI32 ? sizeof(int32_t) : sizeof(float);
+  for (int64_t b0 = 0; b0 < B; b0 += p.batch) {
+    LkArgs a{};
+    a.q = query_bits + b0 * W;
+    a.B = B - b0 < p.batch ? B - b0 : p.batch;
+    a.items = item_bits;
+    a.N = N;
+    a.rows = p.rows;
+    a.gx = static_cast<int>(p.gx);
+    a.k = static_cast<int>(k);
+    a.mask = mask != nullptr ? mask + b0 * mask_words : nullptr;
+    a.mask_words = mask_words;
+    a.nb = static_cast<int>(64 * W + 1);
+    a.nbp = static_cast<int>(p.nbp);
+    a.counts = reinterpret_cast<uint16_t*>(ws + p.counts);
+    a.totals = reinterpret_cast<uint32_t*>(ws + p.totals);
+    a.cut = reinterpret_cast<int32_t*>(ws + p.cut);
+    a.cap = p.cap;
+    a.buf = reinterpret_cast<uint64_t*>(ws + p.buf);
+    const int64_t gy = cdiv(a.B, kLkQpw);
+    RT_CHECK_ARG(gy <= 65535 && a.B <= 65535, "too many queries");
+    const dim3 grid(static_cast<unsigned>(p.gx), static_cast<unsigned>(gy));
+    int st = lk_dispatch<1>(W, a, grid, stream, false);
+    if (st != kOk) return st;
+    lk_prefix_kernel<<<dim3(static_cast<unsigned>(p.nbp / kWave), static_cast<unsigned>(a.B)),
+                       kLkPrefixThreads, 0, stream>>>(a);
+    RT_CHECK_HIP(hipGetLastError());
+    lk_cut_kernel<<<static_cast<unsigned>(a.B), kWave, 0, stream>>>(a);
+    RT_CHECK_HIP(hipGetLastError());
+    st = lk_dispatch<1>(W, a, grid, stream, true);
+    if (st != kOk) return st;
+    lk_rank_kernel<<<dim3(static_cast<unsigned>(cdiv(p.cap, kLkThreads)),
+                          static_cast<unsigned>(a.B)),
+                     kLkThreads, 0, stream>>>(a, out_ids + b0 * k,
+                                              static_cast<char*>(out_scores) + b0 * k * elem,
+                                              score_kind);
+    RT_CHECK_HIP(hipGetLastError());
+  }
   return kOk;
 }
 
