@@ -96,7 +96,7 @@ static int64_t small_seed_rows(int64_t N, int64_t k, int64_t rows_per_wg, int64_
 
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
                    int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t seed_rows_min, bool ranked) {
+                   int64_t seed_rows_min, bool ranked, bool spread) {
   ScanPlan s;
   s.qpg = qpg;
   s.n_qgroups = cdiv(B, qpg);
@@ -120,8 +120,8 @@ ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_p
   // stay short, and without one they hold every row they meet, so few rows a list end in the
   // merge instead of in repeated sorts of full lists by one wave (3K rows of fp16 D = 128,
   // top-100, at 1024 and at 128 rows a workgroup: B = 16 195, 31 us; B = 300 1989, 51 us).
-  s.main = plan_pass(N, 1, s.n_qgroups, s.seeded ? kMainMinRows : kMainMinRows / 2, main_capw,
-                     lists_per_wg, lpq, target_wgs);
+  const int64_t min_rows = !spread ? 4 * kMainMinRows : (s.seeded ? kMainMinRows : kMainMinRows / 2);
+  s.main = plan_pass(N, 1, s.n_qgroups, min_rows, main_capw, lists_per_wg, lpq, target_wgs);
   const size_t lists = s.main.lists_bytes > s.seed.lists_bytes ? s.main.lists_bytes
                                                               : s.seed.lists_bytes;
   const size_t counts = s.main.counts_bytes > s.seed.counts_bytes ? s.main.counts_bytes

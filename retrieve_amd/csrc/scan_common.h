@@ -189,11 +189,13 @@ int blocked_hamming(const uint64_t* query_bits, int64_t B, const uint64_t* item_
 // Rows of the seed sample (at least, and kSeedRowsPerK * k at least): the main pass then keeps
 // about k * N / seed rows composites a query (in expectation, for items in random order).
 // `ranked`: the scan bounds its candidates by the sample's rank-th best (sample_rank) with a
-// fallback, so a sparse sample of a small table serves it too.
+// fallback, so a sparse sample of a small table serves it too. `spread`: a small table may be
+// spread over more workgroups, and so more lists, than one a 1024 rows.
 constexpr int64_t kSeedRows = 1 << 18;
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
                    int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t seed_rows_min = kSeedRows, bool ranked = true);
+                   int64_t seed_rows_min = kSeedRows, bool ranked = true,
+                   bool spread = true);
 
 // Writes the -1 / sentinel pads of an empty result.
 int launch_pad(int64_t* out_ids, void* out_scores, int64_t B, int64_t k, int score_kind,

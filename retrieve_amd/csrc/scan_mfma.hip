@@ -3,8 +3,8 @@
 // bf16 / fp16 × same → fp32 (LiNR's dense scores; v_mfma_f32_16x16x32_bf16 / _f16). Ties go to
 // the lower item index.
 //
-// Each wave multiplies 16-item tiles of the item table against its 16 queries (items as the
-// A operand, queries as B), so after a tile lane l holds the scores of query l % 16 for items
+// Each wave multiplies 16-item tiles of the item table against its 16 queries, or 32 as two
+// groups of 16 (items as the A operand, queries as B), so after a tile lane l holds the scores of query l % 16 for items
 // 4 * (l / 16) + r, r < 4. Every MFMA consumes 64 bytes of each row: lane l feeds bytes
 // [64 s + 16 (l / 16), +16) of its item row and of its query row at step s, the same bytes on
 // both sides (the K order inside an operand is free: exact for integers, and within the fp32
@@ -267,19 +267,23 @@ constexpr size_t main_static_lds() {
   return static_cast<size_t>(kScanWaves) * kTile * tile_pitch<KSTEPS>();
 }
 
-// LDS of the clause bitmaps a main-pass workgroup copies (its 16 queries).
-__host__ __device__ inline size_t clause_lds_bytes(int C) {
-  return static_cast<size_t>(16) * C * kSetWords * sizeof(uint64_t);
+// LDS of the clause bitmaps a main-pass workgroup copies (its 16 G queries).
+__host__ __device__ inline size_t clause_lds_bytes(int C, int G) {
+  return static_cast<size_t>(16) * G * C * kSetWords * sizeof(uint64_t);
 }
 
-// Main pass: every item (row_stride 1), candidate lists per wave.
-template <class Op, int KSTEPS>
+// Main pass: every item (row_stride 1), candidate lists per wave. G query groups a wave: with two
+// each tile is loaded and staged once for 32 queries (top-100 calls with one and with two
+// groups: fp16 1M x 384, 50 queries 409, 300 us; int8 10M x 512, 31 queries 1462, 771 us).
+// Temporal loads where several rows of workgroups read the same tiles gained nothing.
+template <class Op, int KSTEPS, int G>
 __global__ void __launch_bounds__(kScanThreads) scan_mfma_kernel(ScanArgs a) {
   using Score = typename Op::Score;
   constexpr int64_t D = KSTEPS * 64;  // row bytes
   constexpr int P = tile_pitch<KSTEPS>();
   if (a.run_if != nullptr && *a.run_if == 0u) return;  // (uniform: the fallback is not needed)
   constexpr int LOADS = KSTEPS;  // 16-byte loads per lane per tile: 16 * D / 1024
+  constexpr int QW = 16 * G;     // queries of this wave
   extern __shared__ __attribute__((aligned(16))) uint64_t smem[];
   const int lane = lane_id();
   const int wave = threadIdx.x >> 6;
@@ -289,71 +293,90 @@ __global__ void __launch_bounds__(kScanThreads) scan_mfma_kernel(ScanArgs a) {
   int8_t* stage = base + wave * kTile * P;
   uint64_t* scratch = reinterpret_cast<uint64_t*>(base + main_static_lds<KSTEPS>()) + wave * a.capw;
   int* cnt = reinterpret_cast<int*>(base + main_static_lds<KSTEPS>() +
-                                    kScanWaves * a.capw * sizeof(uint64_t)) + wave * 16;
+                                    kScanWaves * a.capw * sizeof(uint64_t)) + wave * QW;
   const int64_t wave_in_group = static_cast<int64_t>(blockIdx.x) * kScanWaves + wave;
   const int64_t waves = static_cast<int64_t>(gridDim.x) * kScanWaves;
   const int64_t slot = static_cast<int64_t>(blockIdx.y) * waves + wave_in_group;
-  if (lane < 16) cnt[lane] = 0;
+  if (lane < QW) cnt[lane] = 0;
 
   const int8_t* I = static_cast<const int8_t*>(a.items);
-  const int64_t qrow = static_cast<int64_t>(blockIdx.y) * 16 + col;
-  v4i qf[KSTEPS];
-  load_query_fragments<KSTEPS>(a, qrow, grp, qf);
-  WaveTopK16<Score> top;
-  top.lists = a.lists + slot * 16 * a.capw;
-  top.cnt = cnt;
-  top.scratch = scratch;
-  top.capw = a.capw;
-  top.k = a.k;
-  top.qmask = a.mask != nullptr && qrow < a.B ? a.mask + qrow * a.mask_words : nullptr;
-  top.clause = a.clause;
-  top.clauses = a.clause.active != nullptr && qrow < a.B;  // a padding column tests nothing
+  const int64_t q0 = static_cast<int64_t>(blockIdx.y) * QW;
+  v4i qf[G][KSTEPS];
+#pragma unroll
+  for (int g = 0; g < G; ++g) load_query_fragments<KSTEPS>(a, q0 + 16 * g + col, grp, qf[g]);
+  WaveTopK16<Score> top[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t qrow = q0 + 16 * g + col;
+    top[g].lists = a.lists + (slot * QW + 16 * g) * a.capw;
+    top[g].cnt = cnt + 16 * g;
+    top[g].scratch = scratch;
+    top[g].capw = a.capw;
+    top[g].k = a.k;
+    top[g].qmask = a.mask != nullptr && qrow < a.B ? a.mask + qrow * a.mask_words : nullptr;
+    top[g].clause = a.clause;
+    // (a padding column tests nothing)
+    top[g].clauses = a.clause.active != nullptr && qrow < a.B;
+  }
   if (a.clause.active != nullptr) {
-    // the group's set bitmaps in LDS (after the lists' counts) when the host planned room
+    // the queries' set bitmaps in LDS (after the lists' counts) when the host planned room
     const uint64_t* bm = nullptr;
+    const int per_row = a.clause.C * kSetWords;
     if (a.clause_lds) {
       uint64_t* lds_bm = reinterpret_cast<uint64_t*>(
           base + main_static_lds<KSTEPS>() + kScanWaves * a.capw * sizeof(uint64_t) +
-          kScanWaves * 16 * sizeof(int));
-      const int per_row = a.clause.C * kSetWords;
-      const int64_t g0 = static_cast<int64_t>(blockIdx.y) * 16;
-      for (int i = threadIdx.x; i < 16 * per_row; i += kScanThreads) {
-        const int64_t b = g0 + i / per_row;
+          kScanWaves * QW * sizeof(int));
+      for (int i = threadIdx.x; i < QW * per_row; i += kScanThreads) {
+        const int64_t b = q0 + i / per_row;
         lds_bm[i] = b < a.B ? a.clause.bitmaps[b * per_row + i % per_row] : 0ull;
       }
       __syncthreads();
-      bm = lds_bm + col * per_row;
+      bm = lds_bm;
     }
-    if (top.clauses) top.crow = clause_row(a.clause, qrow, bm);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (top[g].clauses) {
+        const int at = 16 * g + col;
+        top[g].crow = clause_row(a.clause, q0 + at, bm != nullptr ? bm + at * per_row : nullptr);
+      }
+    }
   }
   if (a.probe.doc_bits != nullptr) {
-    // the group's Bloom clause tables copied to LDS (after the set bitmaps) while they fit, in
+    // the queries' Bloom clause tables copied to LDS (after the set bitmaps) while they fit, in
     // query order; the others are read where they are
     uint64_t* tl = reinterpret_cast<uint64_t*>(
         base + main_static_lds<KSTEPS>() + kScanWaves * a.capw * sizeof(uint64_t) +
-        kScanWaves * 16 * sizeof(int) + (a.clause_lds ? clause_lds_bytes(a.clause.C) : 0));
+        kScanWaves * QW * sizeof(int) + (a.clause_lds ? clause_lds_bytes(a.clause.C, G) : 0));
     const int cap = a.probe_lds / static_cast<int>(sizeof(uint64_t));
     const uint64_t* tables = a.probe.tables;
-    const int64_t g0 = static_cast<int64_t>(blockIdx.y) * 16;
-    const int64_t g1 = g0 + 16 < a.B ? g0 + 16 : a.B;
-    const int64_t o0 = static_cast<int64_t>(tables[g0]);
+    const int64_t g1 = q0 + QW < a.B ? q0 + QW : a.B;
+    const int64_t o0 = static_cast<int64_t>(tables[q0]);
     const int words = static_cast<int>(static_cast<int64_t>(tables[g1]) - o0);
-    top.tables_lds = words <= cap;  // (uniform: the group's tables are contiguous)
-    if (top.tables_lds) {
+    const bool fits = words <= cap;  // (uniform: the wave's tables are contiguous)
+    if (fits) {
       for (int w = threadIdx.x; w < words; w += kScanThreads) tl[w] = tables[o0 + w];
       __syncthreads();
-      top.lds = (lds_cu64*)(tl);
     }
-    if (qrow < a.B) {
-      const int64_t o = static_cast<int64_t>(tables[qrow]);
-      top.table = tables + o;
-      top.lds_at = static_cast<int>(o - o0);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int64_t qrow = q0 + 16 * g + col;
+      top[g].tables_lds = fits;
+      if (fits) top[g].lds = (lds_cu64*)(tl);
+      if (qrow < a.B) {
+        const int64_t o = static_cast<int64_t>(tables[qrow]);
+        top[g].table = tables + o;
+        top[g].lds_at = static_cast<int>(o - o0);
+      }
+      top[g].doc_bits = a.probe.doc_bits;
+      top[g].probe_on = true;
+      top[g].probing = qrow < a.B;
     }
-    top.doc_bits = a.probe.doc_bits;
-    top.probe_on = true;
-    top.probing = qrow < a.B;
   }
-  top.set_tau(qrow < a.B ? (a.tau_in != nullptr ? a.tau_in[qrow] : 0ull) : ~0ull);
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t qrow = q0 + 16 * g + col;
+    top[g].set_tau(qrow < a.B ? (a.tau_in != nullptr ? a.tau_in[qrow] : 0ull) : ~0ull);
+  }
   wave_sync_memory();
 
   const int64_t n = a.n_rows;
@@ -384,11 +407,19 @@ __global__ void __launch_bounds__(kScanThreads) scan_mfma_kernel(ScanArgs a) {
       af[s] = *reinterpret_cast<const v4i*>(stage + col * P + grp * 16 + s * 64);
     }
     if (next < ntiles) load_tile(next, v);
-    typename Op::Acc acc = Op::zero();
+    typename Op::Acc acc[G];
 #pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) acc = Op::mma(af[s], qf[s], acc);
-    const Score sc[4] = {acc[0], acc[1], acc[2], acc[3]};
-    top.push(sc, t * kTile + 4 * grp, n, 1);
+    for (int g = 0; g < G; ++g) acc[g] = Op::zero();
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) acc[g] = Op::mma(af[s], qf[g][s], acc[g]);
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const Score sc[4] = {acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
+      top[g].push(sc, t * kTile + 4 * grp, n, 1);
+    }
     wave_sync_memory();
   };
 
@@ -409,13 +440,17 @@ __global__ void __launch_bounds__(kScanThreads) scan_mfma_kernel(ScanArgs a) {
     for (; t < ntiles; t += waves) tile(t, va, t + waves);
   }
   wave_sync_memory();
-  if (lane < 16) a.counts[slot * 16 + lane] = cnt[lane];
+  if (lane < QW) a.counts[slot * QW + lane] = cnt[lane];
 }
 
 template <int KSTEPS>
-static size_t main_lds_bytes(int capw) {
-  return main_static_lds<KSTEPS>() + kScanWaves * (capw * sizeof(uint64_t) + 16 * sizeof(int));
+static size_t main_lds_bytes(int capw, int G) {
+  return main_static_lds<KSTEPS>() +
+         kScanWaves * (capw * sizeof(uint64_t) + 16 * G * sizeof(int));
 }
+
+// Query groups a wave takes: two above 16 queries.
+static int mfma_groups(int64_t B) { return B > 16 ? 2 : 1; }
 
 // The most the main pass gives the LDS copies below: they are made only while two workgroups
 // still fit a CU.
@@ -427,24 +462,13 @@ constexpr size_t kSeedClauseLds = 32 * 1024;
 constexpr size_t kProbeLdsMin = 4 * 1024;
 constexpr size_t kProbeLdsMax = 24 * 1024;
 
-template <class Op, int KSTEPS>
-static int launch_mfma(const ScanArgs& a, const PassPlan& p, int64_t n_qgroups, bool seed,
-                       hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(p.gx), static_cast<unsigned>(n_qgroups));
-  if (seed) {
-    // the seed copies its group's set bitmaps to LDS when they are small
-    ScanArgs s = a;
-    const size_t bm = a.clause.active != nullptr ? clause_lds_bytes(a.clause.C) : 0;
-    s.clause_lds = bm > 0 && bm <= kSeedClauseLds;
-    seed_mfma_kernel<Op, KSTEPS><<<grid, kScanThreads, s.clause_lds ? bm : 0, stream>>>(s);
-    RT_CHECK_HIP(hipGetLastError());
-    return kOk;
-  }
+template <class Op, int KSTEPS, int G>
+static int launch_mfma_main(const ScanArgs& a, dim3 grid, int capw, hipStream_t stream) {
   ScanArgs m = a;
-  size_t lds = main_lds_bytes<KSTEPS>(p.capw);
+  size_t lds = main_lds_bytes<KSTEPS>(capw, G);
   m.clause_lds =
-      a.clause.active != nullptr && lds + clause_lds_bytes(a.clause.C) <= kMainLdsForTwo;
-  if (m.clause_lds) lds += clause_lds_bytes(a.clause.C);
+      a.clause.active != nullptr && lds + clause_lds_bytes(a.clause.C, G) <= kMainLdsForTwo;
+  if (m.clause_lds) lds += clause_lds_bytes(a.clause.C, G);
   m.probe_lds = 0;
   if (a.probe.doc_bits != nullptr && lds + kProbeLdsMin <= kMainLdsForTwo) {
     const size_t room = kMainLdsForTwo - lds;
@@ -452,13 +476,31 @@ static int launch_mfma(const ScanArgs& a, const PassPlan& p, int64_t n_qgroups, 
     lds += m.probe_lds;
   }
   if (lds > 65536) {
-    RT_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(scan_mfma_kernel<Op, KSTEPS>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     static_cast<int>(lds)));
+    RT_CHECK_HIP(hipFuncSetAttribute(
+        reinterpret_cast<const void*>(scan_mfma_kernel<Op, KSTEPS, G>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
   }
-  scan_mfma_kernel<Op, KSTEPS><<<grid, kScanThreads, lds, stream>>>(m);
+  scan_mfma_kernel<Op, KSTEPS, G><<<grid, kScanThreads, lds, stream>>>(m);
   RT_CHECK_HIP(hipGetLastError());
   return kOk;
+}
+
+template <class Op, int KSTEPS>
+static int launch_mfma(const ScanArgs& a, const PassPlan& p, int64_t n_qgroups, bool seed,
+                       hipStream_t stream) {
+  if (seed) {
+    // (16 queries a seed workgroup); it copies its group's set bitmaps to LDS when they are small
+    const dim3 grid(static_cast<unsigned>(p.gx), static_cast<unsigned>(cdiv(a.B, 16)));
+    ScanArgs s = a;
+    const size_t bm = a.clause.active != nullptr ? clause_lds_bytes(a.clause.C, 1) : 0;
+    s.clause_lds = bm > 0 && bm <= kSeedClauseLds;
+    seed_mfma_kernel<Op, KSTEPS><<<grid, kScanThreads, s.clause_lds ? bm : 0, stream>>>(s);
+    RT_CHECK_HIP(hipGetLastError());
+    return kOk;
+  }
+  const dim3 grid(static_cast<unsigned>(p.gx), static_cast<unsigned>(n_qgroups));
+  return a.qpw == 16 ? launch_mfma_main<Op, KSTEPS, 1>(a, grid, p.capw, stream)
+                     : launch_mfma_main<Op, KSTEPS, 2>(a, grid, p.capw, stream);
 }
 
 // Row sizes supported: 64, 128, 256, 512, 768, 1024 bytes (int8 D; half the D for 16-bit).
@@ -501,9 +543,13 @@ static int64_t mfma_seed_rows(int64_t B, int64_t N) {
 constexpr int kSeedTiles = 4;
 
 // The plan of a scan of B queries over N rows, top-k, over target_wgs main-pass workgroups.
-static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, int64_t target_wgs) {
-  return plan_scan(B, N, k, 16, kScanWaves * 16, target_wgs, mfma_capw(k),
-                   kScanWaves * kTile * kSeedTiles, mfma_seed_rows(B, N));
+// `fixed`: the allocation-free form, whose scratch bounds the lists: one query group a wave, and
+// a small table neither seeded nor spread over more workgroups.
+static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, int64_t target_wgs,
+                          bool fixed = false) {
+  const int64_t qpw = fixed ? 16 : 16 * mfma_groups(B);
+  return plan_scan(B, N, k, qpw, kScanWaves * qpw, target_wgs, mfma_capw(k),
+                   kScanWaves * kTile * kSeedTiles, mfma_seed_rows(B, N), !fixed, !fixed);
 }
 
 // seed scan → seed threshold merge → main scan → final merge, on `stream`, no host sync
@@ -513,7 +559,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
                          int64_t* out_ids, void* out_scores, void* workspace,
                          size_t workspace_bytes, hipStream_t stream,
                          const ClauseCheck& clause = ClauseCheck{},
-                         const BloomProbe& probe = BloomProbe{}) {
+                         const BloomProbe& probe = BloomProbe{}, bool fixed = false) {
   RT_CHECK_ARG(B >= 0 && N >= 0, "B and N must be >= 0");
   RT_CHECK_ARG(k >= 1 && k <= kMaxK, "k must be in [1, %lld], got %lld",
                static_cast<long long>(kMaxK), static_cast<long long>(k));
@@ -527,7 +573,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   if (N == 0) return launch_pad(out_ids, out_scores, B, k, Op::kind, stream);
   RT_CHECK_ARG(queries != nullptr && items != nullptr && workspace != nullptr,
                "queries, items and workspace must not be null");
-  const ScanPlan plan = mfma_plan(B, N, k, main_workgroups());
+  const ScanPlan plan = mfma_plan(B, N, k, main_workgroups(), fixed);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;
@@ -553,7 +599,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   a.B = B;
   a.items = items;
   a.k = static_cast<int>(k);
-  a.qpw = 16;
+  a.qpw = static_cast<int>(plan.qpg);
   a.mask = mask;
   a.mask_words = mask_words;
   a.lists = lists;
@@ -563,7 +609,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   MergeArgs m{};
   m.lists = lists;
   m.counts = counts;
-  m.qpw = 16;
+  m.qpw = static_cast<int>(plan.qpg);
   m.B = B;
   m.k = static_cast<int>(k);
 
@@ -696,8 +742,7 @@ extern "C" int rt_int8_scan_topk_noalloc(const int8_t* queries, int64_t B, const
   RT_CHECK_ARG(B == 0 || (out_ids != nullptr && out_scores != nullptr &&
                           (N == 0 || (queries != nullptr && items != nullptr))),
                "queries, items, out_ids and out_scores must not be null");
-  const size_t need = mfma_plan(B, N, k, main_workgroups())
-                          .total;
+  const size_t need = mfma_plan(B, N, k, main_workgroups(), true).total;
   RT_CHECK_ARG(need <= kNoAllocScratchBytes,
                "rt_int8_scan_topk_noalloc: B = %lld, N = %lld, k = %lld need %zu bytes of "
                "scratch, above its fixed %zu bytes (call rt_int8_scan_topk with a workspace)",
@@ -707,7 +752,7 @@ extern "C" int rt_int8_scan_topk_noalloc(const int8_t* queries, int64_t B, const
   const int st = noalloc_scratch(&ws);
   if (st != kOk) return st;
   return run_mfma_scan<I8Op>(queries, B, items, N, D, k, mask, mask_words, out_ids, out_scores,
-                             ws, kNoAllocScratchBytes, stream);
+                             ws, kNoAllocScratchBytes, stream, ClauseCheck{}, BloomProbe{}, true);
 }
 
 // ---- scans with the exact clause filter tested per candidate --------------------------------

@@ -45,6 +45,25 @@ def test_int8(dev, n, b, k):
     assert np.array_equal(sc.cpu().numpy(), want_sc)
 
 
+@pytest.mark.parametrize("b", [16, 17, 32, 33, 65])
+@pytest.mark.parametrize("n,d,k", [(300, 768, 20), (20_000, 1024, 10), (30_001, 64, 1000)])
+def test_query_groups(dev, n, d, k, b):
+    """Row widths the register-blocked scan does not take, on either side of one and two 16-query
+    groups a wave, plain and masked."""
+    import retrieve_amd.hip  # noqa: F401
+
+    print(f"groups n={n} d={d} b={b} k={k}", flush=True)
+    g = rng(n + d + b)
+    items = g.integers(-20, 21, (n, d), dtype=np.int8)
+    q = g.integers(-20, 21, (b, d), dtype=np.int8)
+    for valid in (None, g.random((b, n)) < 0.1):
+        ids, sc = torch.ops.retrieve_amd.int8_scan_topk(
+            _t(dev, q), _t(dev, items), k, None if valid is None else _t(dev, _pack(valid)))
+        want_ids, want_sc = _want(q, items, k, valid)
+        assert np.array_equal(ids.cpu().numpy(), want_ids)
+        assert np.array_equal(sc.cpu().numpy(), want_sc)
+
+
 @pytest.mark.parametrize("share", [0.2, 0.002, 0.0])
 @pytest.mark.parametrize("n,b,k", [(66_049, 5, 100), (140_001, 33, 100), (20_000, 150, 40),
                                    (70_000, 18, 1000)])
