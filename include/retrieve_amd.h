@@ -363,6 +363,16 @@ int rt_scan_topk_bloom_clauses(const void* queries, int64_t B, const void* items
                                int64_t V, int64_t* out_ids, void* out_scores, void* workspace,
                                size_t workspace_bytes, rt_stream_t stream);
 
+/* The inputs of rt_bloom_search_columns for a probe table of n = rows * per_row list ids (at most
+ * rt_probe_columns_max()): per entry its cluster's start (0 for a list that does not exist), the
+ * inclusive sum of the columns spanned (ceil((len + start % 64) / 64), 0 when empty) and
+ * start % 64.
+ * Replaces: generate_column_info_for_clusters (silvertorch/.../bloom_index_search.cpp:447-490). */
+int64_t rt_probe_columns_max(void);
+int rt_probe_columns(const int64_t* probe_ids, int64_t n, const int64_t* cluster_offsets,
+                     const int64_t* cluster_sizes, int64_t n_lists, int64_t* starts,
+                     int32_t* column_counts_cumsum, int8_t* first_offsets, rt_stream_t stream);
+
 /* The Bloom plans over the probed clusters' columns only: probed cluster i (row i / per_row of a
  * [rows, per_row] probe table) starts at doc position cluster_starts[i] and spans
  * column_counts_cumsum[i] - column_counts_cumsum[i - 1] columns (inclusive int32 cumsum) from

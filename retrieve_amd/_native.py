@@ -141,6 +141,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "rt_search_epilogue": (
         _c_int, [_c_p, _c_p, _c_p, _c_i64, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p],
     ),
+    "rt_probe_columns_max": (_c_i64, []),
+    "rt_probe_columns": (
+        _c_int, [_c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p],
+    ),
     "rt_bloom_search_columns": (
         _c_int,
         [_c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p,

@@ -793,17 +793,21 @@ def _column_info(starts: Tensor, lengths: Tensor, plan_count: int,
     if starts.shape != lengths.shape:
         raise RuntimeError("selected_cluster_offsets must have the shape of "
                            "selected_cluster_lengths")
-    if query_plan_index is not None:
-        if query_plan_index.dim() != 1 or query_plan_index.shape[0] != starts.shape[0]:
-            raise RuntimeError("query_plan_index must be [B]")
-    elif plan_count != starts.shape[0]:
-        raise RuntimeError("without query_plan_index there must be one plan per row")
+    _check_plan_rows(starts.shape[0], plan_count, query_plan_index)
     starts = starts.contiguous()
     off = torch.remainder(starts, 64)
     counts = torch.where(lengths > 0, torch.div(lengths + off + 63, 64, rounding_mode="floor"),
                          torch.zeros_like(lengths))
     return (counts.reshape(-1).cumsum(0).to(torch.int32), off.reshape(-1).to(torch.int8),
             starts.reshape(-1))
+
+
+def _check_plan_rows(rows: int, plan_count: int, query_plan_index: Tensor | None) -> None:
+    if query_plan_index is not None:
+        if query_plan_index.dim() != 1 or query_plan_index.shape[0] != rows:
+            raise RuntimeError("query_plan_index must be [B]")
+    elif plan_count != rows:
+        raise RuntimeError("without query_plan_index there must be one plan per row")
 
 
 def _columns(bloom_index, offsets, plan_offsets, data, data_bytes, plan_count, max_stack, k,
@@ -862,21 +866,31 @@ def _partial_response_prepared(bloom_index, bloom_bundle_b_offsets, plans, plan_
     """Prepared plans, no host sync: ``column_mask_response`` has the caller's static capacity
     ``max_columns``; its words past the probed columns' total are 0
     (``bloom_index_search_cuda.cu:1857-1940``)."""
+    _check_prepared(plans, plan_count, max_stack_size, max_columns)
+    cumsum, first, starts = _column_info(selected_cluster_offsets, selected_cluster_lengths,
+                                         int(plan_count), query_plan_index)
+    words = _prepared_columns(bloom_index, bloom_bundle_b_offsets, plans, plan_count,
+                              max_stack_size, k, hash_k, starts, cumsum,
+                              selected_cluster_lengths.shape[1], query_plan_index, max_columns)
+    return cumsum, first, words
+
+
+def _check_prepared(plans, plan_count, max_stack_size, max_columns) -> None:
     if plans.dtype != torch.int64 or plans.dim() != 1 or plans.numel() < 8 * plan_count:
         raise ValueError("plans must be int64 [8 * plan_count + data words]")
     if max_stack_size > MAX_STACK:
         raise ValueError(f"max_stack_size must be <= {MAX_STACK}")
     if max_columns < 0:
         raise ValueError("max_columns must be >= 0")
+
+
+def _prepared_columns(bloom_index, bloom_bundle_b_offsets, plans, plan_count, max_stack_size, k,
+                      hash_k, starts, cumsum, per_row, query_plan_index, max_columns) -> Tensor:
     plans = plans.contiguous()
     data = plans[8 * plan_count :]
-    cumsum, first, starts = _column_info(selected_cluster_offsets, selected_cluster_lengths,
-                                         int(plan_count), query_plan_index)
-    words = _columns(bloom_index.contiguous(), bloom_bundle_b_offsets.contiguous(), plans, data,
-                     data.numel() * 8, int(plan_count), int(max_stack_size), int(k), int(hash_k),
-                     starts, cumsum, selected_cluster_lengths.shape[1], query_plan_index,
-                     int(max_columns))
-    return cumsum, first, words
+    return _columns(bloom_index.contiguous(), bloom_bundle_b_offsets.contiguous(), plans, data,
+                    data.numel() * 8, int(plan_count), int(max_stack_size), int(k), int(hash_k),
+                    starts, cumsum, per_row, query_plan_index, int(max_columns))
 
 
 _LIB.impl("bloom_index_search_batch_return_partial_response", _partial_response, "CUDA")
@@ -1244,16 +1258,32 @@ def _payload_bloom(bloom_index, bloom_bundle_b_offsets, plans, plan_count, max_s
     if biggest is None:
         return None
     n_lists = offs.numel()
-    valid = (probes >= 0) & (probes < n_lists)
-    cluster = torch.where(valid, probes, 0)
-    starts = torch.where(valid, offs[cluster], 0).contiguous()
-    lengths = torch.where(valid, sizes[cluster], 0).contiguous()
     # a payload of at most `biggest` docs spans at most biggest / 64 + 2 columns
     max_columns = probes.numel() * ((biggest + 63) // 64 + 1)
     qpi = None if query_plan_index is None else query_plan_index.to(torch.int64)
-    return _partial_response_prepared(bloom_index, bloom_bundle_b_offsets, plans, plan_count,
-                                      max_stack_size, starts, lengths, bloom_k, hash_k, qpi,
-                                      max_columns)
+    if probes.numel() > nat.lib().rt_probe_columns_max():
+        valid = (probes >= 0) & (probes < n_lists)
+        cluster = torch.where(valid, probes, 0)
+        starts = torch.where(valid, offs[cluster], 0).contiguous()
+        lengths = torch.where(valid, sizes[cluster], 0).contiguous()
+        return _partial_response_prepared(bloom_index, bloom_bundle_b_offsets, plans, plan_count,
+                                          max_stack_size, starts, lengths, bloom_k, hash_k, qpi,
+                                          max_columns)
+    _check_prepared(plans, plan_count, max_stack_size, max_columns)
+    _check_plan_rows(probes.shape[0], int(plan_count), qpi)
+    n = probes.numel()
+    starts = torch.empty((n,), dtype=torch.int64, device=probes.device)
+    cumsum = torch.empty((n,), dtype=torch.int32, device=probes.device)
+    first = torch.empty((n,), dtype=torch.int8, device=probes.device)
+    with torch.cuda.device(probes.device):
+        st = nat.lib().rt_probe_columns(
+            nat.ptr(probes), n, nat.ptr(offs), nat.ptr(sizes), n_lists, nat.ptr(starts),
+            nat.ptr(cumsum), nat.ptr(first), nat.stream(probes.device))
+    nat.check(st)
+    words = _prepared_columns(bloom_index, bloom_bundle_b_offsets, plans, plan_count,
+                              max_stack_size, bloom_k, hash_k, starts, cumsum, probes.shape[1],
+                              qpi, max_columns)
+    return cumsum, first, words
 
 
 # Row widths (int8 D) the full-scan kernels take; other widths run the IVF kernel.
@@ -1330,10 +1360,14 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
     if exact:
         slots = item_clause_attrs.to(torch.int32).contiguous()
         cs = clause_slots.to(torch.int64).contiguous()
-        rev = clause_is_reverse.to(torch.int8).contiguous()
-        qv = query_clause_attrs.to(torch.int64)
-        qv = torch.where((qv >= -1) & (qv <= 2**31 - 1), qv, -(2**31)).to(torch.int32)
-        qv = qv.contiguous()
+        rev = clause_is_reverse.contiguous()
+        # (a bool flag is its 0 / 1 byte: a view, not a copy kernel a call)
+        rev = rev.view(torch.int8) if rev.dtype == torch.bool else rev.to(torch.int8)
+
+        def clamped():  # values no doc may hold (outside [-1, 2^31 - 1]) as INT32_MIN
+            v = query_clause_attrs.to(torch.int64)
+            v = torch.where((v >= -1) & (v <= 2**31 - 1), v, -(2**31)).to(torch.int32)
+            return v.contiguous()
     full = (divisor_for_int8 == -1 and offs.numel() == 1 and probes.shape[1] == 1
             and width >= n and d in _FULL_SCAN_D
             and _one_list_is_the_table(cluster_offsets, cluster_sizes, n))
@@ -1347,6 +1381,9 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
                                      max_stack_size, bloom_k, hash_k, query_plan_index, probes,
                                      offs, sizes)
         if partial is not None or plans is None:
+            if exact:  # (the scan itself takes int32 values below -1 for INT32_MIN)
+                qv = query_clause_attrs.contiguous() \
+                    if query_clause_attrs.dtype == torch.int32 else clamped()
             cum, first, words = partial if partial is not None else (None, None, None)
             ws = nat.workspace(lib.rt_ivf_search_workspace(b, width, k), dev)
             with torch.cuda.device(dev):
@@ -1374,6 +1411,7 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
         mask = bm[query_plan_index.to(torch.int64)] if query_plan_index is not None else bm[:b]
         mask = mask.contiguous()
     if exact:
+        qv = clamped()
         out = torch.empty((b, (n + 63) // 64), dtype=torch.int64, device=dev)
         with torch.cuda.device(dev):
             st = lib.rt_clause_slots_filter(

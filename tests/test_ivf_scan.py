@@ -71,3 +71,35 @@ def test_layouts(dev, b, n, n_lists, n_probe, k, width):
     for dtype in (np.int64, np.int32):
         ids, sc = _run(*args, **kw, query_clause_attrs=_t(dev, qa.astype(dtype)))
         assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+
+
+@pytest.mark.parametrize("b,n_probe", [(1, 1), (5, 130), (130, 126), (130, 127)])
+def test_bloom_payloads(dev, b, n_probe):
+    """The probed columns' table from one kernel (up to 16,384 probe entries) and past it: Bloom
+    plans with the recheck give the exact filter's result; lists that do not exist, empty lists
+    and starts inside a column."""
+    import retrieve_amd.st as st
+    from retrieve_amd import bloom as bl
+
+    g = rng(330 + b + n_probe)
+    n, d, c, k, lists = 6000, 64, 2, 25, 200
+    items, offsets, sizes, perm = _ivf(g, n, d, lists)
+    sizes = np.where(g.random(lists) < 0.1, 0, sizes)
+    q = g.standard_normal((b, d)).astype(np.float32)
+    probes = np.stack([g.permutation(lists)[:n_probe] for _ in range(b)]).astype(np.int64)
+    probes[0, 0] = lists
+    attrs = g.integers(0, 5, (n, c, 1)).astype(np.int64)
+    qa = g.integers(0, 5, (b, c)).astype(np.int64)
+    rev = np.zeros(c, bool)
+    words, boffs = torch.ops.st.bloom_index_build_fixed(*st.attrs_to_features(_t(dev, attrs)),
+                                                        64, 3)
+    blob, count, stack = st.prepare_plans(bl.queries_to_expressions(qa, rev), 7, dev)
+    ids, sc = _run(dev, q, probes, offsets, sizes, items, perm, 0.3, k, n, bloom_index=words,
+                   bloom_bundle_b_offsets=boffs, plans=blob, plan_count=count,
+                   max_stack_size=stack, bloom_k=3, hash_k=7,
+                   item_clause_attrs=_t(dev, attrs[:, :, 0].T.astype(np.int32)),
+                   clause_slots=_t(dev, np.arange(c + 1, dtype=np.int64)),
+                   clause_is_reverse=_t(dev, rev), query_clause_attrs=_t(dev, qa))
+    want = ost.search(q, probes, offsets, sizes, items, perm, [0.3], k, n,
+                      valid=of.clause_match(attrs, rev, qa))
+    assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
