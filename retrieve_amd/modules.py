@@ -581,8 +581,12 @@ class LiNRV3(RetrievalModule):
         if prepared is None:
             cand, _ = self.stage1(query)
             return self.stage2(query, candidate_ids=cand)
-        cand, _ = self.stage1.forward_bits(query, _filter(self.filter).mask_bits(prepared))
-        return self.stage2(query, candidate_ids=cand, counts=(cand >= 0).sum(dim=1))
+        # the shortlist's ids alone: its scores are not needed, and the re-rank skips the -1 past a
+        # row's passing items, so they need no counting either (six launches less a batch)
+        bits = _filter(self.filter).mask_bits(prepared)
+        cand, _ = xops.hamming_scan_topk(self.stage1._project_query(query),
+                                         self.stage1.item_bits, self.stage1.k, bits)
+        return self.stage2(query, candidate_ids=cand)
 
 
 def _check_pool(candidate_pool: int) -> None:
