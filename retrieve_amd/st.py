@@ -1248,6 +1248,12 @@ def _max_cluster(sizes: Tensor) -> int | None:
     return hit
 
 
+def _n_lists(offs: Tensor, sizes: Tensor) -> int:
+    """The lists of an index: those with both an offset and a size (CSR offsets hold one entry
+    more). Probe ids from there on name no list."""
+    return min(offs.numel(), sizes.numel())
+
+
 def _payload_bloom(bloom_index, bloom_bundle_b_offsets, plans, plan_count, max_stack_size,
                    bloom_k, hash_k, query_plan_index, probes, offs, sizes):
     """The Bloom words of every row's probed payloads only (``bloom_index_search_cuda.cu:
@@ -1257,7 +1263,7 @@ def _payload_bloom(bloom_index, bloom_bundle_b_offsets, plans, plan_count, max_s
     biggest = _max_cluster(sizes)
     if biggest is None:
         return None
-    n_lists = offs.numel()
+    n_lists = _n_lists(offs, sizes)
     # a payload of at most `biggest` docs spans at most biggest / 64 + 2 columns
     max_columns = probes.numel() * ((biggest + 63) // 64 + 1)
     qpi = None if query_plan_index is None else query_plan_index.to(torch.int64)
@@ -1354,6 +1360,7 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
     offs = cluster_offsets.to(torch.int64).contiguous()
     sizes = cluster_sizes.to(torch.int64).contiguous()
     probes = probe_ids.to(torch.int64).contiguous()
+    n_lists = _n_lists(offs, sizes)
     lib = nat.lib()
     if plans is not None and (bloom_index is None or bloom_bundle_b_offsets is None):
         raise RuntimeError("plans need bloom_index and bloom_bundle_b_offsets")
@@ -1389,7 +1396,7 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
             with torch.cuda.device(dev):
                 st = lib.rt_ivf_search_payload_filters(
                     nat.ptr(codes), nat.ptr(scales), b, nat.ptr(item_codes), n, d,
-                    nat.ptr(probes), probes.shape[1], nat.ptr(offs), nat.ptr(sizes), offs.numel(),
+                    nat.ptr(probes), probes.shape[1], nat.ptr(offs), nat.ptr(sizes), n_lists,
                     width, nat.ptr(cum), nat.ptr(first), nat.ptr(words),
                     0 if first is None else first.numel(), 0 if words is None else words.numel(),
                     nat.ptr(slots) if exact else None,
@@ -1442,7 +1449,7 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
     with torch.cuda.device(dev):
         st = lib.rt_ivf_search(
             nat.ptr(codes), nat.ptr(scales), b, nat.ptr(item_codes), n, d, nat.ptr(probes),
-            probes.shape[1], nat.ptr(offs), nat.ptr(sizes), offs.numel(), width, nat.ptr(mask),
+            probes.shape[1], nat.ptr(offs), nat.ptr(sizes), n_lists, width, nat.ptr(mask),
             0 if mask is None else mask.shape[1], int(divisor_for_int8), nat.ptr(perm),
             perm.numel(), nat.ptr(gs), k, nat.ptr(ids), nat.ptr(scores), nat.ptr(ws), ws.numel(),
             nat.stream(dev))
@@ -1460,7 +1467,7 @@ def _search_large_k(codes, scales, item_codes, probes, offs, sizes, width, mask,
     from retrieve_amd import large_k
 
     b = codes.shape[0]
-    n_lists = offs.numel()
+    n_lists = _n_lists(offs, sizes)
     dev = codes.device
     valid = (probes >= 0) & (probes < n_lists)
     cluster = torch.where(valid, probes, 0)

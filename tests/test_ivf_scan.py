@@ -103,3 +103,42 @@ def test_bloom_payloads(dev, b, n_probe):
     want = ost.search(q, probes, offsets, sizes, items, perm, [0.3], k, n,
                       valid=of.clause_match(attrs, rev, qa))
     assert np.array_equal(ids, want[0]) and np.array_equal(sc, want[1])
+
+
+@pytest.mark.parametrize("end", ["n", "zero"])
+def test_probe_past_the_sizes(dev, end):
+    """CSR offsets hold one entry more than the sizes: a probe of that id names no list, with every
+    filter form and above k = 1024. (The sizes are a view whose next entry, in the same
+    allocation, is a large count.)"""
+    import retrieve_amd.st as st
+    from retrieve_amd import bloom as bl
+
+    g = rng(340)
+    n, d, b, c, lists = 6000, 64, 4, 2, 60
+    items, offsets, sizes, perm = _ivf(g, n, d, lists)
+    csr = _t(dev, np.append(offsets, n if end == "n" else 0))
+    lens = _t(dev, np.append(sizes, 5000))[:lists]
+    q = g.standard_normal((b, d)).astype(np.float32)
+    probes = np.stack([g.permutation(lists)[:12] for _ in range(b)]).astype(np.int64)
+    probes[:, 0] = lists
+    attrs = g.integers(0, 3, (n, c, 1)).astype(np.int64)
+    qa = g.integers(0, 3, (b, c)).astype(np.int64)
+    rev = np.zeros(c, bool)
+    exact = of.clause_match(attrs, rev, qa)
+    words, boffs = torch.ops.st.bloom_index_build_fixed(*st.attrs_to_features(_t(dev, attrs)),
+                                                        64, 3)
+    blob, count, stack = st.prepare_plans(bl.queries_to_expressions(qa, rev), 7, dev)
+    clauses = dict(item_clause_attrs=_t(dev, attrs[:, :, 0].T.astype(np.int32)),
+                   clause_slots=_t(dev, np.arange(c + 1, dtype=np.int64)),
+                   clause_is_reverse=_t(dev, rev), query_clause_attrs=_t(dev, qa))
+    bloom = dict(bloom_index=words, bloom_bundle_b_offsets=boffs, plans=blob, plan_count=count,
+                 max_stack_size=stack, bloom_k=3, hash_k=7)
+    for valid, k, kw in ((None, 25, {}), (exact, 25, clauses), (exact, 25, {**bloom, **clauses}),
+                         (exact, 25, dict(filtering_bit_mask=_t(dev, _pack(exact)))),
+                         (None, 1100, {})):
+        print(f"probe past the sizes end={end} k={k} {sorted(kw)}", flush=True)
+        ids, sc = torch.ops.st.search(_t(dev, q), _t(dev, probes), csr, lens, _t(dev, items),
+                                      _t(dev, perm), _t(dev, np.float32([0.3])), k, n, -1, **kw)
+        want = ost.search(q, probes, offsets, sizes, items, perm, [0.3], k, n, valid=valid)
+        assert np.array_equal(ids.cpu().numpy(), want[0])
+        assert np.array_equal(sc.cpu().numpy(), want[1])
