@@ -267,18 +267,22 @@ def _hamming_call(query_bits, item_bits, k, mask, score_dtype):
 
 @torch.library.custom_op("retrieve_amd::hamming_scan_topk", mutates_args=(), device_types="cuda")
 def hamming_scan_topk(
-    query_bits: Tensor, item_bits: Tensor, k: int, mask: Tensor | None = None
+    query_bits: Tensor, item_bits: Tensor, k: int, mask: Tensor | None = None,
+    float_scores: bool = False,
 ) -> tuple[Tensor, Tensor]:
     """Exact 1-bit Hamming full-scan top-k on the integer score ``64 W - 2 popcount(q ^ item)``:
     ``(ids int64 [B, k], scores int32 [B, k])``, ties to the lower index, ``-1`` /
-    ``INT32_MIN`` where fewer than ``k`` items pass ``mask``."""
-    return _hamming_call(query_bits, item_bits, k, mask, torch.int32)
+    ``INT32_MIN`` where fewer than ``k`` items pass ``mask``. With ``float_scores`` the scores
+    are written as fp32, ``-inf`` in the places of ``INT32_MIN``."""
+    return _hamming_call(query_bits, item_bits, k, mask,
+                         torch.float32 if float_scores else torch.int32)
 
 
 @hamming_scan_topk.register_fake
-def _(query_bits, item_bits, k, mask=None):
+def _(query_bits, item_bits, k, mask=None, float_scores=False):
     b = query_bits.shape[0]
-    return (query_bits.new_empty((b, k)), query_bits.new_empty((b, k), dtype=torch.int32))
+    return (query_bits.new_empty((b, k)),
+            query_bits.new_empty((b, k), dtype=torch.float32 if float_scores else torch.int32))
 
 
 @torch.library.custom_op(

@@ -378,8 +378,8 @@ class _PackedBitsKNN(RetrievalModule):
     def forward_bits(self, query: Tensor, bits: Tensor | None) -> tuple[Tensor, Tensor]:
         """Full scan restricted to the items set in packed ``bits``: ``(ids, fp32 scores)``,
         ``-1`` / ``-inf`` past the passing items."""
-        ids, s = xops.hamming_scan_topk(self._project_query(query), self.item_bits, self.k, bits)
-        return ids, torch.where(ids >= 0, s.to(torch.float32), float("-inf"))
+        return xops.hamming_scan_topk(self._project_query(query), self.item_bits, self.k, bits,
+                                      True)
 
     def forward(self, query: Tensor, candidate_ids: Tensor | None = None,
                 counts: Tensor | None = None) -> tuple[Tensor, Tensor]:
@@ -581,11 +581,8 @@ class LiNRV3(RetrievalModule):
         if prepared is None:
             cand, _ = self.stage1(query)
             return self.stage2(query, candidate_ids=cand)
-        # the shortlist's ids alone: its scores are not needed, and the re-rank skips the -1 past a
-        # row's passing items, so they need no counting either (six launches less a batch)
-        bits = _filter(self.filter).mask_bits(prepared)
-        cand, _ = xops.hamming_scan_topk(self.stage1._project_query(query),
-                                         self.stage1.item_bits, self.stage1.k, bits)
+        # (the re-rank skips the -1 past a row's passing items: they need no counting)
+        cand, _ = self.stage1.forward_bits(query, _filter(self.filter).mask_bits(prepared))
         return self.stage2(query, candidate_ids=cand)
 
 

@@ -57,3 +57,27 @@ def test_batches(dev):
     want_ids, want_sc = osc.hamming_topk(q[rows], items, k, valid[rows])
     assert np.array_equal(ids[rows.tolist()].cpu().numpy(), want_ids)
     assert np.array_equal(sc[rows.tolist()].cpu().numpy(), want_sc)
+
+
+@pytest.mark.parametrize("k", [40, 1500])
+def test_float_scores(dev, k):
+    """A packed-bits module's filtered scan: fp32 scores with -inf past the passing items, the
+    integer scan's values."""
+    import retrieve_amd.hip  # noqa: F401
+    from retrieve_amd.modules import SimHashKNN
+
+    g = rng(81 + k)
+    n, b, d = 3000, 5, 64
+    m = SimHashKNN(k, k_bits=128, seed=2)
+    m.register_index(_t(dev, g.standard_normal((n, d)).astype(np.float32)))
+    q = _t(dev, g.standard_normal((b, d)).astype(np.float32))
+    valid = g.random((b, n)) < 0.2
+    valid[0] = False
+    valid[1, 30:] = False
+    bits = _t(dev, _pack(valid))
+    print(f"float scores k={k}", flush=True)
+    ids, sc = m.forward_bits(q, bits)
+    want_ids, want = torch.ops.retrieve_amd.hamming_scan_topk(m._project_query(q), m.item_bits,
+                                                              k, bits)
+    assert sc.dtype == torch.float32 and torch.equal(ids, want_ids)
+    assert torch.equal(sc, torch.where(want_ids >= 0, want.float(), float("-inf")))

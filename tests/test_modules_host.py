@@ -129,3 +129,29 @@ def test_blocked_gate_mirrors_the_kernel_plan():
     assert hip._use_blocked(64, 256, 700)  # two 32 KiB stages beside 1024-entry lists
     assert not hip._use_blocked(31, 256, 100)  # below the blocked batch
     assert hip._use_blocked(300, 512, 990)  # narrow 32-row tiles: lists of 1024
+
+
+def test_linr_v3_takes_its_shortlist_from_forward_bits(mods):
+    """The filtered forward's shortlist is what stage 1's ``forward_bits`` returns, also where a
+    subclass overrides it."""
+    shortlist = torch.tensor([[3, 1, -1]])
+    seen = {}
+
+    class Stage1(mods.OneBitKNN):
+        def forward_bits(self, query, bits):
+            seen["bits"] = bits
+            return shortlist, torch.zeros((1, 3))
+
+    class Stage2(mods.PrefilterKNN):
+        def forward(self, query, candidate_ids=None, counts=None):
+            return candidate_ids, counts
+
+    class Words(mods.ExactAttributeFilter):
+        def mask_bits(self, q):
+            return q
+
+    v3 = mods.LiNRV3(2, candidate_pool=3, filter=Words())
+    v3.stage1, v3.stage2 = Stage1(3), Stage2(2)
+    prepared = torch.tensor([[7]])
+    cand, _ = v3(torch.zeros((1, 64)), prepared)
+    assert torch.equal(cand, shortlist) and seen["bits"] is prepared
