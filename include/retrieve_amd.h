@@ -4,7 +4,8 @@
  * Conventions for every entry point:
  * - pointers are device pointers (HIP) unless stated; inputs are read-only and borrowed;
  *   outputs are caller-allocated; scratch comes from a caller-allocated `workspace` whose
- *   size the matching `*_workspace` function returns;
+ *   size the matching `*_workspace` function returns (for the current device, the one the call
+ *   runs on);
  * - work is enqueued on `stream` (a hipStream_t); no entry point synchronizes the host;
  * - the return value is 0 on success, else a status: 1 invalid argument (shape, size or
  *   range), 2 unsupported type/width, 3 a HIP call failed, 4 workspace too small;

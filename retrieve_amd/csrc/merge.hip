@@ -23,7 +23,7 @@ const char* last_error() { return g_error; }
 
 // ---- planning ---------------------------------------------------------------------------
 
-// Workgroups a seed pass aims for, and the main pass's when the device cannot be queried.
+// Workgroups a seed pass aims for.
 static constexpr int64_t kTargetWorkgroups = 2048;
 // At least this many sampled rows per wanted item (keeps the main pass's candidates near
 // k * N / seed_rows for large k).
@@ -36,9 +36,14 @@ static constexpr int64_t kMainMinRows = 256;
 // per query group).
 static constexpr int64_t kMaxListBytes = int64_t{2} << 30;
 
+// `list_tile` (0: not known): rows of one tile that a list meets, tiles dealt in turn to the lists
+// of a query; the most a tile can add. The lists are then cut to the rows they can meet and one
+// tile's room: a list of that length never fills, so it is never sorted and needs neither a
+// power of two nor k entries. (100K rows at k = 1000, one query: 20 MB of lists; 504 MB at the
+// full 2048 entries a list.)
 static PassPlan plan_pass(int64_t n_rows, int64_t row_stride, int64_t n_qgroups, int64_t min_rows,
                           int capw, int64_t lists_per_wg, int64_t lists_per_query_per_wg,
-                          int64_t target_wgs, int64_t min_gx = 1) {
+                          int64_t target_wgs, int64_t min_gx = 1, int64_t list_tile = 0) {
   PassPlan p;
   p.n_rows = n_rows;
   p.row_stride = row_stride;
@@ -60,23 +65,30 @@ static PassPlan plan_pass(int64_t n_rows, int64_t row_stride, int64_t n_qgroups,
   p.gx = cdiv(n_rows, p.strip);
   if (p.gx < 1) p.gx = 1;
   p.S = p.gx * lists_per_query_per_wg;
-  p.lists_bytes = static_cast<size_t>(p.gx) * n_qgroups * lists_per_wg * capw * sizeof(uint64_t);
+  if (list_tile > 0) {
+    const int64_t meets = cdiv(n_rows, list_tile * p.S) * list_tile;
+    const int64_t cap = cdiv(meets + list_tile, kTile) * kTile;
+    p.capw = static_cast<int>(cap < capw ? cap : capw);
+  }
+  p.lists_bytes =
+      static_cast<size_t>(p.gx) * n_qgroups * lists_per_wg * p.capw * sizeof(uint64_t);
   p.counts_bytes = static_cast<size_t>(p.gx) * n_qgroups * lists_per_wg * sizeof(int);
   // the seed's flat one-entry lists: [B rounded up to groups][S]
   return p;
 }
 
-int64_t main_workgroups() {
+int64_t device_cus() {
   int dev = 0;
   int cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0) {
-    return kTargetWorkgroups;
+    return 256;
   }
-  const int64_t t = static_cast<int64_t>(cus) * kMainWorkgroupsPerCU;
-  return t < kMaxResidentWorkgroups ? t : kMaxResidentWorkgroups;
+  return cus;
 }
+
+int64_t main_workgroups() { return device_cus() * kMainWorkgroupsPerCU; }
 
 // Sampled rows of a table too small for the full sample: one row in 16, 8 or 4, the sparsest whose
 // one-entry lists are enough for the bound's rank; 0 where none is (the scan then runs unseeded).
@@ -96,7 +108,7 @@ static int64_t small_seed_rows(int64_t N, int64_t k, int64_t rows_per_wg, int64_
 
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
                    int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t seed_rows_min, bool ranked, bool spread) {
+                   int64_t list_tile, int64_t seed_rows_min, bool ranked, bool spread) {
   ScanPlan s;
   s.qpg = qpg;
   s.n_qgroups = cdiv(B, qpg);
@@ -121,7 +133,8 @@ ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_p
   // merge instead of in repeated sorts of full lists by one wave (3K rows of fp16 D = 128,
   // top-100, at 1024 and at 128 rows a workgroup: B = 16 195, 31 us; B = 300 1989, 51 us).
   const int64_t min_rows = !spread ? 4 * kMainMinRows : (s.seeded ? kMainMinRows : kMainMinRows / 2);
-  s.main = plan_pass(N, 1, s.n_qgroups, min_rows, main_capw, lists_per_wg, lpq, target_wgs);
+  s.main = plan_pass(N, 1, s.n_qgroups, min_rows, main_capw, lists_per_wg, lpq, target_wgs, 1,
+                     list_tile);
   const size_t lists = s.main.lists_bytes > s.seed.lists_bytes ? s.main.lists_bytes
                                                               : s.seed.lists_bytes;
   const size_t counts = s.main.counts_bytes > s.seed.counts_bytes ? s.main.counts_bytes

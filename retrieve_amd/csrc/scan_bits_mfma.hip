@@ -384,12 +384,6 @@ int bits_qgroups(int64_t B) {
   return static_cast<int>(g < kMaxQGroups ? g : kMaxQGroups);
 }
 
-ScanPlan bits_plan(int64_t B, int64_t N, int64_t k, int64_t target_wgs) {
-  const int64_t qpg = 16 * bits_qgroups(B);
-  return plan_scan(B, N, k, qpg, kScanWaves * qpg, target_wgs, bits_capw(k),
-                   kScanWaves * kTileRows, kSeedRows / 2);
-}
-
 // LDS of a main-pass workgroup: each wave's compaction scratch and list lengths.
 size_t bits_main_lds(int capw, int nq) {
   return kScanWaves * (static_cast<size_t>(capw) * sizeof(uint64_t) + 16 * nq * sizeof(int));
@@ -399,6 +393,16 @@ size_t bits_main_lds(int capw, int nq) {
 // workgroups a CU.
 bool bits_small_tiles(int nq, int capw) {
   return (nq == 2 || nq == 3) && kWavesSmall * bits_main_lds(capw, nq) <= kLdsPerCU;
+}
+
+ScanPlan bits_plan(int64_t B, int64_t N, int64_t k) {
+  const int nq = bits_qgroups(B);
+  const int64_t qpg = 16 * nq;
+  // (the 64-row-tile form: three workgroups a CU, its occupancy)
+  const int64_t target = bits_small_tiles(nq, bits_capw(k)) ? main_workgroups() * kWavesSmall / 2
+                                                            : main_workgroups();
+  return plan_scan(B, N, k, qpg, kScanWaves * qpg, target, bits_capw(k), kScanWaves * kTileRows,
+                   kTileRows, kSeedRows / 2);
 }
 
 template <int NQ, int TG>
@@ -424,7 +428,7 @@ int launch_bits(const ScanArgs& a, const PassPlan& p, int64_t nqg, bool seed,
   }
   const size_t lds = bits_main_lds(p.capw, NQ);
   if constexpr (NQ == 2 || NQ == 3) {
-    if (bits_small_tiles(NQ, p.capw)) return launch_main<NQ, kTileGroupsSmall>(a, grid, lds, stream);
+    if (bits_small_tiles(NQ, bits_capw(a.k))) return launch_main<NQ, kTileGroupsSmall>(a, grid, lds, stream);
   }
   return launch_main<NQ, kTileGroups>(a, grid, lds, stream);
 }
@@ -442,7 +446,7 @@ int dispatch_bits(int nq, const ScanArgs& a, const PassPlan& p, int64_t nqg, boo
 }  // namespace
 
 size_t bits_mfma_workspace(int64_t B, int64_t N, int64_t k) {
-  return bits_plan(B > 0 ? B : 1, N, k, kMaxResidentWorkgroups).total;
+  return bits_plan(B > 0 ? B : 1, N, k).total;
 }
 
 // seed scan → rank-th bound merge → main scan → final merge (→ fallback scan and merge while
@@ -461,10 +465,7 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
                    reinterpret_cast<uintptr_t>(item_bits) % 16 == 0,
                "query_bits must be 4-byte and item_bits 16-byte aligned");
   const int nq = bits_qgroups(B);
-  // (the 64-row-tile form: three workgroups a CU, its occupancy)
-  const bool small_tiles = bits_small_tiles(nq, bits_capw(k));
-  const ScanPlan plan =
-      bits_plan(B, N, k, small_tiles ? main_workgroups() * kWavesSmall / 2 : main_workgroups());
+  const ScanPlan plan = bits_plan(B, N, k);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;

@@ -1071,16 +1071,16 @@ __global__ void __launch_bounds__(256) mask_transpose_kernel(const uint64_t* mas
 // The plan, and with a mask the transposed mask's place at the end of the workspace.
 // The plan; after its own areas the speculative bounds [B] and the fallback flag, then, with a
 // mask, the transposed mask.
-static ScanPlan blk_plan(int64_t B, int64_t N, int64_t k, int64_t row_bytes, int64_t target_cus,
-                         bool bits, bool masked, size_t* off_mask_t = nullptr,
-                         size_t* off_spec = nullptr) {
+static ScanPlan blk_plan(int64_t B, int64_t N, int64_t k, int64_t row_bytes, bool bits,
+                         bool masked, size_t* off_mask_t = nullptr, size_t* off_spec = nullptr) {
   const bool wide = blk_choose_wide(row_bytes, B, k, bits, masked);
   // the row-quarter layout covers column tiles 0-3 only (B <= kBlkWideMaxBatch = 128), the bit
   // codes' eight row parts tiles 0-1 (B <= 64): their lists are sized for those queries
   const int halves = blk_halves(row_bytes, wide, bits);
   const int64_t qpg = halves == 8 ? kBlkQpg / 4 : (halves == 4 ? kBlkQpg / 2 : kBlkQpg);
-  ScanPlan p = plan_scan(B, N, k, qpg, halves * qpg, target_cus * (wide ? 1 : 2),
-                         blk_capw(k, blk_rows(row_bytes, wide, bits)), kBlkRows);
+  const int rows = blk_rows(row_bytes, wide, bits);
+  ScanPlan p = plan_scan(B, N, k, qpg, halves * qpg, device_cus() * (wide ? 1 : 2),
+                         blk_capw(k, rows), kBlkRows, rows / halves);
   if (off_spec != nullptr) *off_spec = align_up(p.total, 256);
   p.total = align_up(p.total, 256) + align_up(static_cast<size_t>(B) * sizeof(uint64_t), 256) +
             256;
@@ -1120,17 +1120,13 @@ static int run_blocked(const void* queries, int64_t B, const void* items, int64_
   if (N == 0) return launch_pad(out_ids, out_scores, B, k, score_kind, stream);
   RT_CHECK_ARG(queries != nullptr && items != nullptr && workspace != nullptr,
                "queries, items and workspace must not be null");
-  int dev = 0;
-  int cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess) {
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  }
   const bool wide = blk_choose_wide(row_bytes, B, k, Op::kBits, mask != nullptr);
   size_t off_mask_t = 0;
   size_t off_spec = 0;
-  const ScanPlan plan = blk_plan(B, N, k, row_bytes, cus, Op::kBits, mask != nullptr,
-                                 &off_mask_t, &off_spec);
-  RT_CHECK_ARG(blk_stages(row_bytes, plan.main.capw, wide, Op::kBits, mask != nullptr) != 0,
+  const ScanPlan plan =
+      blk_plan(B, N, k, row_bytes, Op::kBits, mask != nullptr, &off_mask_t, &off_spec);
+  const int full_capw = blk_capw(k, blk_rows(row_bytes, wide, Op::kBits));
+  RT_CHECK_ARG(blk_stages(row_bytes, full_capw, wide, Op::kBits, mask != nullptr) != 0,
                "k = %lld is too large for the blocked scan at %lld-byte rows",
                static_cast<long long>(k), static_cast<long long>(row_bytes));
   if (workspace_bytes < plan.total) {

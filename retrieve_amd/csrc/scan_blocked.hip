@@ -7,7 +7,7 @@ using namespace rt;
 extern "C" size_t rt_blocked_scan_topk_workspace(int64_t B, int64_t N, int64_t row_bytes,
                                                  int64_t k, int masked) {
   // (the most workgroups any device runs: the workspace covers every CU count)
-  return blk_plan(B, N, k, row_bytes, kMaxResidentWorkgroups, false, masked != 0).total;
+  return blk_plan(B, N, k, row_bytes, false, masked != 0).total;
 }
 
 // dtype: 0 int8 (int32 scores), 1 bf16, 2 fp16, 3 fp32 (float scores); D elements per row.

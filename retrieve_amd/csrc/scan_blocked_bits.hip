@@ -10,7 +10,7 @@ bool blocked_hamming_fits(int64_t B, int64_t W, int64_t k, bool masked) {
 }
 
 size_t blocked_hamming_workspace(int64_t B, int64_t N, int64_t W, int64_t k, bool masked) {
-  return blk_plan(B, N, k, 8 * W, kMaxResidentWorkgroups, true, masked).total;
+  return blk_plan(B, N, k, 8 * W, true, masked).total;
 }
 
 int blocked_hamming(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, int64_t N,

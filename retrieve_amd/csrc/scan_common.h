@@ -37,7 +37,8 @@ struct ScanArgs {
   int64_t strip;           // rows per workgroup, a multiple of kTile
   int k;
   int qpw;                 // queries per wave (a query group), for scans that vary it
-  int capw;                // list capacity (>= k + the appends one tile can make)
+  int capw;                // list capacity (>= k + the appends one tile can make, or the rows
+                           // the list can meet + those appends)
   const uint64_t* tau_in;  // [B] lower bounds (composites) or null
   const uint64_t* mask;    // [B, mask_words] item bits, item d at bit 63 - d % 64, or null
   int64_t mask_words;
@@ -147,13 +148,13 @@ struct ScanPlan {
   bool split = false;  // room for a split merge at off_parts
 };
 
-// Upper bound on a main pass's workgroups (the workspace functions size for it).
-constexpr int64_t kMaxResidentWorkgroups = 4096;
 // Main-pass workgroups per CU: two, each streaming its share of every window of the table
 // (measured best on MI355X; more workgroups only add candidate lists).
 constexpr int64_t kMainWorkgroupsPerCU = 2;
 
-// Main-pass workgroups for the current device: CUs x kMainWorkgroupsPerCU.
+// CUs of the current device (256 where there is none), and its main-pass workgroups: CUs x
+// kMainWorkgroupsPerCU. The workspace functions and the launches plan for the same count.
+int64_t device_cus();
 int64_t main_workgroups();
 
 // The 1-bit Hamming top-k on the int8 matrix cores (scan_blocked_bits.hip): codes of W 64-bit
@@ -183,9 +184,10 @@ int blocked_hamming(const uint64_t* query_bits, int64_t B, const uint64_t* item_
                     int64_t mask_t_stride = 0);
 
 // Sizes the passes for B queries over N rows and top-k. A workgroup row (grid.y) covers qpg
-// queries and each workgroup keeps lists_per_wg candidate lists (of main_capw entries in the
-// main pass); the main pass runs target_wgs workgroups in all; a seed workgroup scores at
-// least seed_rows_per_wg sampled rows.
+// queries and each workgroup keeps lists_per_wg candidate lists (in the main pass of main_capw
+// entries, or the rows a list can meet where those are fewer: list_tile rows a tile); the main
+// pass runs target_wgs workgroups in all; a seed workgroup scores at least seed_rows_per_wg
+// sampled rows.
 // Rows of the seed sample (at least, and kSeedRowsPerK * k at least): the main pass then keeps
 // about k * N / seed rows composites a query (in expectation, for items in random order).
 // `ranked`: the scan bounds its candidates by the sample's rank-th best (sample_rank) with a
@@ -194,7 +196,7 @@ int blocked_hamming(const uint64_t* query_bits, int64_t B, const uint64_t* item_
 constexpr int64_t kSeedRows = 1 << 18;
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
                    int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t seed_rows_min = kSeedRows, bool ranked = true,
+                   int64_t list_tile, int64_t seed_rows_min = kSeedRows, bool ranked = true,
                    bool spread = true);
 
 // Writes the -1 / sentinel pads of an empty result.

@@ -233,6 +233,11 @@ static int dispatch_ham(int64_t W, const ScanArgs& a, const PassPlan& p, int64_t
   return dispatch_ham_from<1>(W, a, p, nqg, seed, stream);
 }
 
+static ScanPlan ham_plan(int64_t B, int64_t N, int64_t k, int qpw) {
+  return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), ham_capw(k),
+                   kScanWaves * kHamTile, kHamTile, kSeedRows, false);
+}
+
 static int ham_qpw(int64_t B) { return static_cast<int>(B < kHamMaxQpw ? B : kHamMaxQpw); }
 
 // From this batch on, the blocked scan on the fp4 matrix cores (bits as e2m1 nibbles) takes the
@@ -273,9 +278,7 @@ extern "C" size_t rt_hamming_scan_topk_workspace(int64_t B, int64_t N, int64_t W
     return blocked_hamming_workspace(B, N, W, k, masked != 0);
   }
   const int qpw = ham_qpw(B > 0 ? B : 1);
-  return plan_scan(B, N, k, qpw, kScanWaves * qpw, kMaxResidentWorkgroups, ham_capw(k),
-                   kScanWaves * kHamTile, kSeedRows, false)
-      .total;
+  return ham_plan(B, N, k, qpw).total;
 }
 
 extern "C" int rt_hamming_scan_topk(const uint64_t* query_bits, int64_t B,
@@ -310,8 +313,7 @@ extern "C" int rt_hamming_scan_topk(const uint64_t* query_bits, int64_t B,
                            out_scores, kind, workspace, workspace_bytes, stream);
   }
   const int qpw = ham_qpw(B);
-  const ScanPlan plan = plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), ham_capw(k),
-                                  kScanWaves * kHamTile, kSeedRows, false);
+  const ScanPlan plan = ham_plan(B, N, k, qpw);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;

@@ -542,14 +542,14 @@ static int64_t mfma_seed_rows(int64_t B, int64_t N) {
 // 2.349-2.352 ms with eight, 2.338-2.341 ms with four (the plain int8 scan 2.253 / 2.260 ms).
 constexpr int kSeedTiles = 4;
 
-// The plan of a scan of B queries over N rows, top-k, over target_wgs main-pass workgroups.
-// `fixed`: the allocation-free form, whose scratch bounds the lists: one query group a wave, and
-// a small table neither seeded nor spread over more workgroups.
-static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, int64_t target_wgs,
-                          bool fixed = false) {
+// The plan of a scan of B queries over N rows, top-k. `fixed`: the allocation-free form, whose
+// scratch bounds the lists: one query group a wave, and a small table neither seeded nor spread
+// over more workgroups, its lists not cut.
+static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, bool fixed = false) {
   const int64_t qpw = fixed ? 16 : 16 * mfma_groups(B);
-  return plan_scan(B, N, k, qpw, kScanWaves * qpw, target_wgs, mfma_capw(k),
-                   kScanWaves * kTile * kSeedTiles, mfma_seed_rows(B, N), !fixed, !fixed);
+  return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), mfma_capw(k),
+                   kScanWaves * kTile * kSeedTiles, fixed ? 0 : kTile, mfma_seed_rows(B, N),
+                   !fixed, !fixed);
 }
 
 // seed scan → seed threshold merge → main scan → final merge, on `stream`, no host sync
@@ -573,7 +573,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   if (N == 0) return launch_pad(out_ids, out_scores, B, k, Op::kind, stream);
   RT_CHECK_ARG(queries != nullptr && items != nullptr && workspace != nullptr,
                "queries, items and workspace must not be null");
-  const ScanPlan plan = mfma_plan(B, N, k, main_workgroups(), fixed);
+  const ScanPlan plan = mfma_plan(B, N, k, fixed);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;
@@ -677,8 +677,7 @@ using namespace rt;
 
 extern "C" size_t rt_int8_scan_topk_workspace(int64_t B, int64_t N, int64_t D, int64_t k) {
   (void)D;
-  return mfma_plan(B, N, k, kMaxResidentWorkgroups)
-      .total;
+  return mfma_plan(B, N, k).total;
 }
 
 extern "C" int rt_int8_scan_topk(const int8_t* queries, int64_t B, const int8_t* items,
@@ -742,7 +741,7 @@ extern "C" int rt_int8_scan_topk_noalloc(const int8_t* queries, int64_t B, const
   RT_CHECK_ARG(B == 0 || (out_ids != nullptr && out_scores != nullptr &&
                           (N == 0 || (queries != nullptr && items != nullptr))),
                "queries, items, out_ids and out_scores must not be null");
-  const size_t need = mfma_plan(B, N, k, main_workgroups(), true).total;
+  const size_t need = mfma_plan(B, N, k, true).total;
   RT_CHECK_ARG(need <= kNoAllocScratchBytes,
                "rt_int8_scan_topk_noalloc: B = %lld, N = %lld, k = %lld need %zu bytes of "
                "scratch, above its fixed %zu bytes (call rt_int8_scan_topk with a workspace)",
@@ -758,8 +757,7 @@ extern "C" int rt_int8_scan_topk_noalloc(const int8_t* queries, int64_t B, const
 // ---- scans with the exact clause filter tested per candidate --------------------------------
 
 static size_t mfma_plan_bytes(int64_t B, int64_t N, int64_t k) {
-  return mfma_plan(B, N, k, kMaxResidentWorkgroups)
-      .total;
+  return mfma_plan(B, N, k).total;
 }
 
 extern "C" size_t rt_scan_topk_clauses_workspace(int64_t B, int64_t N, int64_t D, int64_t k,
@@ -854,8 +852,7 @@ extern "C" int rt_scan_topk_bloom_clauses(
 
 extern "C" size_t rt_dense_scan_topk_workspace(int64_t B, int64_t N, int64_t D, int64_t k) {
   (void)D;
-  return mfma_plan(B, N, k, kMaxResidentWorkgroups)
-      .total;
+  return mfma_plan(B, N, k).total;
 }
 
 extern "C" int rt_dense_scan_topk(const void* queries, int64_t B, const void* items, int64_t N,

@@ -63,9 +63,9 @@ def _blocked(q: Tensor, items: Tensor, k: int, dtype: int, mask: Tensor | None,
     n = items.shape[0]
     lib = nat.lib()
     dev = q.device
-    ws = nat.workspace(lib.rt_blocked_scan_topk_workspace(b, n, d * q.element_size(), k,
-                                                          int(mask is not None)), dev)
     with torch.cuda.device(dev):
+        ws = nat.workspace(lib.rt_blocked_scan_topk_workspace(b, n, d * q.element_size(), k,
+                                                              int(mask is not None)), dev)
         st = lib.rt_blocked_scan_topk(
             nat.ptr(q), b, nat.ptr(items), n, d, k, dtype, nat.ptr(mask),
             0 if mask is None else mask.shape[1], nat.ptr(ids), nat.ptr(scores), nat.ptr(ws),
@@ -123,9 +123,8 @@ def int8_scan_topk(
         _blocked(q, item_codes, k, 0, mask, ids, scores)
         return ids, scores
     lib = nat.lib()
-    ws_bytes = lib.rt_int8_scan_topk_workspace(b, n, d, k)
-    ws = nat.workspace(ws_bytes, dev)
     with torch.cuda.device(dev):
+        ws = nat.workspace(lib.rt_int8_scan_topk_workspace(b, n, d, k), dev)
         st = lib.rt_int8_scan_topk(
             nat.ptr(q), b, nat.ptr(item_codes), n, d, k, nat.ptr(mask),
             0 if mask is None else mask.shape[1],
@@ -193,8 +192,8 @@ def dense_scan_topk(
         _blocked(q, item_embs, k, 1 + _DENSE_DTYPES[q.dtype], mask, ids, scores)
         return ids, scores
     lib = nat.lib()
-    ws = nat.workspace(lib.rt_dense_scan_topk_workspace(b, n, d, k), dev)
     with torch.cuda.device(dev):
+        ws = nat.workspace(lib.rt_dense_scan_topk_workspace(b, n, d, k), dev)
         st = lib.rt_dense_scan_topk(
             nat.ptr(q), b, nat.ptr(item_embs), n, d, k, _DENSE_DTYPES[q.dtype], nat.ptr(mask),
             0 if mask is None else mask.shape[1], nat.ptr(ids), nat.ptr(scores), nat.ptr(ws),
@@ -253,9 +252,9 @@ def _hamming_call(query_bits, item_bits, k, mask, score_dtype):
     ids = torch.empty((b, k), dtype=torch.int64, device=dev)
     scores = torch.empty((b, k), dtype=score_dtype, device=dev)
     lib = nat.lib()
-    ws = nat.workspace(lib.rt_hamming_scan_topk_workspace(b, n, w, k, int(mask is not None)),
-                       dev)
     with torch.cuda.device(dev):
+        ws = nat.workspace(lib.rt_hamming_scan_topk_workspace(b, n, w, k, int(mask is not None)),
+                           dev)
         st = lib.rt_hamming_scan_topk(
             nat.ptr(q), b, nat.ptr(item_bits), n, w, k, nat.ptr(mask),
             0 if mask is None else mask.shape[1], nat.ptr(ids), nat.ptr(scores),
@@ -627,8 +626,8 @@ def hamming_scan_topk_clauses(
     v = qs.shape[2]
     ids = torch.empty((b, k), dtype=torch.int64, device=dev)
     scores = torch.empty((b, k), dtype=torch.int32, device=dev)
-    ws = nat.workspace(lib.rt_hamming_scan_topk_clauses_workspace(b, n, w, k, c, v), dev)
     with torch.cuda.device(dev):
+        ws = nat.workspace(lib.rt_hamming_scan_topk_clauses_workspace(b, n, w, k, c, v), dev)
         st = lib.rt_hamming_scan_topk_clauses(
             nat.ptr(q), b, nat.ptr(item_bits), n, w, k, nat.ptr(mask), mask.shape[1], ts,
             nat.ptr(item_clause_attrs), item_clause_attrs.element_size(), c, a, nat.ptr(rev),

@@ -90,3 +90,26 @@ def test_no_alloc_rejections_need_no_gpu():
     assert st == 1 and b"must not be null" in lib.rt_last_error()
     st = lib.rt_int8_scan_topk(None, 2, None, 10, 64, 5, None, 0, None, None, None, 0, None)
     assert st == 1 and b"null" in lib.rt_last_error()
+
+
+def test_scan_workspaces_follow_the_rows():
+    """A scan's lists are no longer than the rows they can meet: a query's lists hold about the
+    table's rows once, whatever k is (a list a wave, one tile's room in each)."""
+    import torch  # noqa: F401
+
+    from retrieve_amd import _native
+
+    lib = _native.lib()
+    for n in (1000, 20_000, 100_000, 300_000):
+        for b in (1, 16, 31, 200):
+            for k in (10, 100, 1000):
+                queries = -(-b // 32) * 32  # whole query groups of a wave
+                rows = n + 64 * 8192  # (at most 8192 lists a query, a tile of up to 64 rows each)
+                bound = queries * rows * 8 + (16 << 20)
+                for need in (lib.rt_int8_scan_topk_workspace(b, n, 512, k),
+                             lib.rt_dense_scan_topk_workspace(b, n, 128, k),
+                             lib.rt_hamming_scan_topk_workspace(b, n, 2, k, 0)):
+                    assert need <= bound, (n, b, k, need >> 20)
+    # one query over a 51 MB table
+    assert lib.rt_int8_scan_topk_workspace(1, 100_000, 512, 1000) <= 64 << 20
+    assert lib.rt_int8_scan_topk_workspace(16, 100_000, 512, 100) <= 32 << 20
