@@ -317,7 +317,13 @@ static int dispatch_cand(const CandArgs& a, dim3 grid, size_t lds, hipStream_t s
   return launch_cand<KIND, 64, 8, 2>(a, grid, lds, stream);
 }
 
-static int cand_capw(int64_t k) { return static_cast<int>(next_pow2(k + kWave)); }
+// List capacity: k and a batch's appends, a power of two (sorted whole), or the candidates a wave
+// meets and those appends where they are fewer (such a list never fills and is never sorted).
+static int cand_capw(int64_t k, int64_t P, int64_t S) {
+  const int64_t full = next_pow2(k + kWave);
+  const int64_t meets = cdiv(P, S * kWave) * kWave + kWave;
+  return static_cast<int>(meets < full ? meets : full);
+}
 
 // A query's lists hold up to k entries each (a wave starts without a bound), so its merge is split
 // from few lists, up to a batch whose merges fill the CUs.
@@ -340,7 +346,7 @@ using namespace rt;
 extern "C" size_t rt_cand_topk_workspace(int64_t B, int64_t P, int64_t k) {
   if (B <= 0 || P <= 0 || k <= 0) return 256;
   const int64_t S = cand_gx(B, P) * kCandWaves;
-  return align_up(static_cast<size_t>(B * S) * cand_capw(k) * sizeof(uint64_t), 256) +
+  return align_up(static_cast<size_t>(B * S) * cand_capw(k, P, S) * sizeof(uint64_t), 256) +
          align_up(static_cast<size_t>(B * S) * sizeof(int), 256) +
          (B <= kCandSplitMaxB ? static_cast<size_t>(B) * kMergeParts * k * sizeof(uint64_t) : 0);
 }
@@ -383,7 +389,7 @@ static int cand_topk(const void* queries, int64_t B, const void* items, int64_t 
   }
   const int64_t gx = cand_gx(B, P);
   const int64_t S = gx * kCandWaves;
-  const int capw = cand_capw(k);
+  const int capw = cand_capw(k, P, S);
   RT_CHECK_ARG(B <= 65535, "B must be <= 65535");
   CandArgs a{};
   a.queries = queries;

@@ -871,7 +871,13 @@ static int dispatch_ivf(int64_t D, const IvfArgs& a, dim3 grid, size_t lds, hipS
   return launch_ivf<64, 8, 2>(a, grid, lds, stream);
 }
 
-static int ivf_capw(int64_t k) { return static_cast<int>(next_pow2(k + kWave)); }
+// List capacity: k and a batch's appends, a power of two (sorted whole), or the slots of a wave's run
+// and those appends where they are fewer (such a list never fills and is never sorted).
+static int ivf_capw(int64_t k, int64_t width, int64_t S) {
+  const int64_t full = next_pow2(k + kWave);
+  const int64_t run = cdiv(width, S * kWave) * kWave + kWave;
+  return static_cast<int>(run < full ? run : full);
+}
 
 // A row's lists hold up to k entries each (a wave starts without a bound), so its merge is split
 // from far fewer lists than a seeded scan's, up to a batch whose merges fill the CUs: 64 rows of
@@ -1001,7 +1007,7 @@ extern "C" int rt_pack_oporp(const float* x, int64_t rows, int64_t dim, const in
 extern "C" size_t rt_ivf_search_workspace(int64_t B, int64_t width, int64_t k) {
   if (B <= 0 || k <= 0) return 256;
   const int64_t S = ivf_gx(B, width) * kIvfWaves;
-  return align_up(static_cast<size_t>(B * S) * ivf_capw(k) * sizeof(uint64_t), 256) +
+  return align_up(static_cast<size_t>(B * S) * ivf_capw(k, width, S) * sizeof(uint64_t), 256) +
          align_up(static_cast<size_t>(B * S) * sizeof(int), 256) +
          align_up(static_cast<size_t>(B * k) * sizeof(float), 256) +
          (B <= kIvfSplitMaxB ? static_cast<size_t>(B) * kMergeParts * k * sizeof(uint64_t) : 0);
@@ -1038,7 +1044,7 @@ static int ivf_search(const int8_t* q_codes, const float* q_scales, int64_t B,
   }
   const int64_t gx = ivf_gx(B, width);
   const int64_t S = gx * kIvfWaves;
-  const int capw = ivf_capw(k);
+  const int capw = ivf_capw(k, width, S);
   IvfArgs a{};
   a.q = q_codes;
   a.B = B;

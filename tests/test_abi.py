@@ -113,3 +113,23 @@ def test_scan_workspaces_follow_the_rows():
     # one query over a 51 MB table
     assert lib.rt_int8_scan_topk_workspace(1, 100_000, 512, 1000) <= 64 << 20
     assert lib.rt_int8_scan_topk_workspace(16, 100_000, 512, 100) <= 32 << 20
+
+
+def test_candidate_workspaces_follow_the_candidates():
+    """The candidate and IVF scans' lists hold about the row's candidates (or slots) once, whatever k
+    is: at most 1024 lists a query, each up to two batches of 64 over its share."""
+    import torch  # noqa: F401
+
+    from retrieve_amd import _native
+
+    lib = _native.lib()
+    for b in (1, 8, 64, 256):
+        for p in (100, 5000, 80_000, 1_000_000):
+            for k in (10, 100, 1000):
+                lists = 8 * b * (p + 1024 * 128)
+                bound = lists + 8 * b * 8 * k + 12 * b * k + (4 << 20)
+                assert lib.rt_cand_topk_workspace(b, p, k) <= bound, (b, p, k)
+                assert lib.rt_ivf_search_workspace(b, p, k) <= bound, (b, p, k)
+    # 80K candidates (or slots) of 16 queries at k = 1000
+    assert lib.rt_cand_topk_workspace(16, 80_000, 1000) <= 24 << 20
+    assert lib.rt_ivf_search_workspace(16, 80_000, 1000) <= 24 << 20
