@@ -439,6 +439,7 @@ static int cand_topk(const void* queries, int64_t B, const void* items, int64_t 
         reinterpret_cast<char*>(a.list_counts) +
         align_up(static_cast<size_t>(B * S) * sizeof(int), 256));
     m.part_slots = kCandPartSlots;
+    m.max_entries = P;
   }
   return launch_merge(m, stream);
 }

@@ -94,6 +94,7 @@ struct MergeArgs {
   // and merges those (flat) in a second launch.
   uint64_t* part_buf;
   int part_slots;  // lists a part holds at least (0: kMergeMinPartSlots)
+  int64_t max_entries;  // entries a query's lists hold at most (0: not known)
   // (set by launch_merge) parts per query, and the parts' output in the first launch
   int parts;
   uint64_t* part_out;

@@ -1102,6 +1102,7 @@ static int ivf_search(const int8_t* q_codes, const float* q_scales, int64_t B,
     m.score_kind = score_kind;
     m.part_buf = parts;
     m.part_slots = kIvfPartSlots;
+    m.max_entries = width;
     st = launch_merge(m, stream);
     if (st != kOk) return st;
   } else {
