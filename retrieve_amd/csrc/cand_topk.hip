@@ -143,6 +143,8 @@ struct CandArgs {
 // Bound: the gather of P rows a query, at best the row bytes from HBM; what limits it is how
 // many rows are in flight. One row a group and step, its id load waited for first, 16 queries
 // over 80K of 800K fp16 rows of 128 each took 263 us; 64 ids a load and V rows in flight take 65.
+// A wave takes up to 64 ids at a time, fewer where 64 would leave some waves a round more than
+// others (256 queries of 3000 fp32 rows of 1024 574 us at 64, 462 so).
 template <int KIND, int L, int NC, int V>
 __global__ void __launch_bounds__(kCandThreads) cand_scan_kernel(CandArgs a) {
   using Op = CandOp<KIND>;
@@ -200,13 +202,17 @@ __global__ void __launch_bounds__(kCandThreads) cand_scan_kernel(CandArgs a) {
   for (int i = 1, v = V / 2; v > 0; i <<= 1, v >>= 1) own |= (gl & i) ? v : 0;
   uint64_t tau = 0;  // composites below it cannot reach this wave's best k
   int cnt = 0;
-  const int64_t step = S * kWave;
+  // ids a wave takes at a time: the fewest that leave every wave the same number of rounds
+  const int64_t rounds = count > 0 ? (count + S * kWave - 1) / (S * kWave) : 1;
+  const int64_t chunk = (count + S * rounds - 1) / (S * rounds);  // <= 64
+  const int64_t step = S * chunk;
   const int8_t* I = static_cast<const int8_t*>(a.items);
-  const int64_t* ids = a.ids + b * a.P;
-  int64_t next = slot * kWave + lane < count ? ids[slot * kWave + lane] : -1;
-  for (int64_t base = slot * kWave; base < count; base += step) {
+  const int64_t* ids = a.ids + b * a.P + lane;
+  const int64_t left = lane < chunk ? count - lane : 0;  // bases below it hold an id of this lane
+  int64_t next = slot * chunk < left ? ids[slot * chunk] : -1;
+  for (int64_t base = slot * chunk; base < count; base += step) {
     int64_t item = next;
-    next = base + step + lane < count ? ids[base + step + lane] : -1;
+    next = base + step < left ? ids[base + step] : -1;
     bool ok = item >= 0 && item < a.N;  // ids outside the table are skipped, not read
     int64_t r = ok ? item : 0;
     if (a.rows != nullptr && ok) {
@@ -330,13 +336,25 @@ static int cand_capw(int64_t k, int64_t P, int64_t S) {
 constexpr int kCandPartSlots = 16;
 constexpr int64_t kCandSplitMaxB = 128;
 
-// Workgroups per query: ~2048 in all, at most one per 256 candidates (64 a wave).
-static int64_t cand_gx(int64_t B, int64_t P) {
+// Workgroups per query: ~2048 in all, at most one per 256 candidates (64 a wave), or per 64 where
+// the rows are wide: a wave then has only four or two of them in flight (one query, 200 rows of
+// 8 KB: 59, 27 us).
+static int64_t cand_gx(int64_t B, int64_t P, bool wide) {
   int64_t gx = cdiv(2048, B > 0 ? B : 1);
-  const int64_t by_rows = cdiv(P, kCandThreads);
+  const int64_t by_rows = cdiv(P, wide ? kWave : kCandThreads);
   gx = gx < by_rows ? gx : by_rows;
   gx = gx < 1 ? 1 : gx;
   return gx < kCandMaxWgsPerQuery ? gx : kCandMaxWgsPerQuery;
+}
+
+// Rows of more bytes have fewer than eight in flight a wave.
+constexpr int64_t kCandWideRow = 2048;
+
+static size_t cand_workspace(int64_t B, int64_t P, int64_t k, bool wide) {
+  const int64_t S = cand_gx(B, P, wide) * kCandWaves;
+  return align_up(static_cast<size_t>(B * S) * cand_capw(k, P, S) * sizeof(uint64_t), 256) +
+         align_up(static_cast<size_t>(B * S) * sizeof(int), 256) +
+         (B <= kCandSplitMaxB ? static_cast<size_t>(B) * kMergeParts * k * sizeof(uint64_t) : 0);
 }
 
 }  // namespace rt
@@ -345,10 +363,9 @@ using namespace rt;
 
 extern "C" size_t rt_cand_topk_workspace(int64_t B, int64_t P, int64_t k) {
   if (B <= 0 || P <= 0 || k <= 0) return 256;
-  const int64_t S = cand_gx(B, P) * kCandWaves;
-  return align_up(static_cast<size_t>(B * S) * cand_capw(k, P, S) * sizeof(uint64_t), 256) +
-         align_up(static_cast<size_t>(B * S) * sizeof(int), 256) +
-         (B <= kCandSplitMaxB ? static_cast<size_t>(B) * kMergeParts * k * sizeof(uint64_t) : 0);
+  const size_t narrow = cand_workspace(B, P, k, false);
+  const size_t wide = cand_workspace(B, P, k, true);
+  return narrow > wide ? narrow : wide;
 }
 
 namespace rt {
@@ -387,7 +404,7 @@ static int cand_topk(const void* queries, int64_t B, const void* items, int64_t 
     set_error("workspace too small: %zu < %zu", workspace_bytes, need);
     return kWorkspaceTooSmall;
   }
-  const int64_t gx = cand_gx(B, P);
+  const int64_t gx = cand_gx(B, P, rb > kCandWideRow);
   const int64_t S = gx * kCandWaves;
   const int capw = cand_capw(k, P, S);
   RT_CHECK_ARG(B <= 65535, "B must be <= 65535");

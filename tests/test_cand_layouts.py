@@ -112,3 +112,27 @@ def test_float(dev, dtype, d):
         bound = np.abs(iv[got]) @ np.abs(qv[r]) * d * 2.0**-24
         assert (np.abs(sc[r, at] - exact) <= bound).all()
         assert (np.diff(sc[r, at]) <= 0).all()
+
+
+@pytest.mark.parametrize("d", [64, 4096])
+@pytest.mark.parametrize("p", [1, 63, 65, 257, 1025])
+def test_shares(dev, d, p):
+    """Counts around a wave's 64 ids and the shares of one and of several rounds, narrow and wide
+    rows."""
+    import retrieve_amd.hip  # noqa: F401
+
+    g = rng(560 + d + p)
+    n, k = 1500, 20
+    counts = np.array([p, p - 1, p // 2, min(p, 64), min(p, 1), 0], np.int64)
+    b = len(counts)
+    items = g.integers(-9, 10, (n, d), dtype=np.int8)
+    q = g.integers(-9, 10, (b, d), dtype=np.int8)
+    cand = np.stack([g.permutation(n)[:p] for _ in range(b)]).astype(np.int64)
+    print(f"shares d={d} p={p}", flush=True)
+    ids, sc = torch.ops.retrieve_amd.int8_candidates_topk(_t(dev, q), _t(dev, items),
+                                                          _t(dev, cand), _t(dev, counts), k)
+    dots = q.astype(np.int64) @ items.astype(np.int64).T
+    want_ids, want_sc = _oracle(lambda r, c: dots[r, c], cand, counts, k, n,
+                                np.iinfo(np.int32).min)
+    assert np.array_equal(ids.cpu().numpy(), want_ids)
+    assert np.array_equal(sc.cpu().numpy(), want_sc)
