@@ -233,9 +233,25 @@ static int dispatch_ham(int64_t W, const ScanArgs& a, const PassPlan& p, int64_t
   return dispatch_ham_from<1>(W, a, p, nqg, seed, stream);
 }
 
+// Whether a table too small for a seed is spread over more workgroups than one a 1024 rows. Without
+// a bound a wave's list takes every row it meets: a wave of 256 rows sorts it again and again
+// (6 us a query of the wave up to k = 32, 12-21 from there), a spread table's lists never fill
+// and all its rows go to the merge (1.2 us a thousand). So it is spread where neither sorts (k
+// above 192), else where the queries that a wave scores outweigh the rows and the spread lists
+// sort little. 128-bit codes, not spread and spread: 100K rows at k = 10, one query 35, 142 us,
+// 32 queries 239, 175; 100K at k = 100, one query 132, 169, 8 queries 286, 174; 200K at k = 50, 24
+// queries 455, 307; 400K at k = 129, 16 queries 519, 732.
+static bool ham_spread(int64_t N, int64_t k, int qpw) {
+  if (k > 192) return true;
+  const int64_t rows = cdiv(N, main_workgroups() * kScanWaves);  // of a wave, spread
+  if (rows > (k <= 32 ? 64 : (k <= 128 ? 128 : 192))) return false;
+  const int64_t q = qpw;
+  return N <= (k <= 32 ? 4096 * q - 8192 : (k <= 96 ? 14336 * q - 16384 : 20480 * q - 8192));
+}
+
 static ScanPlan ham_plan(int64_t B, int64_t N, int64_t k, int qpw) {
   return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), ham_capw(k),
-                   kScanWaves * kHamTile, kHamTile, kSeedRows, false);
+                   kScanWaves * kHamTile, kHamTile, kSeedRows, false, ham_spread(N, k, qpw));
 }
 
 static int ham_qpw(int64_t B) { return static_cast<int>(B < kHamMaxQpw ? B : kHamMaxQpw); }

@@ -133,3 +133,19 @@ def test_candidate_workspaces_follow_the_candidates():
     # 80K candidates (or slots) of 16 queries at k = 1000
     assert lib.rt_cand_topk_workspace(16, 80_000, 1000) <= 24 << 20
     assert lib.rt_ivf_search_workspace(16, 80_000, 1000) <= 24 << 20
+
+
+def test_popcount_scan_is_spread_where_it_pays():
+    """A 1-bit scan of a table too small for a seed takes one workgroup a 1024 rows for one query
+    and a small k (98 workgroups of four lists for 100K rows), and more for a large batch or k."""
+    import torch  # noqa: F401
+
+    from retrieve_amd import _native
+
+    def need(b, n, k):
+        return _native.lib().rt_hamming_scan_topk_workspace(b, n, 2, k, 0)
+
+    assert need(1, 100_000, 10) <= 98 * 4 * 128 * 8 + (64 << 10)
+    assert need(4, 100_000, 10) <= 4 * need(1, 100_000, 10)
+    assert need(32, 100_000, 10) >= 32 * 390 * 4 * 64 * 8
+    assert need(1, 100_000, 1000) >= 390 * 4 * 64 * 8
