@@ -1,5 +1,6 @@
 // The exact top-k merge over the scan waves' lists, launch planning, and the library's error
 // store.
+#include <atomic>
 #include <cstdarg>
 #include <cstdlib>
 
@@ -77,14 +78,20 @@ static PassPlan plan_pass(int64_t n_rows, int64_t row_stride, int64_t n_qgroups,
   return p;
 }
 
+// (asked once per device: planning is done twice a call, for the workspace and for the launch)
 int64_t device_cus() {
+  constexpr int kDefault = 256;
+  constexpr int kDevices = 64;
+  static std::atomic<int> known[kDevices];
   int dev = 0;
-  int cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return kDefault;
+  int cus = dev < kDevices ? known[dev].load(std::memory_order_relaxed) : 0;
+  if (cus > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0) {
-    return 256;
+    return kDefault;
   }
+  if (dev < kDevices) known[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
 
