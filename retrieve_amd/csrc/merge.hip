@@ -104,36 +104,52 @@ int64_t main_workgroups() { return device_cus() * kMainWorkgroupsPerCU; }
 // 43 / 45 / 62 us (6K rows at B = 50: 35 us unseeded, 51 seeded, so no sample below
 // kSeedMinRows rows); 1M rows unseeded 152 / 1216 / 4811 us, seeded 73 / 89 / 169; exact fp32
 // 100K rows at B = 1024 2230 us unseeded, 302 seeded.
-static int64_t small_seed_rows(int64_t N, int64_t k, int64_t rows_per_wg, int64_t lpq) {
+//
+// Where the fallback needs the lists' k-th best (seed.rows_least), there are 1.5 k lists at least:
+// without that bound a table whose sampled rows are better than the rest (one row block in 16,
+// say) is scanned a second time from nothing and all its rows merged by one workgroup a query
+// (int8 D = 128, one query: 300K rows at k = 100 379 us, 1M at k = 1000 1824; 60 and 118 behind
+// it; without a sample 84 and 360). *rows_per_wg is halved down to rows_least while the lists are
+// fewer than 2 k.
+static int64_t small_seed_rows(int64_t N, int64_t k, const SeedSpec& seed, int64_t lpq,
+                               int64_t* rows_per_wg) {
   for (const int64_t stride : {16, 8, 4}) {
     const int64_t rows = N / stride / kSeedBlock * kSeedBlock;
     if (rows < kSeedMinRows) continue;
-    if (rows / rows_per_wg * lpq * 4 >= 5 * sample_rank(k, N / rows)) return rows;
+    int64_t wg = seed.rows_per_wg;
+    while (seed.rows_least > 0 && wg > seed.rows_least && rows / wg * lpq < 2 * k) wg /= 2;
+    const int64_t lists = rows / wg * lpq;
+    if (lists * 4 < 5 * sample_rank(k, N / rows)) continue;
+    if (seed.rows_least > 0 && lists * 2 < 3 * k) continue;
+    *rows_per_wg = wg;
+    return rows;
   }
   return 0;
 }
 
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
-                   int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t list_tile, int64_t seed_rows_min, bool ranked, bool spread) {
+                   int64_t target_wgs, int main_capw, int64_t list_tile, const SeedSpec& seed,
+                   bool spread) {
   ScanPlan s;
   s.qpg = qpg;
   s.n_qgroups = cdiv(B, qpg);
   // a query's lists per workgroup: every wave scores all of the row's queries (lists_per_wg ==
   // waves * qpg), or one wave owns each query (lists_per_wg == qpg)
   const int64_t lpq = lists_per_wg / qpg;
-  int64_t seed_rows = seed_rows_min > kSeedRowsPerK * k ? seed_rows_min : kSeedRowsPerK * k;
+  int64_t seed_rows = seed.rows > kSeedRowsPerK * k ? seed.rows : kSeedRowsPerK * k;
+  int64_t rows_per_wg = seed.rows_per_wg;
   s.seeded = N >= 8 * seed_rows;
-  if (!s.seeded && ranked) {
-    seed_rows = small_seed_rows(N, k, seed_rows_per_wg, lpq);
-    s.seeded = seed_rows > 0;
+  if (!s.seeded && seed.ranked) {
+    seed_rows = small_seed_rows(N, k, seed, lpq, &rows_per_wg);
+    s.sparse = seed_rows > 0;
+    s.seeded = s.sparse;
   }
   if (s.seeded) {
     // one-entry lists (each seed wave's best); at least 2k of them per query (their k-th is the
     // safe bound, their rank-th the speculative one; 4k cost configuration 5's step 1.5 % in
     // seed workgroups, each loading the group's queries)
-    s.seed = plan_pass(seed_rows, N / seed_rows, s.n_qgroups, seed_rows_per_wg, 1, lists_per_wg,
-                       lpq, kTargetWorkgroups, cdiv(2 * k, lpq));
+    s.seed = plan_pass(seed_rows, N / seed_rows, s.n_qgroups, rows_per_wg, 1, lists_per_wg, lpq,
+                       kTargetWorkgroups, cdiv(2 * k, lpq));
   }
   // A small table is spread over as many workgroups as its rows allow: behind a bound its lists
   // stay short, and without one they hold every row they meet, so few rows a list end in the
@@ -149,7 +165,9 @@ ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_p
   s.off_lists = 0;
   s.off_counts = align_up(lists, 256);
   s.off_tau = s.off_counts + align_up(counts, 256);
-  s.off_flag = s.off_tau + align_up(static_cast<size_t>(B) * sizeof(uint64_t), 256);
+  s.off_safe = s.off_tau + align_up(static_cast<size_t>(B) * sizeof(uint64_t), 256);
+  s.off_flag =
+      s.off_safe + (s.sparse ? align_up(static_cast<size_t>(B) * sizeof(uint64_t), 256) : 0);
   s.off_parts = s.off_flag + 256;
   s.split = B <= kMergeSplitMaxB;
   s.total = s.off_parts +

@@ -128,11 +128,12 @@ struct BitsQueries {
 
 // Seed pass over the strided sample: per query, each wave's best composite over its rows,
 // written to a.lists[q * S + wave index] (S = waves of the grid row). The sample is cut into
-// chunks of kTileRows rows from row 0 (a sample block of kSeedBlock consecutive items holds
-// whole chunks); a workgroup's waves take the parts of the chunks within its strip (a multiple
-// of 16 rows from a multiple of 16) in turn, every load of a part issued before its sums. With
-// strips of 512 rows: 1024 lists a query from the default 2^17 sampled rows, few to merge, and
-// far more than the rank whose best the merge takes.
+// chunks of kTileRows rows from row 0, or of 64, 32 or 16 where a strip holds fewer than a chunk a
+// wave (a sample block of kSeedBlock consecutive items holds whole chunks); a workgroup's waves
+// take the parts of the chunks within its strip (a multiple of 16 rows from a multiple of 16) in
+// turn, every load of a part issued before its sums. With strips of 512 rows: 1024 lists a query
+// from the default 2^17 sampled rows, few to merge, and far more than the rank whose best the
+// merge takes.
 template <int NQ>
 __global__ void __launch_bounds__(kScanThreads) bits_seed_kernel(ScanArgs a) {
   constexpr int QPW = 16 * NQ;
@@ -150,10 +151,12 @@ __global__ void __launch_bounds__(kScanThreads) bits_seed_kernel(ScanArgs a) {
   uint64_t best[NQ];
 #pragma unroll
   for (int j = 0; j < NQ; ++j) best[j] = 0ull;
-  const int64_t c1 = s1 > s0 ? (s1 - 1) / kTileRows : -1;  // the strip's last chunk
-  for (int64_t c = s0 / kTileRows + wave; c <= c1; c += kScanWaves) {
-    const int64_t r0 = c * kTileRows > s0 ? c * kTileRows : s0;
-    const int64_t r1 = c * kTileRows + kTileRows < s1 ? c * kTileRows + kTileRows : s1;
+  int chunk = kTileRows;
+  while (chunk > kGroupRows && chunk * kScanWaves > a.strip) chunk /= 2;
+  const int64_t c1 = s1 > s0 ? (s1 - 1) / chunk : -1;  // the strip's last chunk
+  for (int64_t c = s0 / chunk + wave; c <= c1; c += kScanWaves) {
+    const int64_t r0 = c * chunk > s0 ? c * chunk : s0;
+    const int64_t r1 = c * chunk + chunk < s1 ? c * chunk + chunk : s1;
     // the part's rows are consecutive items from sample_item(r0): one descriptor, rows past
     // r1 read as zeros and are never kept
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -401,8 +404,8 @@ ScanPlan bits_plan(int64_t B, int64_t N, int64_t k) {
   // (the 64-row-tile form: three workgroups a CU, its occupancy)
   const int64_t target = bits_small_tiles(nq, bits_capw(k)) ? main_workgroups() * kWavesSmall / 2
                                                             : main_workgroups();
-  return plan_scan(B, N, k, qpg, kScanWaves * qpg, target, bits_capw(k), kScanWaves * kTileRows,
-                   kTileRows, kSeedRows / 2);
+  const SeedSpec seed{kScanWaves * kTileRows, kSeedRows / 2, true, kScanWaves * kGroupRows};
+  return plan_scan(B, N, k, qpg, kScanWaves * qpg, target, bits_capw(k), kTileRows, seed);
 }
 
 template <int NQ, int TG>
@@ -453,8 +456,9 @@ size_t bits_mfma_workspace(int64_t B, int64_t N, int64_t k) {
 // the flag is set), on `stream`, no host sync. The seed's bound is its sample's rank-th best
 // (sample_rank), not its k-th: the main pass then keeps about rank * stride candidates a query
 // instead of k * stride. A query that ends with fewer than k entries behind a bound above 0
-// raises the flag, and the fallback main pass and merge without the bound (both returning at
-// once while the flag is clear) keep the results exact.
+// raises the flag, and the fallback main pass and merge (both returning at once while the flag is
+// clear) keep the results exact: behind the k-th best of a sparse sample's lists, else without a
+// bound.
 int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, int64_t N,
               int64_t k, const uint64_t* mask, int64_t mask_words, int64_t* out_ids,
               void* out_scores, int score_kind, void* workspace, size_t workspace_bytes,
@@ -474,9 +478,11 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
   uint64_t* lists = reinterpret_cast<uint64_t*>(ws + plan.off_lists);
   int* counts = reinterpret_cast<int*>(ws + plan.off_counts);
   uint64_t* tau = reinterpret_cast<uint64_t*>(ws + plan.off_tau);
+  uint64_t* safe_tau = reinterpret_cast<uint64_t*>(ws + plan.off_safe);
   uint32_t* spec_flag = reinterpret_cast<uint32_t*>(ws + plan.off_flag);
   const int rank = plan.seeded ? sample_rank(k, plan.seed.row_stride) : static_cast<int>(k);
   const bool speculative = plan.seeded && rank < k;
+  const bool safe = plan.sparse && rank < k;
 
   ScanArgs a{};
   a.queries = query_bits;
@@ -507,13 +513,20 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
     m.capw = 1;
     m.flat = true;  // one entry per seed wave, contiguous per query
     m.S = plan.seed.S;
-    m.tau_out = tau;
-    m.k = rank;
+    if (safe) {
+      m.tau_out = safe_tau;
+      m.tau2_out = tau;
+      m.k2 = rank;
+    } else {
+      m.tau_out = tau;
+      m.k = rank;
+    }
     m.spec_flag = speculative ? spec_flag : nullptr;  // (cleared)
     st = launch_merge(m, stream);
     if (st != kOk) return st;
     m.k = static_cast<int>(k);
     m.tau_out = nullptr;
+    m.tau2_out = nullptr;
     m.flat = false;
     m.spec_flag = nullptr;
   }
@@ -538,11 +551,11 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
   if (speculative) {
     m.spec_flag = spec_flag;
     m.spec_tau = tau;
-    m.safe_tau = nullptr;
+    m.safe_tau = safe ? safe_tau : nullptr;
   }
   st = launch_merge(m, stream);
   if (st != kOk || !speculative) return st;
-  a.tau_in = nullptr;
+  a.tau_in = safe ? safe_tau : nullptr;
   a.run_if = spec_flag;
   st = dispatch_bits(nq, a, plan.main, plan.n_qgroups, false, stream);
   if (st != kOk) return st;

@@ -1080,7 +1080,7 @@ static ScanPlan blk_plan(int64_t B, int64_t N, int64_t k, int64_t row_bytes, boo
   const int64_t qpg = halves == 8 ? kBlkQpg / 4 : (halves == 4 ? kBlkQpg / 2 : kBlkQpg);
   const int rows = blk_rows(row_bytes, wide, bits);
   ScanPlan p = plan_scan(B, N, k, qpg, halves * qpg, device_cus() * (wide ? 1 : 2),
-                         blk_capw(k, rows), kBlkRows, rows / halves);
+                         blk_capw(k, rows), rows / halves, SeedSpec{kBlkRows});
   if (off_spec != nullptr) *off_spec = align_up(p.total, 256);
   p.total = align_up(p.total, 256) + align_up(static_cast<size_t>(B) * sizeof(uint64_t), 256) +
             256;

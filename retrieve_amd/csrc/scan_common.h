@@ -142,10 +142,12 @@ struct ScanPlan {
   int64_t qpg = 16;        // queries per workgroup row (grid.y groups)
   int64_t n_qgroups = 0;
   bool seeded = false;
+  bool sparse = false;     // seeded by a sparse sample of a small table
   PassPlan seed;
   PassPlan main;
   // workspace layout (byte offsets)
-  size_t off_lists = 0, off_counts = 0, off_tau = 0, off_flag = 0, off_parts = 0, total = 0;
+  size_t off_lists = 0, off_counts = 0, off_tau = 0, off_safe = 0, off_flag = 0, off_parts = 0,
+         total = 0;
   bool split = false;  // room for a split merge at off_parts
 };
 
@@ -187,17 +189,23 @@ int blocked_hamming(const uint64_t* query_bits, int64_t B, const uint64_t* item_
 // Sizes the passes for B queries over N rows and top-k. A workgroup row (grid.y) covers qpg
 // queries and each workgroup keeps lists_per_wg candidate lists (in the main pass of main_capw
 // entries, or the rows a list can meet where those are fewer: list_tile rows a tile); the main
-// pass runs target_wgs workgroups in all; a seed workgroup scores at least seed_rows_per_wg
-// sampled rows.
-// Rows of the seed sample (at least, and kSeedRowsPerK * k at least): the main pass then keeps
-// about k * N / seed rows composites a query (in expectation, for items in random order).
-// `ranked`: the scan bounds its candidates by the sample's rank-th best (sample_rank) with a
-// fallback, so a sparse sample of a small table serves it too. `spread`: a small table may be
-// spread over more workgroups, and so more lists, than one a 1024 rows.
+// pass runs target_wgs workgroups in all. `spread`: a small table may be spread over more
+// workgroups, and so more lists, than one a 1024 rows.
 constexpr int64_t kSeedRows = 1 << 18;
+struct SeedSpec {
+  int64_t rows_per_wg;  // sampled rows a seed workgroup scores at least
+  // Rows of the sample (at least, and kSeedRowsPerK * k at least): the main pass then keeps
+  // about k * N / rows composites a query (in expectation, for items in random order).
+  int64_t rows = kSeedRows;
+  // The scan bounds its candidates by the sample's rank-th best (sample_rank) with a fallback, so
+  // a sparse sample of a small table serves it too.
+  bool ranked = true;
+  // Not 0: rows a workgroup of a sparse sample may be cut to, so that the k-th best of the
+  // sample's lists exists; the fallback then runs behind it.
+  int64_t rows_least = 0;
+};
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
-                   int64_t target_wgs, int main_capw, int64_t seed_rows_per_wg,
-                   int64_t list_tile, int64_t seed_rows_min = kSeedRows, bool ranked = true,
+                   int64_t target_wgs, int main_capw, int64_t list_tile, const SeedSpec& seed,
                    bool spread = true);
 
 // Writes the -1 / sentinel pads of an empty result.

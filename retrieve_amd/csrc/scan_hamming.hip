@@ -250,8 +250,9 @@ static bool ham_spread(int64_t N, int64_t k, int qpw) {
 }
 
 static ScanPlan ham_plan(int64_t B, int64_t N, int64_t k, int qpw) {
-  return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), ham_capw(k),
-                   kScanWaves * kHamTile, kHamTile, kSeedRows, false, ham_spread(N, k, qpw));
+  const SeedSpec seed{kScanWaves * kHamTile, kSeedRows, false};
+  return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), ham_capw(k), kHamTile, seed,
+                   ham_spread(N, k, qpw));
 }
 
 static int ham_qpw(int64_t B) { return static_cast<int>(B < kHamMaxQpw ? B : kHamMaxQpw); }

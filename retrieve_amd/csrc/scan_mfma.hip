@@ -547,9 +547,10 @@ constexpr int kSeedTiles = 4;
 // over more workgroups, its lists not cut.
 static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, bool fixed = false) {
   const int64_t qpw = fixed ? 16 : 16 * mfma_groups(B);
+  const SeedSpec seed{kScanWaves * kTile * kSeedTiles, mfma_seed_rows(B, N), !fixed,
+                      kScanWaves * kTile};
   return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), mfma_capw(k),
-                   kScanWaves * kTile * kSeedTiles, fixed ? 0 : kTile, mfma_seed_rows(B, N),
-                   !fixed, !fixed);
+                   fixed ? 0 : kTile, seed, !fixed);
 }
 
 // seed scan → seed threshold merge → main scan → final merge, on `stream`, no host sync
@@ -582,6 +583,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   uint64_t* lists = reinterpret_cast<uint64_t*>(ws + plan.off_lists);
   int* counts = reinterpret_cast<int*>(ws + plan.off_counts);
   uint64_t* tau = reinterpret_cast<uint64_t*>(ws + plan.off_tau);
+  uint64_t* safe_tau = reinterpret_cast<uint64_t*>(ws + plan.off_safe);
   uint32_t* spec_flag = reinterpret_cast<uint32_t*>(ws + plan.off_flag);
   // The seed's bound is its sample's rank-th best (sample_rank: k -> about 13 at k = 100 and one
   // row in 57 sampled), not its k-th: the main pass then keeps about rank * stride candidates a
@@ -589,10 +591,12 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   // exact clauses alone (a sampled item that passes them is not probed), which bounds the
   // filter's k-th best only where the plans pass every item the clauses pass. A query that
   // ends with fewer than k entries behind a bound above 0 raises a flag, and a fallback main
-  // pass and merge without the bound (both returning at once while the flag is clear) keep the
-  // results exact.
+  // pass and merge (both returning at once while the flag is clear) keep the results exact: behind
+  // the k-th best of a sparse sample's lists, a bound of what the seed tests (not of the probe), else
+  // without a bound.
   const int rank = plan.seeded ? sample_rank(k, plan.seed.row_stride) : static_cast<int>(k);
   const bool speculative = plan.seeded && (rank < k || probe.doc_bits != nullptr);
+  const bool safe = plan.sparse && rank < k && probe.doc_bits == nullptr;
 
   ScanArgs a{};
   a.queries = queries;
@@ -624,13 +628,20 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
     m.capw = 1;
     m.flat = true;  // one entry per seed wave, contiguous per query
     m.S = plan.seed.S;
-    m.tau_out = tau;
-    m.k = rank;
+    if (safe) {
+      m.tau_out = safe_tau;
+      m.tau2_out = tau;
+      m.k2 = rank;
+    } else {
+      m.tau_out = tau;
+      m.k = rank;
+    }
     m.spec_flag = speculative ? spec_flag : nullptr;  // (cleared)
     st = launch_merge(m, stream);
     if (st != kOk) return st;
     m.k = static_cast<int>(k);
     m.tau_out = nullptr;
+    m.tau2_out = nullptr;
     m.flat = false;
     m.spec_flag = nullptr;
   }
@@ -657,11 +668,11 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   if (speculative) {
     m.spec_flag = spec_flag;
     m.spec_tau = tau;
-    m.safe_tau = nullptr;
+    m.safe_tau = safe ? safe_tau : nullptr;
   }
   st = launch_merge(m, stream);
   if (st != kOk || !speculative) return st;
-  a.tau_in = nullptr;
+  a.tau_in = safe ? safe_tau : nullptr;
   a.run_if = spec_flag;
   st = dispatch_mfma<Op>(row_bytes, a, plan.main, plan.n_qgroups, false, stream);
   if (st != kOk) return st;

@@ -141,3 +141,49 @@ def test_clauses(dev, b):
     want_ids, want_sc = _want(q, items, k, valid)
     assert np.array_equal(ids.cpu().numpy(), want_ids)
     assert np.array_equal(sc.cpu().numpy(), want_sc)
+
+
+def _sampled(n, stride):
+    rows = n // stride // SEED_BLOCK * SEED_BLOCK
+    r = np.arange(rows)
+    return r // SEED_BLOCK * SEED_BLOCK * (n // rows) + r % SEED_BLOCK
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("n,stride,k", [(70_001, 16, 10), (70_001, 16, 100), (110_001, 4, 1000),
+                                        (200_003, 8, 1000)])
+@pytest.mark.parametrize("b", [1, 20])
+def test_fallback_behind_the_kth(dev, b, n, stride, k, masked):
+    """Sampled rows better than the rest, per-wave scans: the fallback runs behind the k-th best of
+    the sample's lists."""
+    import retrieve_amd.hip  # noqa: F401
+
+    print(f"fallback int8 n={n} b={b} k={k} masked={masked}", flush=True)
+    g = rng(n + b + k)
+    items = g.integers(-20, 21, (n, 64), dtype=np.int8)
+    items[_sampled(n, stride)] *= 2
+    q = g.integers(-20, 21, (b, 64), dtype=np.int8)
+    valid = g.random((b, n)) < 0.5 if masked else None
+    ids, sc = torch.ops.retrieve_amd.int8_scan_topk(
+        _t(dev, q), _t(dev, items), k, None if valid is None else _t(dev, _pack(valid)))
+    want_ids, want_sc = _want(q, items, k, valid)
+    assert np.array_equal(ids.cpu().numpy(), want_ids)
+    assert np.array_equal(sc.cpu().numpy(), want_sc)
+
+
+@pytest.mark.parametrize("n,stride,k", [(17_000, 4, 20), (70_001, 16, 100), (110_001, 4, 1000)])
+@pytest.mark.parametrize("b", [1, 40, 100])
+def test_fallback_behind_the_kth_bits(dev, b, n, stride, k):
+    """The same over 512-bit codes: half of a sampled row's words are some query's."""
+    import retrieve_amd.hip  # noqa: F401
+
+    print(f"fallback bits n={n} b={b} k={k}", flush=True)
+    g = rng(n + b + k)
+    items = g.integers(-2**63, 2**63 - 1, (n, 8), dtype=np.int64)
+    q = g.integers(-2**63, 2**63 - 1, (b, 8), dtype=np.int64)
+    at = _sampled(n, stride)
+    items[at, :4] = q[g.integers(0, b, at.size), :4]
+    ids, sc = torch.ops.retrieve_amd.hamming_scan_topk(_t(dev, q), _t(dev, items), k)
+    want_ids, want_sc = osc.hamming_topk(q, items, k)
+    assert np.array_equal(ids.cpu().numpy(), want_ids)
+    assert np.array_equal(sc.cpu().numpy(), want_sc)
