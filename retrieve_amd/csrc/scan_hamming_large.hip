@@ -16,8 +16,8 @@
 //   4. emit pass: the same ranges scored again; an item with h <= h* goes to its popcount's
 //      start plus its range's running sum plus an LDS counter. Ties at h* are emitted by the
 //      ranges up to the one where they reach kk, whose ties may run past it;
-//   5. rank: entries of one popcount and range lie together in no order; each finds its place
-//      among them by id and is written there if that is below kk.
+//   5. rank: entries of one popcount and range (a cell) lie together in no order; each finds its
+//      place among them by id and is written there if that is below kk.
 // Two passes over the codes, whose bound is the popcounts (2 W XOR and 2 W bit counts an item
 // and query) and the mask bits. Counting into one histogram a query and appending through one
 // counter a query (same-address atomics, a third pass for the ties and two block sorts) took
@@ -35,9 +35,11 @@ constexpr int kLkTiles = 2;         // 64-item tiles a wave scores together
 constexpr int64_t kLkMaxRows = 8192;  // items of a range at most (its ties may overrun k)
 constexpr int64_t kLkMinRows = 1024;  // and at least, where the table allows
 constexpr int64_t kLkTargetWgs = 2048;
+constexpr int kLkRankWalk = 64;     // entries of a cell that each of them walks
 constexpr int kLkPrefixThreads = 1024;
 constexpr int kLkPrefixSegs = kLkPrefixThreads / kWave;
-// Counts and entries of the queries taken at a time (the others follow on the same workspace).
+// Counts and entries of the queries taken at a time (the others follow on the same workspace), or
+// those of eight queries where they are more: at most 3.2 % of the codes' bytes and 1 MiB.
 constexpr size_t kLkMaxBytes = size_t{256} << 20;
 
 typedef __attribute__((address_space(4))) const uint32_t ku32;
@@ -260,12 +262,27 @@ __global__ void __launch_bounds__(kWave) lk_cut_kernel(LkArgs a) {
   }
 }
 
-// An entry's place: its cell (entries of one popcount and range) starts where the entries to its
-// left stop being of the cell, and it follows those of the cell that have lower ids.
+// An entry's place: its cell (entries of one popcount and range, which lie together in no order)
+// starts at the sums that the emit pass started from, and it follows those of the cell that have
+// lower ids. A cell of few entries is walked by each of them (random codes: one or two entries).
+// Tables of many equal codes have cells of up to kLkMaxRows, where the walks are quadratic: those
+// are ranked by a bitmap of the range's ids in LDS, one cell of the block's entries after another
+// (at most five a block). 3M 128-bit codes, 16 queries at k = 5000, the whole call: all codes equal
+// 875 us walked, 235 now (163 of it the count pass' same-address adds, 14 this kernel); random
+// codes 97, 94.
 __global__ void __launch_bounds__(kLkThreads) lk_rank_kernel(LkArgs a, int64_t* out_ids,
                                                              void* out_scores, int score_kind) {
+  __shared__ uint32_t bits[kLkThreads];    // the cell's ids, a bit an item of the range
+  __shared__ int before[kLkThreads];       // ids of the cell in the words before
+  __shared__ int first[kLkWaves];
+  __shared__ int part[kLkWaves];
+  __shared__ int cell_at[3];               // the cell's first entry, its end, its range
+  static_assert(kLkMaxRows == 32 * kLkThreads, "a thread a word of the bitmap");
+  const int tid = threadIdx.x;
+  const int lane = lane_id();
+  const int wave = tid >> 6;
   const int64_t q = blockIdx.y;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kLkThreads + threadIdx.x;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kLkThreads + tid;
   const int kk = a.cut[q * 4 + 1];
   const int n = a.cut[q * 4 + 2];
   auto put = [&](int64_t at, int64_t id, int32_t score, bool pad) {
@@ -278,26 +295,75 @@ __global__ void __launch_bounds__(kLkThreads) lk_rank_kernel(LkArgs a, int64_t* 
     }
   };
   if (i >= kk && i < a.k) put(i, -1, 0, true);
-  if (i >= n) return;
+  if (i - tid >= n) return;  // (the whole block)
+  const bool have = i < n;
   const uint64_t* e = a.buf + q * a.cap;
-  const uint64_t c = e[i];
+  const uint64_t c = have ? e[i] : 0ull;
   const uint32_t rows = static_cast<uint32_t>(a.rows);
-  const uint32_t cell = composite_item(c) / rows;
-  auto same = [&](uint64_t x) {
-    return composite_key(x) == composite_key(c) && composite_item(x) / rows == cell;
-  };
-  int64_t at = i;
-  for (int64_t j = i - 1; j >= 0; --j) {
-    const uint64_t x = e[j];
-    if (!same(x)) break;
-    at -= x < c ? 1 : 0;  // (smaller composite: higher id)
+  const uint32_t id = have ? composite_item(c) : 0u;
+  const int cell = static_cast<int>(id / rows);
+  const int32_t score = have ? i32_of_key(composite_key(c)) : 0;
+  int s0 = 0;
+  int s1 = 0;
+  if (have) {
+    const int h = (a.nb - 1 - score) / 2;
+    const uint32_t* starts = a.totals + q * a.nbp + h;
+    const uint16_t* sums = a.counts + (q * a.gx + cell) * a.nbp + h;
+    s0 = static_cast<int>(starts[0] + sums[0]);
+    // (saturated sums and starts lie past n)
+    const uint32_t end = cell + 1 < a.gx ? starts[0] + sums[a.nbp]
+                                         : (h + 1 < a.nb ? starts[1] : 0x7fffffffu);
+    s1 = end < static_cast<uint32_t>(n) ? static_cast<int>(end) : n;
   }
-  for (int64_t j = i + 1; j < n; ++j) {
-    const uint64_t x = e[j];
-    if (!same(x)) break;
-    at += x > c ? 1 : 0;
+  int at = s0;
+  bool pending = s1 - s0 > kLkRankWalk;
+  if (!pending) {
+    for (int j = s0; j < s1; ++j) at += e[j] > c ? 1 : 0;  // (greater composite: lower id)
   }
-  if (at < kk) put(at, composite_item(c), i32_of_key(composite_key(c)), false);
+  while (true) {
+    // the first entry that is not placed yet names the cell
+    const uint64_t bal = __ballot(pending);
+    if (lane == 0) first[wave] = bal != 0ull ? tid + __builtin_ctzll(bal) : kLkThreads;
+    __syncthreads();
+    int f = kLkThreads;
+#pragma unroll
+    for (int w = 0; w < kLkWaves; ++w) f = first[w] < f ? first[w] : f;
+    if (f == kLkThreads) break;  // (the whole block)
+    if (tid == f) {
+      cell_at[0] = s0;
+      cell_at[1] = s1;
+      cell_at[2] = cell;
+    }
+    bits[tid] = 0u;
+    __syncthreads();
+    const uint32_t id0 = static_cast<uint32_t>(cell_at[2]) * rows;
+    for (int j = cell_at[0] + tid; j < cell_at[1]; j += kLkThreads) {
+      const uint32_t off = composite_item(e[j]) - id0;
+      atomicOr(&bits[off >> 5], 1u << (off & 31u));
+    }
+    __syncthreads();
+    const int own = __builtin_popcount(bits[tid]);
+    int incl = own;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int y = __shfl_up(incl, off);
+      incl += lane >= off ? y : 0;
+    }
+    if (lane == kWave - 1) part[wave] = incl;
+    __syncthreads();
+    int base = incl - own;
+    for (int w = 0; w < wave; ++w) base += part[w];
+    before[tid] = base;
+    __syncthreads();
+    if (pending && s0 == cell_at[0]) {
+      const uint32_t off = id - id0;
+      at = s0 + before[off >> 5] +
+           __builtin_popcount(bits[off >> 5] & ((1u << (off & 31u)) - 1u));
+      pending = false;
+    }
+    __syncthreads();  // (read before the next cell's replace them)
+  }
+  if (have && at < kk) put(at, id, score, false);
 }
 
 struct LkPlan {

@@ -81,3 +81,49 @@ def test_float_scores(dev, k):
                                                               k, bits)
     assert sc.dtype == torch.float32 and torch.equal(ids, want_ids)
     assert torch.equal(sc, torch.where(want_ids >= 0, want.float(), float("-inf")))
+
+
+@pytest.mark.parametrize("b,n,k", [(1, 5000, 3000), (9, 20_011, 8192), (2048, 73_728, 8192)])
+def test_cells(dev, b, n, k):
+    """Runs of one popcount as long as the cells that their entries walk (64), one longer, and
+    whole ranges (up to 8192 items: the last shape's), cut by the end of k."""
+    import retrieve_amd.hip  # noqa: F401
+
+    runs = [64, 65, 1, 63, 128, 700, 2]
+    pop = np.resize(np.repeat(np.arange(len(runs)), runs), n)
+    pop[n // 2 :] = 7  # one popcount from here on
+    items = np.zeros((n, 2), np.int64)
+    items[:, 1] = (1 << (3 * pop + 1)) - 1
+    q = np.zeros((b, 2), np.int64)
+    print(f"large k cells b={b} n={n} k={k}", flush=True)
+    ids, sc = torch.ops.retrieve_amd.hamming_scan_topk(_t(dev, q), _t(dev, items), k)
+    h = 3 * pop + 1
+    want = np.argsort(h, kind="stable")[:k]
+    assert (ids == _t(dev, want)[None]).all()
+    assert (sc == _t(dev, (128 - 2 * h[want]).astype(np.int32))[None]).all()
+
+
+def test_equal_codes_cost(dev):
+    """A table of one code is one cell a range, which costs no more than a few times what random
+    codes do. (Each of 8192 entries walking 8192 took 26 times as long, 11.7 ms; the bitmap 3.2
+    times, for the passes' same-address adds.)"""
+    import retrieve_amd.hip  # noqa: F401
+
+    g = rng(83)
+    n, b, k = 1_000_000, 256, 8192
+    q = _t(dev, g.integers(-2**63, 2**63 - 1, (b, 2), dtype=np.int64))
+    items = _t(dev, g.integers(-2**63, 2**63 - 1, (n, 2), dtype=np.int64))
+    print("large k cost of equal codes", flush=True)
+
+    def took(codes):
+        times = []
+        for _ in range(6):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            torch.ops.retrieve_amd.hamming_scan_topk(q, codes, k)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    assert took(items[:1].expand(n, 2).contiguous()) < 10 * took(items)
