@@ -535,8 +535,7 @@ __device__ inline void load_clauses(const IvfArgs& a, int64_t b, IvfClauses* cl)
   const uint64_t active = __ballot(v != -1);
   if (v != -1) {
     const int i = __popcll(active & ((1ull << tid) - 1ull));
-    // (values below -1 stand for "no doc holds it")
-    cl->value[i] = v < -1 ? INT32_MIN : v;
+    cl->value[i] = v;
     cl->reverse[i] = a.reverse[tid] != 0;
     const int64_t r0 = a.cslots[tid];
     const int64_t r1 = a.cslots[tid + 1];

@@ -1371,10 +1371,13 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
         # (a bool flag is its 0 / 1 byte: a view, not a copy kernel a call)
         rev = rev.view(torch.int8) if rev.dtype == torch.bool else rev.to(torch.int8)
 
-        def clamped():  # values no doc may hold (outside [-1, 2^31 - 1]) as INT32_MIN
-            v = query_clause_attrs.to(torch.int64)
-            v = torch.where((v >= -1) & (v <= 2**31 - 1), v, -(2**31)).to(torch.int32)
-            return v.contiguous()
+        # values no doc may hold (outside [-1, 2^31 - 1]) as INT32_MIN; int32 ones in one kernel
+        if query_clause_attrs.dtype == torch.int32:
+            qv = torch.nn.functional.threshold(query_clause_attrs.contiguous(), -2, -(2**31))
+        else:
+            qv = query_clause_attrs.to(torch.int64)
+            qv = torch.where((qv >= -1) & (qv <= 2**31 - 1), qv, -(2**31)).to(torch.int32)
+            qv = qv.contiguous()
     full = (divisor_for_int8 == -1 and offs.numel() == 1 and probes.shape[1] == 1
             and width >= n and d in _FULL_SCAN_D
             and _one_list_is_the_table(cluster_offsets, cluster_sizes, n))
@@ -1388,9 +1391,6 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
                                      max_stack_size, bloom_k, hash_k, query_plan_index, probes,
                                      offs, sizes)
         if partial is not None or plans is None:
-            if exact:  # (the scan itself takes int32 values below -1 for INT32_MIN)
-                qv = query_clause_attrs.contiguous() \
-                    if query_clause_attrs.dtype == torch.int32 else clamped()
             cum, first, words = partial if partial is not None else (None, None, None)
             ws = nat.workspace(lib.rt_ivf_search_workspace(b, width, k), dev)
             with torch.cuda.device(dev):
@@ -1418,7 +1418,6 @@ def _st_search(query, probe_ids, cluster_offsets, cluster_sizes, item_codes, sor
         mask = bm[query_plan_index.to(torch.int64)] if query_plan_index is not None else bm[:b]
         mask = mask.contiguous()
     if exact:
-        qv = clamped()
         out = torch.empty((b, (n + 63) // 64), dtype=torch.int64, device=dev)
         with torch.cuda.device(dev):
             st = lib.rt_clause_slots_filter(

@@ -142,3 +142,44 @@ def test_probe_past_the_sizes(dev, end):
         want = ost.search(q, probes, offsets, sizes, items, perm, [0.3], k, n, valid=valid)
         assert np.array_equal(ids.cpu().numpy(), want[0])
         assert np.array_equal(sc.cpu().numpy(), want[1])
+
+
+def test_values_below_minus_one(dev):
+    """The C entry compares clause values as they are (only -1 is inactive): a query value below -1
+    finds the docs that hold it; torch.ops.st.search takes such values for ones that none holds."""
+    import retrieve_amd.st as st
+    from retrieve_amd import _native as nat
+
+    g = rng(350)
+    n, d, b, k, lists = 3000, 64, 3, 30, 10
+    items, offsets, sizes, perm = _ivf(g, n, d, lists)
+    q = g.standard_normal((b, d)).astype(np.float32)
+    probes = np.stack([g.permutation(lists)[:6] for _ in range(b)]).astype(np.int64)
+    vals = g.choice(np.array([-(2**31), -7, -2, 0, 3], np.int32), n)
+    qa = np.array([[-7], [-2], [-(2**31)]], np.int32)
+    rev = np.zeros(1, bool)
+    cs = np.array([0, 1], np.int64)
+    t = [_t(dev, x) for x in (q, items, probes, offsets, sizes, perm, vals[None], cs,
+                              rev.astype(np.int8), qa, np.float32([0.3]))]
+    tq, ti, tp, to, ts, tperm, tv, tcs, trev, tqa, tgs = t
+    codes, scales = st.quantize_rows(tq)
+    ids = torch.empty((b, k), dtype=torch.int64, device=dev)
+    sc = torch.empty((b, k), dtype=torch.float32, device=dev)
+    lib = nat.lib()
+    width = (n + 31) // 32 * 32
+    ws = nat.workspace(lib.rt_ivf_search_workspace(b, width, k), dev)
+    print("clause values below -1 through the C entry", flush=True)
+    nat.check(lib.rt_ivf_search_payload_filters(
+        nat.ptr(codes), nat.ptr(scales), b, nat.ptr(ti), n, d, nat.ptr(tp), 6, nat.ptr(to),
+        nat.ptr(ts), lists, width, None, None, None, 0, 0, nat.ptr(tv), 1, nat.ptr(tcs), 1,
+        nat.ptr(trev), nat.ptr(tqa), -1, nat.ptr(tperm), n, nat.ptr(tgs), k, nat.ptr(ids),
+        nat.ptr(sc), nat.ptr(ws), ws.numel(), nat.stream(dev)))
+    want = ost.search(q, probes, offsets, sizes, items, perm, [0.3], k, n,
+                      valid=vals[None] == qa)
+    assert np.array_equal(ids.cpu().numpy(), want[0]) and np.array_equal(sc.cpu().numpy(), want[1])
+    lowest = np.broadcast_to(vals[None] == -(2**31), (b, n))
+    want = ost.search(q, probes, offsets, sizes, items, perm, [0.3], k, n, valid=lowest)
+    for dtype in (torch.int32, torch.int64):
+        got = _run(dev, q, probes, offsets, sizes, items, perm, 0.3, k, n, item_clause_attrs=tv,
+                   clause_slots=tcs, clause_is_reverse=trev, query_clause_attrs=tqa.to(dtype))
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
