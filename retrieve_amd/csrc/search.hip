@@ -857,8 +857,12 @@ static int launch_ivf(const IvfArgs& a, dim3 grid, size_t lds, hipStream_t strea
 }
 
 // L lanes of NC chunks a row: narrow groups fold few partial dots (8 lanes take a 128-byte line
-// together); V rows in flight a group, 64 or fewer registers of them.
+// together); V rows in flight a group, 64 or fewer registers of them. (Rows of 16 and 32 bytes in
+// groups of four lanes leave most of the lanes idle: 2M rows, 64 queries of 64 of 1024 lists, the
+// scan 126 and 128 us so, 109 and 120 in one and two.)
 static int dispatch_ivf(int64_t D, const IvfArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
+  if (D <= 16) return launch_ivf<1, 1, 1>(a, grid, lds, stream);
+  if (D <= 32) return launch_ivf<2, 1, 2>(a, grid, lds, stream);
   if (D <= 64) return launch_ivf<4, 1, 4>(a, grid, lds, stream);
   if (D <= 128) return launch_ivf<8, 1, 8>(a, grid, lds, stream);
   if (D <= 192) return launch_ivf<4, 3, 4>(a, grid, lds, stream);

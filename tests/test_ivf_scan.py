@@ -15,7 +15,7 @@ from tests.test_search import _ivf, _run, _t
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("d", [16, 64, 80, 128, 192, 208, 256, 512, 528, 1024, 1040, 2064, 4112])
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 80, 128, 192, 208, 256, 512, 528, 1024, 1040, 2064, 4112])
 def test_widths(dev, d):
     g = rng(300 + d)
     n, b, k, lists = 3000, 3, 40, 30
