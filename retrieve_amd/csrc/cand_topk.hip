@@ -283,7 +283,10 @@ __global__ void __launch_bounds__(kCandThreads) cand_scan_kernel(CandArgs a) {
       if (bal == 0ull) continue;
       if (keep) list[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = c;
       cnt += __popcll(bal);
-      if (cnt > a.capw - E) {
+      // (room for the next batch, where there is one)
+      const bool more = count > kCutRows || base + step < count ||
+                        (e0 + E < kWave && (have >> (e0 + E)) != 0ull);
+      if (more && cnt > a.capw - E) {
         if (lane == 0) cnt_lds[wave] = cnt;
         const uint64_t nt = wave_compact(list, &cnt_lds[wave], scratch, a.capw, a.k);
         cnt = cnt_lds[wave];

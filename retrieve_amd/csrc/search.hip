@@ -623,14 +623,16 @@ __global__ void __launch_bounds__(kIvfThreads) ivf_scan_kernel(IvfArgs a) {
   uint64_t tau = 0;
   int cnt = 0;     // entries of this wave's list
   int queued = 0;  // slots waiting to be scored
+  const bool cut = total > kCutRows;
   // the row of the scored batch that this lane owns: the folds below leave lane gl (its low bits
   // reversed) with row v of its group
   int own = 0;
 #pragma unroll
   for (int i = 1, v = V / 2; v > 0; i <<= 1, v >>= 1) own |= (gl & i) ? v : 0;
 
-  // scores queue entries [0, n), n <= E
-  auto score = [&](int at, int n) {
+  // scores queue entries [at, at + n), n <= E; `more`: the wave may append again, or its list is
+  // to be cut to k for the merge's sake
+  auto score = [&](int at, int n, bool more) {
     v4i x[V][NC];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
@@ -676,7 +678,7 @@ __global__ void __launch_bounds__(kIvfThreads) ivf_scan_kernel(IvfArgs a) {
     if (bal == 0ull) return;
     if (keep) list[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = c;
     cnt += __popcll(bal);
-    if (cnt > a.capw - E) {
+    if (more && cnt > a.capw - E) {
       if (lane == 0) lds->cnt[wave] = cnt;
       const uint64_t nt = wave_compact(list, &lds->cnt[wave], scratch, a.capw, a.k);
       cnt = lds->cnt[wave];
@@ -768,9 +770,9 @@ __global__ void __launch_bounds__(kIvfThreads) ivf_scan_kernel(IvfArgs a) {
     wave_sync_memory();
     const bool last = s1 - base <= kIvfUnroll * kWave;
     int at = 0;
-    for (; queued - at >= E; at += E) score(at, E);
+    for (; queued - at >= E; at += E) score(at, E, cut || !last || queued - at > E);
     if (last) {
-      if (at < queued) score(at, queued - at);
+      if (at < queued) score(at, queued - at, cut);
       break;
     }
     // the remainder (fewer than E <= 64) moves to the front

@@ -47,6 +47,14 @@ struct KeepAll {
   __device__ bool operator()(uint64_t) const { return true; }
 };
 
+// Lists of a scan without a bound may end over k entries, up to their capacity: the sort of a list
+// that nothing more is appended to only spares the merge entries. It is left out where a query
+// scores at most this many rows, which one round of the merge takes in or nearly so: the sort is
+// 8 us of one wave (256 queries of 8000 candidates at k = 100 144 us with it, 126 without; 200
+// IVF rows of 3100 slots of 32 bytes 98, 89), and made above (one IVF row of 62K slots over 244 waves at k =
+// 100 87 us with it, 104 without).
+constexpr int64_t kCutRows = 16384;
+
 // Sorts list[0, *count) (global) through `scratch` (LDS, sort_n entries: a power of two >=
 // *count), keeps the best min(count, k) of the entries `keep_entry` accepts (the others drop
 // out), and returns the k-th composite (0 while fewer than k are held). Called by the whole
