@@ -51,8 +51,8 @@ struct KeepAll {
 // that nothing more is appended to only spares the merge entries. It is left out where a query
 // scores at most this many rows, which one round of the merge takes in or nearly so: the sort is
 // 8 us of one wave (256 queries of 8000 candidates at k = 100 144 us with it, 126 without; 200
-// IVF rows of 3100 slots of 32 bytes 98, 89), and made above (one IVF row of 62K slots over 244 waves at k =
-// 100 87 us with it, 104 without).
+// IVF rows of 3100 slots of 32 bytes 98, 89), and made above (one IVF row of 62K slots over 244
+// waves at k = 100 87 us with it, 104 without).
 constexpr int64_t kCutRows = 16384;
 
 // Sorts list[0, *count) (global) through `scratch` (LDS, sort_n entries: a power of two >=
