@@ -139,7 +139,7 @@ ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_p
   int64_t seed_rows = seed.rows > kSeedRowsPerK * k ? seed.rows : kSeedRowsPerK * k;
   int64_t rows_per_wg = seed.rows_per_wg;
   s.seeded = N >= 8 * seed_rows;
-  if (!s.seeded && seed.ranked) {
+  if (!s.seeded && seed.ranked && N >= seed.least_table) {
     seed_rows = small_seed_rows(N, k, seed, lpq, &rows_per_wg);
     s.sparse = seed_rows > 0;
     s.seeded = s.sparse;

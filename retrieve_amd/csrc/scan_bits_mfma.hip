@@ -398,13 +398,14 @@ bool bits_small_tiles(int nq, int capw) {
   return (nq == 2 || nq == 3) && kWavesSmall * bits_main_lds(capw, nq) <= kLdsPerCU;
 }
 
-ScanPlan bits_plan(int64_t B, int64_t N, int64_t k) {
+ScanPlan bits_plan(int64_t B, int64_t N, int64_t k, bool masked) {
   const int nq = bits_qgroups(B);
   const int64_t qpg = 16 * nq;
   // (the 64-row-tile form: three workgroups a CU, its occupancy)
   const int64_t target = bits_small_tiles(nq, bits_capw(k)) ? main_workgroups() * kWavesSmall / 2
                                                             : main_workgroups();
-  const SeedSpec seed{kScanWaves * kTileRows, kSeedRows / 2, true, kScanWaves * kGroupRows};
+  const SeedSpec seed{kScanWaves * kTileRows, kSeedRows / 2, true, kScanWaves * kGroupRows,
+                      masked ? seed_least_masked(B) : 0};
   return plan_scan(B, N, k, qpg, kScanWaves * qpg, target, bits_capw(k), kTileRows, seed);
 }
 
@@ -449,7 +450,9 @@ int dispatch_bits(int nq, const ScanArgs& a, const PassPlan& p, int64_t nqg, boo
 }  // namespace
 
 size_t bits_mfma_workspace(int64_t B, int64_t N, int64_t k) {
-  return bits_plan(B > 0 ? B : 1, N, k).total;
+  const size_t plain = bits_plan(B > 0 ? B : 1, N, k, false).total;
+  const size_t masked = bits_plan(B > 0 ? B : 1, N, k, true).total;
+  return plain > masked ? plain : masked;
 }
 
 // seed scan → rank-th bound merge → main scan → final merge (→ fallback scan and merge while
@@ -469,7 +472,7 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
                    reinterpret_cast<uintptr_t>(item_bits) % 16 == 0,
                "query_bits must be 4-byte and item_bits 16-byte aligned");
   const int nq = bits_qgroups(B);
-  const ScanPlan plan = bits_plan(B, N, k);
+  const ScanPlan plan = bits_plan(B, N, k, mask != nullptr);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;

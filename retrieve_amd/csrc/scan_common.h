@@ -192,6 +192,12 @@ int blocked_hamming(const uint64_t* query_bits, int64_t B, const uint64_t* item_
 // pass runs target_wgs workgroups in all. `spread`: a small table may be spread over more
 // workgroups, and so more lists, than one a 1024 rows.
 constexpr int64_t kSeedRows = 1 << 18;
+// The smallest table whose scan under a mask takes a sparse sample. Few rows of a smaller one pass
+// a filter, so that the merge takes them all sooner than the sample's four launches end. Top-100,
+// unseeded and seeded: int8 D = 128 at B = 16, 100K rows of which 0.1, 2, 10, 25, 100 % pass 31, 32,
+// 37, 44, 73 and 44, 50, 50, 51, 49 us; 200K 31, 38, 44, 58, 97 and 44, 55, 52, 51, 50; 512-bit
+// codes at B = 100, 50K rows 33, 48, 63, 89, 144 and 49, 70, 69, 70, 66.
+inline int64_t seed_least_masked(int64_t B) { return B < 32 ? 1 << 18 : 1 << 16; }
 struct SeedSpec {
   int64_t rows_per_wg;  // sampled rows a seed workgroup scores at least
   // Rows of the sample (at least, and kSeedRowsPerK * k at least): the main pass then keeps
@@ -203,6 +209,8 @@ struct SeedSpec {
   // Not 0: rows a workgroup of a sparse sample may be cut to, so that the k-th best of the
   // sample's lists exists; the fallback then runs behind it.
   int64_t rows_least = 0;
+  // Tables of fewer rows take no sparse sample.
+  int64_t least_table = 0;
 };
 ScanPlan plan_scan(int64_t B, int64_t N, int64_t k, int64_t qpg, int64_t lists_per_wg,
                    int64_t target_wgs, int main_capw, int64_t list_tile, const SeedSpec& seed,

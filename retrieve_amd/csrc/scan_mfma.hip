@@ -545,12 +545,19 @@ constexpr int kSeedTiles = 4;
 // The plan of a scan of B queries over N rows, top-k. `fixed`: the allocation-free form, whose
 // scratch bounds the lists: one query group a wave, and a small table neither seeded nor spread
 // over more workgroups, its lists not cut.
-static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, bool fixed = false) {
+static ScanPlan mfma_plan(int64_t B, int64_t N, int64_t k, bool masked, bool fixed = false) {
   const int64_t qpw = fixed ? 16 : 16 * mfma_groups(B);
   const SeedSpec seed{kScanWaves * kTile * kSeedTiles, mfma_seed_rows(B, N), !fixed,
-                      kScanWaves * kTile};
+                      kScanWaves * kTile, masked ? seed_least_masked(B) : 0};
   return plan_scan(B, N, k, qpw, kScanWaves * qpw, main_workgroups(), mfma_capw(k),
                    fixed ? 0 : kTile, seed, !fixed);
+}
+
+// (with and without a mask)
+static size_t mfma_plan_bytes(int64_t B, int64_t N, int64_t k) {
+  const size_t plain = mfma_plan(B, N, k, false).total;
+  const size_t masked = mfma_plan(B, N, k, true).total;
+  return plain > masked ? plain : masked;
 }
 
 // seed scan → seed threshold merge → main scan → final merge, on `stream`, no host sync
@@ -574,7 +581,7 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   if (N == 0) return launch_pad(out_ids, out_scores, B, k, Op::kind, stream);
   RT_CHECK_ARG(queries != nullptr && items != nullptr && workspace != nullptr,
                "queries, items and workspace must not be null");
-  const ScanPlan plan = mfma_plan(B, N, k, fixed);
+  const ScanPlan plan = mfma_plan(B, N, k, mask != nullptr, fixed);
   if (workspace_bytes < plan.total) {
     set_error("workspace too small: %zu < %zu", workspace_bytes, plan.total);
     return kWorkspaceTooSmall;
@@ -688,7 +695,7 @@ using namespace rt;
 
 extern "C" size_t rt_int8_scan_topk_workspace(int64_t B, int64_t N, int64_t D, int64_t k) {
   (void)D;
-  return mfma_plan(B, N, k).total;
+  return mfma_plan_bytes(B, N, k);
 }
 
 extern "C" int rt_int8_scan_topk(const int8_t* queries, int64_t B, const int8_t* items,
@@ -752,7 +759,7 @@ extern "C" int rt_int8_scan_topk_noalloc(const int8_t* queries, int64_t B, const
   RT_CHECK_ARG(B == 0 || (out_ids != nullptr && out_scores != nullptr &&
                           (N == 0 || (queries != nullptr && items != nullptr))),
                "queries, items, out_ids and out_scores must not be null");
-  const size_t need = mfma_plan(B, N, k, true).total;
+  const size_t need = mfma_plan(B, N, k, mask != nullptr, true).total;
   RT_CHECK_ARG(need <= kNoAllocScratchBytes,
                "rt_int8_scan_topk_noalloc: B = %lld, N = %lld, k = %lld need %zu bytes of "
                "scratch, above its fixed %zu bytes (call rt_int8_scan_topk with a workspace)",
@@ -767,9 +774,6 @@ extern "C" int rt_int8_scan_topk_noalloc(const int8_t* queries, int64_t B, const
 
 // ---- scans with the exact clause filter tested per candidate --------------------------------
 
-static size_t mfma_plan_bytes(int64_t B, int64_t N, int64_t k) {
-  return mfma_plan(B, N, k).total;
-}
 
 extern "C" size_t rt_scan_topk_clauses_workspace(int64_t B, int64_t N, int64_t D, int64_t k,
                                                  int64_t C, int64_t V) {
@@ -863,7 +867,7 @@ extern "C" int rt_scan_topk_bloom_clauses(
 
 extern "C" size_t rt_dense_scan_topk_workspace(int64_t B, int64_t N, int64_t D, int64_t k) {
   (void)D;
-  return mfma_plan(B, N, k).total;
+  return mfma_plan_bytes(B, N, k);
 }
 
 extern "C" int rt_dense_scan_topk(const void* queries, int64_t B, const void* items, int64_t N,

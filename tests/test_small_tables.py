@@ -187,3 +187,32 @@ def test_fallback_behind_the_kth_bits(dev, b, n, stride, k):
     want_ids, want_sc = osc.hamming_topk(q, items, k)
     assert np.array_equal(ids.cpu().numpy(), want_ids)
     assert np.array_equal(sc.cpu().numpy(), want_sc)
+
+
+@pytest.mark.parametrize("n,b", [(262_143, 3), (262_144, 31), (65_535, 33), (65_536, 40)])
+def test_masked_sample(dev, n, b):
+    """Masked scans on either side of the smallest table that takes a sparse sample (below and from
+    32 queries), rows of no, few and all passing items: int8 of a width without the blocked scan,
+    and 512-bit codes."""
+    import retrieve_amd.hip  # noqa: F401
+
+    print(f"masked sample n={n} b={b}", flush=True)
+    g = rng(n + b)
+    k = 50
+    valid = np.zeros((b, n), bool)
+    valid[0] = True
+    valid[1:-1] = g.random((b - 2, n)) < 0.02
+    mask = _t(dev, _pack(valid))
+    items = g.integers(-20, 21, (n, 768), dtype=np.int8)
+    q = g.integers(-20, 21, (b, 768), dtype=np.int8)
+    rows = np.r_[0:3, b - 2 : b]
+    ids, sc = torch.ops.retrieve_amd.int8_scan_topk(_t(dev, q), _t(dev, items), k, mask)
+    want_ids, want_sc = _want(q[rows], items, k, valid[rows])
+    assert np.array_equal(ids.cpu().numpy()[rows], want_ids)
+    assert np.array_equal(sc.cpu().numpy()[rows], want_sc)
+    codes = g.integers(-2**63, 2**63 - 1, (n, 8), dtype=np.int64)
+    qc = g.integers(-2**63, 2**63 - 1, (b, 8), dtype=np.int64)
+    ids, sc = torch.ops.retrieve_amd.hamming_scan_topk(_t(dev, qc), _t(dev, codes), k, mask)
+    want_ids, want_sc = osc.hamming_topk(qc[rows], codes, k, valid[rows])
+    assert np.array_equal(ids.cpu().numpy()[rows], want_ids)
+    assert np.array_equal(sc.cpu().numpy()[rows], want_sc)
