@@ -6,7 +6,7 @@ using namespace rt;
 
 extern "C" size_t rt_blocked_scan_topk_workspace(int64_t B, int64_t N, int64_t row_bytes,
                                                  int64_t k, int masked) {
-  // (the most workgroups any device runs: the workspace covers every CU count)
+  // (planned for the current device's CUs, as the launch is)
   return blk_plan(B, N, k, row_bytes, false, masked != 0).total;
 }
 

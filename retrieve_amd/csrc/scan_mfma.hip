@@ -449,7 +449,10 @@ static size_t main_lds_bytes(int capw, int G) {
          kScanWaves * (capw * sizeof(uint64_t) + 16 * G * sizeof(int));
 }
 
-// Query groups a wave takes: two above 16 queries.
+// Query groups a wave takes: two above 16 queries, also where 32 queries' set bitmaps leave the
+// Bloom tables little LDS and the registers one wave a SIMD (30M x 512 int8 top-100 under clauses
+// and probe, 17 / 24 / 31 queries, one group and two: 4.58 / 4.49 / 4.43 and 2.40 / 2.52 / 2.62 ms;
+// 3M 577 / 556 / 548 and 403 / 456 / 493 us).
 static int mfma_groups(int64_t B) { return B > 16 ? 2 : 1; }
 
 // The most the main pass gives the LDS copies below: they are made only while two workgroups

@@ -563,7 +563,8 @@ __host__ __device__ constexpr size_t ivf_lds_bytes() { return (sizeof(IvfLds) + 
 // query's chunks and loads V rows of NC 16-byte chunks a lane before it uses the first, and V
 // partial dots are folded across the lanes by halves (each exchange hands half of the values to
 // the other lane), so a lane ends with one row's dot. Bound: the latency of the dependent loads
-// (filter, then row), hidden by the rows in flight and eight workgroups a CU. Docs that the
+// (filter, then row), hidden by the rows in flight and three to five workgroups a CU (81
+// to 144 registers; the LDS of a full list's sort allows one at k = 1000). Docs that the
 // filter drops cost no row load and no reduction, and plain (not streaming) loads keep rows that
 // other queries of the batch probe in the caches. Filtering and scoring one slot a group step by
 // step, the same scans took (before, now): 3M x 128, 64 queries of 64 probes in 1024 lists under

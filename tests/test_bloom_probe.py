@@ -156,7 +156,8 @@ def _unfused(x, k):
 
 @pytest.mark.parametrize("b,n,d,k,from_sets", [
     (1, 40_000, 128, 10, True), (16, 60_000, 512, 100, True), (31, 50_000, 128, 64, False),
-    (16, 2_200_000, 128, 100, True), (7, 2_200_000, 64, 1000, False)])
+    (16, 2_200_000, 128, 100, True), (7, 2_200_000, 64, 1000, False),
+    (17, 60_000, 512, 100, True), (31, 300_001, 512, 300, False)])
 def test_int8_probe_scan(dev, b, n, d, k, from_sets):
     """Bit for bit with the unfused pair, and with the oracle's top-k over Bloom AND exact
     (Bloom from the unfused search's words, whose parity the search tests hold) where N is
