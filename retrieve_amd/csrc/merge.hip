@@ -105,12 +105,12 @@ int64_t main_workgroups() { return device_cus() * kMainWorkgroupsPerCU; }
 // kSeedMinRows rows); 1M rows unseeded 152 / 1216 / 4811 us, seeded 73 / 89 / 169; exact fp32
 // 100K rows at B = 1024 2230 us unseeded, 302 seeded.
 //
-// Where the fallback needs the lists' k-th best (seed.rows_least), there are 1.5 k lists at least:
-// without that bound a table whose sampled rows are better than the rest (one row block in 16,
-// say) is scanned a second time from nothing and all its rows merged by one workgroup a query
+// Where the fallback needs a bound that k lists reach (seed.rows_least), there are 1.5 k lists at
+// least: without that bound a table whose sampled rows are better than the rest (one row block in
+// 16, say) is scanned a second time from nothing and all its rows merged by one workgroup a query
 // (int8 D = 128, one query: 300K rows at k = 100 379 us, 1M at k = 1000 1824; 60 and 118 behind
-// it; without a sample 84 and 360). *rows_per_wg is halved down to rows_least while the lists are
-// fewer than 2 k.
+// the lists' k-th best; without a sample 84 and 360). *rows_per_wg is halved down to rows_least
+// while the lists are fewer than 2 k.
 static int64_t small_seed_rows(int64_t N, int64_t k, const SeedSpec& seed, int64_t lpq,
                                int64_t* rows_per_wg) {
   for (const int64_t stride : {16, 8, 4}) {
@@ -240,15 +240,22 @@ __device__ __forceinline__ void wave_append(uint64_t* dst, int* counter, bool ke
 // largest key counted with repeats, or, when a digit pass finds the kth largest key's bucket
 // holding exactly the keys still wanted, that bucket's lowest possible value (the search
 // stops there).
-// 1 <= kth <= n. Every thread of the block calls it.
+// 1 <= kth <= n. Every thread of the block calls it. edge_k (kth < edge_k <= n, or 0): *edge also
+// gets the lowest possible value of the edge_k-th largest key's bucket of the first digit, which at
+// least edge_k keys reach: a bound for the price of a compare in the first pass (a second select
+// for the exact edge_k-th cost a call 2 us: 800K fp16 rows under clauses, B = 16 100 us, 98 so).
 __device__ uint64_t block_select_desc(const uint64_t* keys, int n, int kth, unsigned* hist,
-                                      int* sh, uint64_t* red) {
+                                      int* sh, uint64_t* red, int edge_k = 0,
+                                      uint64_t* edge = nullptr) {
   const int tid = threadIdx.x;
   uint64_t kmin;
   uint64_t kmax;
   block_minmax(keys, n, red, &kmin, &kmax);
   const uint64_t diff = kmin ^ kmax;
-  if (diff == 0ull) return kmin;
+  if (diff == 0ull) {
+    if (edge_k > 0) *edge = kmin;
+    return kmin;
+  }
   int top = 63 - __builtin_clzll(diff);  // highest bit where keys differ
   uint64_t mask = top == 63 ? 0ull : ~((2ull << top) - 1ull);
   uint64_t prefix = kmin & mask;
@@ -299,8 +306,17 @@ __device__ uint64_t block_select_desc(const uint64_t* keys, int n, int kth, unsi
           run += c[j];
         }
       }
+      const unsigned want2 = static_cast<unsigned>(edge_k);
+      if (excl < want2 && want2 <= incl) {
+        unsigned run = excl;
+        int j = 0;
+        while (run + c[j] < want2) run += c[j++];
+        sh[4] = 255 - 4 * lane - j;
+      }
     }
     __syncthreads();
+    if (edge_k > 0) *edge = prefix | static_cast<uint64_t>(sh[4]) << low;
+    edge_k = 0;  // (the first digit alone)
     prefix |= static_cast<uint64_t>(sh[0]) << low;
     mask |= dmask << low;
     const bool done = sh[3] != 0 || low == 0;
@@ -325,7 +341,7 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(MergeArgs m) {
   __shared__ unsigned hist[256];
   __shared__ int part[kMergeThreads];
   __shared__ uint64_t red[2 * kMergeWaves];
-  __shared__ int sh[4];
+  __shared__ int sh[5];
   __shared__ int fill;
   const int tid = threadIdx.x;
   if (m.run_if != nullptr && *m.run_if == 0u) return;  // (uniform: the fallback is not needed)
@@ -381,6 +397,7 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(MergeArgs m) {
   // later rounds gather only what beats it and their selects run over a few survivors.
   // Empty entries (0) are dropped from the start.
   uint64_t thr = 0ull;
+  uint64_t edge = 0ull;
   int held = 0;
   for (int e0 = 0; e0 < total; e0 += CHUNK) {
     const int n = total - e0 < CHUNK ? total - e0 : CHUNK;
@@ -432,7 +449,11 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(MergeArgs m) {
     __syncthreads();
     const int cnt = held + fill;
     if (cnt > k) {
-      const uint64_t kth = block_select_desc(buf, cnt, k, hist, sh, red);
+      const bool with_edge = m.edge_out != nullptr && cnt >= m.edge_k;
+      uint64_t e = 0ull;
+      const uint64_t kth =
+          block_select_desc(buf, cnt, k, hist, sh, red, with_edge ? m.edge_k : 0, &e);
+      edge = e > edge ? e : edge;
       thr = kth;
       if (tid == 0) sh[2] = 0;
       __syncthreads();
@@ -481,6 +502,7 @@ __global__ void __launch_bounds__(kMergeThreads) merge_kernel(MergeArgs m) {
           m.tau_keep ? (m.tau_base != nullptr ? m.tau_base[q] : m.tau_out[q]) : 0ull;
       m.tau_out[q] = t > old ? t : old;
       if (m.tau2_out != nullptr) m.tau2_out[q] = t2 > t ? t2 : t;
+      if (m.edge_out != nullptr) m.edge_out[q] = edge;
       if (m.spec_flag != nullptr && q == 0) *m.spec_flag = 0u;
     }
     return;

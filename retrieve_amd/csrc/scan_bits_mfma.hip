@@ -460,8 +460,8 @@ size_t bits_mfma_workspace(int64_t B, int64_t N, int64_t k) {
 // (sample_rank), not its k-th: the main pass then keeps about rank * stride candidates a query
 // instead of k * stride. A query that ends with fewer than k entries behind a bound above 0
 // raises the flag, and the fallback main pass and merge (both returning at once while the flag is
-// clear) keep the results exact: behind the k-th best of a sparse sample's lists, else without a
-// bound.
+// clear) keep the results exact: behind a bound just below the k-th best of a sparse sample's lists
+// (MergeArgs::edge_out), else without a bound.
 int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, int64_t N,
               int64_t k, const uint64_t* mask, int64_t mask_words, int64_t* out_ids,
               void* out_scores, int score_kind, void* workspace, size_t workspace_bytes,
@@ -516,20 +516,18 @@ int bits_mfma(const uint64_t* query_bits, int64_t B, const uint64_t* item_bits, 
     m.capw = 1;
     m.flat = true;  // one entry per seed wave, contiguous per query
     m.S = plan.seed.S;
+    m.tau_out = tau;
+    m.k = rank;
     if (safe) {
-      m.tau_out = safe_tau;
-      m.tau2_out = tau;
-      m.k2 = rank;
-    } else {
-      m.tau_out = tau;
-      m.k = rank;
+      m.edge_out = safe_tau;
+      m.edge_k = static_cast<int>(k);
     }
     m.spec_flag = speculative ? spec_flag : nullptr;  // (cleared)
     st = launch_merge(m, stream);
     if (st != kOk) return st;
     m.k = static_cast<int>(k);
     m.tau_out = nullptr;
-    m.tau2_out = nullptr;
+    m.edge_out = nullptr;
     m.flat = false;
     m.spec_flag = nullptr;
   }

@@ -77,6 +77,8 @@ struct MergeArgs {
   const uint64_t* tau_base;  // threshold mode with tau_keep: the bound to keep, or null
   uint64_t* tau2_out;  // threshold mode, not null: also the k2-th composite (k2 < k), at least
   int k2;              // the k-th (0 when fewer than k2 entries exist)
+  uint64_t* edge_out;  // threshold mode, not null: also a bound that at least edge_k entries reach
+  int edge_k;          // (> k), a little below the edge_k-th (0 when fewer exist)
   const uint32_t* run_if;    // not null: the merge runs only if *run_if != 0 (a fallback merge)
   // Speculative bounds: in threshold mode block 0 clears *spec_flag; in final mode a query that
   // holds fewer than k entries although its bound spec_tau[q] is above the safe safe_tau[q]
@@ -206,8 +208,8 @@ struct SeedSpec {
   // The scan bounds its candidates by the sample's rank-th best (sample_rank) with a fallback, so
   // a sparse sample of a small table serves it too.
   bool ranked = true;
-  // Not 0: rows a workgroup of a sparse sample may be cut to, so that the k-th best of the
-  // sample's lists exists; the fallback then runs behind it.
+  // Not 0: rows a workgroup of a sparse sample may be cut to, so that k of the
+  // sample's lists hold an entry; the fallback then runs behind a bound that they reach.
   int64_t rows_least = 0;
   // Tables of fewer rows take no sparse sample.
   int64_t least_table = 0;

@@ -602,8 +602,8 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
   // filter's k-th best only where the plans pass every item the clauses pass. A query that
   // ends with fewer than k entries behind a bound above 0 raises a flag, and a fallback main
   // pass and merge (both returning at once while the flag is clear) keep the results exact: behind
-  // the k-th best of a sparse sample's lists, a bound of what the seed tests (not of the probe), else
-  // without a bound.
+  // a bound just below the k-th best of a sparse sample's lists (MergeArgs::edge_out), which holds
+  // for what the seed tests (not for the probe), else without a bound.
   const int rank = plan.seeded ? sample_rank(k, plan.seed.row_stride) : static_cast<int>(k);
   const bool speculative = plan.seeded && (rank < k || probe.doc_bits != nullptr);
   const bool safe = plan.sparse && rank < k && probe.doc_bits == nullptr;
@@ -638,20 +638,18 @@ static int run_mfma_scan(const void* queries, int64_t B, const void* items, int6
     m.capw = 1;
     m.flat = true;  // one entry per seed wave, contiguous per query
     m.S = plan.seed.S;
+    m.tau_out = tau;
+    m.k = rank;
     if (safe) {
-      m.tau_out = safe_tau;
-      m.tau2_out = tau;
-      m.k2 = rank;
-    } else {
-      m.tau_out = tau;
-      m.k = rank;
+      m.edge_out = safe_tau;
+      m.edge_k = static_cast<int>(k);
     }
     m.spec_flag = speculative ? spec_flag : nullptr;  // (cleared)
     st = launch_merge(m, stream);
     if (st != kOk) return st;
     m.k = static_cast<int>(k);
     m.tau_out = nullptr;
-    m.tau2_out = nullptr;
+    m.edge_out = nullptr;
     m.flat = false;
     m.spec_flag = nullptr;
   }
